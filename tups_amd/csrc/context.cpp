@@ -325,6 +325,7 @@ int tups_destroy(tups_ctx* c) {
   f(c->pae_y);
   f(c->pae_ym);
   f(c->pae_rows);
+  pae_plan_free(c);
   for (int i = 0; i < kEvents; ++i)
     if (c->ev[i]) hipEventDestroy(c->ev[i]);
   for (int i = 0; i < 2; ++i)
@@ -408,7 +409,10 @@ int tups_upload(tups_ctx* c, int32_t which, int32_t ch, const double* host) {
   TUPS_CHECK(p, TUPS_EINVAL, "array/channel not resident in this context");
   TUPS_HIP(hipMemcpyAsync(p, host, array_elems(c, which) * sizeof(double2), hipMemcpyHostToDevice, c->stream));
   TUPS_HIP(hipStreamSynchronize(c->stream));
-  if (which == TUPS_M) c->m_built = true;
+  if (which == TUPS_M) {
+    c->m_built = true;
+    c->pae_plan_valid = false;
+  }
   if (which == TUPS_PHIR) c->phir_valid = true;
   return TUPS_OK;
 }
@@ -526,8 +530,10 @@ int tups_build_m(tups_ctx* c) {
   int rc = ensure_tables(c);
   if (rc) return rc;
   rc = launch_build_m(c);
-  if (!rc) c->m_built = true;
-  return rc;
+  if (rc) return rc;
+  c->m_built = true;
+  c->pae_plan_valid = false;
+  return pae_plan_ensure(c);
 }
 
 int tups_pae(tups_ctx* c) {
@@ -537,6 +543,7 @@ int tups_pae(tups_ctx* c) {
   TUPS_CHECK(c->phir_valid, TUPS_ESTATE, "calculate_PAE before calc_PhiR");
   int rc = ensure_tables(c);
   if (rc) return rc;
+  if ((rc = pae_plan_ensure(c))) return rc;
   return launch_pae(c);
 }
 

@@ -27,6 +27,7 @@
 // and Lambda*Nc on the l=1 block (SRC/parquet_EQOuter.f90:48-59): F is read
 // (as Phi) and written exactly once, the minimum traffic of the crossing.
 #include "internal.h"
+#include "lds_dma.h"
 
 namespace tups {
 
@@ -625,11 +626,18 @@ struct PaeMmArgs {
   const double2* M[4];
   const double2* phir[4];
   const int* signs;
-  double2* Y;  // [kt = 4 pair + 2 routine + target][qw][j = l3 + Nl l4 + Nl^2 R][n]: n = 64 block + c,
-               // block = bx + ceil(Nf / 8) by, nu1 = 8 bx + c % 8, nu2 = 8 by + c / 8
+  double2* Y;  // [kt = 4 pair + 2 routine + target][qw][j = l3 + Nl l4 + Nl^2 R][n]; dense form: n = 64 block + c,
+               // block = bx + ceil(Nf / 8) by, nu1 = 8 bx + c % 8, nu2 = 8 by + c / 8; plan: n = nu1 + Nf nu2
   const int* rows;  // GEMM row -> (l1, l2, Q) row index l1 + Nl l2 + Nl^2 m, or null for all rows in order
   int nf, nl, nw, nibz, nr, nz, kk, rr, tiles_r, tiles_n, nbf;  // nbf = ceil(Nf / 8), tiles_n = nbf^2
   double inv_nx, nc_aux;
+  // the plan over the nonzero elements of M: column length (Nf^2 padded to 16), column tiles of
+  // 16, and its tables (PaePlanHost)
+  int nn, tiles, ng0, ng1, chunks, chunk_rows, nused;
+  const int *ubeg, *ulist, *kidx, *used, *used_by;  // kidx: four bytes a k-step
+  const int2* seg;
+  const long long* boff;  // [(group kPlanBlocks + slot) kPlanRows + r]: 2 x element offset of the row + (l1 = l2 = 0), or -1
+  const double2* frag;    // [step][lane]: M in the order of the MFMA's A operand
 };
 
 // 0-based (nu1, nu2) of blocked column n; false for the padding of the last blocks
@@ -661,23 +669,38 @@ __device__ __forceinline__ bool pae_reaches(int p, int rt, int nu1, int nu2, int
 // Y for all (kt, qw, j, n): one thread per n for a fixed (j, qw).  The gathers of
 // neighbouring n at neighbouring qw share cache lines of PhiR (the frequency
 // maps shift nu1 against qw), so qw varies fastest over the workgroups of one
-// XCD.  grid: ((Nf^2 + 255) / 256) * kk * nw
+// XCD.  With the plan only the inner indices that some row needs are formed (66 of
+// 100 at Nl = 5, 320 of 486 at Nl = 9, 46 and 239 for phbar->ph).
+// grid: ceil(columns / 256) * (inner indices) * nw
+template <bool PLAN>
 __global__ __launch_bounds__(256) void pae_ybuild(PaeMmArgs a) {
   const int nf = a.nf, nl = a.nl, nw = a.nw, nz = a.nz;
-  const int ncol = 64 * a.tiles_n;
+  const int ncol = PLAN ? a.nn : 64 * a.tiles_n;
   const int nbn = ncol / 256 + (ncol % 256 ? 1 : 0);
   const int logical = xcd_remap(blockIdx.x, gridDim.x);
   const int w0 = logical % nw, rest = logical / nw;
-  const int j = rest / nbn, qw = w0 + 1;
-  const int n = (rest - j * nbn) * 256 + threadIdx.x;
+  const int ju = rest / nbn, qw = w0 + 1;
+  const int j = PLAN ? a.used[ju] : ju;
+  const int by = PLAN ? a.used_by[ju] : 15;
+  const int n = (rest - ju * nbn) * 256 + threadIdx.x;
   if (n >= ncol) return;
   const size_t nn = (size_t)ncol;
-  auto at = [&](int kt) { return ((size_t)(kt * nw + w0) * a.kk + j) * nn + n; };
+  auto put = [&](int kt, double2 v) {
+    if (by >> (kt >> 1) & 1) a.Y[((size_t)(kt * nw + w0) * a.kk + j) * nn + n] = v;
+  };
   int nu1, nu2;
-  if (!pae_col(a, n, nu1, nu2)) {
+  bool real;
+  if (PLAN) {
+    nu2 = n / nf;
+    nu1 = n - nu2 * nf;
+    real = nu2 < nf;
+  } else {
+    real = pae_col(a, n, nu1, nu2);
+  }
+  if (!real) {
     // padding columns: finite zeros (their products land in columns the epilogue drops)
 #pragma unroll
-    for (int kt = 0; kt < 8; ++kt) a.Y[at(kt)] = make_double2(0.0, 0.0);
+    for (int kt = 0; kt < 8; ++kt) put(kt, make_double2(0.0, 0.0));
     return;
   }
   ++nu1;
@@ -706,14 +729,14 @@ __global__ __launch_bounds__(256) void pae_ybuild(PaeMmArgs a) {
                             nf + 1 - nu1, nu1 - qw - w2t + 2);
   const Term t3 = make_term(pb_plain, pb_tr, dn + 1, nu1, clampnu(qw - nu1 - dn + nf, nf), 1 - dn,
                             nf + 1 - nu1, clampnu(nu1 - qw - (1 - dn) + 2, nf));
-  a.Y[at(0)] = comb(0, 1, t0, -0.5, -1.5);  // phbar->ph -> d
-  a.Y[at(1)] = comb(0, 1, t0, -0.5, 0.5);   //           -> m
-  a.Y[at(2)] = comb(2, 3, t1, 0.5, 1.5);    // pp->ph    -> d
-  a.Y[at(3)] = comb(2, 3, t1, -0.5, 0.5);   //           -> m
-  a.Y[at(4)] = comb(0, 1, t2, 0.5, -1.5);   // ph->pp    -> s
-  a.Y[at(5)] = comb(0, 1, t2, 0.5, 0.5);    //           -> t
-  a.Y[at(6)] = comb(0, 1, t3, 0.5, -1.5);   // phbar->pp -> s
-  a.Y[at(7)] = comb(0, 1, t3, -0.5, -0.5);  //           -> t
+  put(0, comb(0, 1, t0, -0.5, -1.5));  // phbar->ph -> d
+  put(1, comb(0, 1, t0, -0.5, 0.5));   //           -> m
+  put(2, comb(2, 3, t1, 0.5, 1.5));    // pp->ph    -> d
+  put(3, comb(2, 3, t1, -0.5, 0.5));   //           -> m
+  put(4, comb(0, 1, t2, 0.5, -1.5));   // ph->pp    -> s
+  put(5, comb(0, 1, t2, 0.5, 0.5));    //           -> t
+  put(6, comb(0, 1, t3, 0.5, -1.5));   // phbar->pp -> s
+  put(7, comb(0, 1, t3, -0.5, -0.5));  //           -> t
 }
 
 // One workgroup per 64 x 64 output tile of one (qw, pair, target); four waves of
@@ -848,7 +871,174 @@ __global__ __launch_bounds__(256, 4) void pae_mm(PaeMmArgs a) {
     }
 }
 
-static int pae_gemm_path(tups_ctx* c) {
+// The same products over the plan: one workgroup per (group of row blocks, tile of
+// 16 columns, qw), both targets of the pair.  Per routine it stages the group's
+// inner indices of Y for its columns in LDS by direct loads (at most kPlanChunk at a
+// time), then each wave runs the k-steps of its row blocks: M comes in fragment
+// order, two steps ahead, and serves both targets.  A row needs 3 to 10% of the
+// inner indices (the rest of M is zero), so the products fall to the order of the
+// streams (Phi in, F out), and the split is made for those: small groups, so that
+// three workgroups per CU cover each other's staging, products and epilogue; the
+// groups of one column tile next to each other on one XCD, so that its part of Y is
+// read from HBM once.  Tiles of 16 columns follow a routine's frequency band more
+// closely than the dense form's 8 x 8 blocks.  Nx = 8, Nf = 64, Nl = 5: 1.98 ms a
+// call with 6.3 GB of streams (the dense form 5.35 ms); Nx = 8, Nf = 32, Nl = 9:
+// 1.41 against 9.8 ms.  One target per workgroup and groups of 16 blocks, with twice
+// the M reads per product: 2.68 and 1.65 ms.
+__global__ __launch_bounds__(256, 3) void pae_sparse(PaeMmArgs a) {
+  extern __shared__ double2 ys[];  // [target][chunk][16]
+  const int nf = a.nf, per = a.ng0 + a.ng1;
+  const int logical = xcd_remap(blockIdx.x, gridDim.x);
+  const int g = logical % per, rest = logical / per;
+  const int tile = rest % a.tiles, w0 = rest / a.tiles;
+  const int p = g >= a.ng0 ? 1 : 0;
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = tile * 16 + li;
+  const int nu2 = n / nf, nu1 = n - nu2 * nf;
+  const bool ok = nu2 < nf;
+  double2* ys1 = ys + a.chunk_rows * 16;
+  d4 re[2][kPlanSlots], im[2][kPlanSlots];
+#pragma unroll
+  for (int i = 0; i < kPlanSlots; ++i)
+#pragma unroll
+    for (int t = 0; t < 2; ++t) re[t][i] = im[t][i] = d4{0.0, 0.0, 0.0, 0.0};
+  for (int rt = 0; rt < 2; ++rt) {
+    // every wave holds the same 16 columns, so this is uniform over the workgroup
+    if (!__any(ok && pae_reaches(p, rt, nu1 + 1, nu2 + 1, w0 + 1, nf, a.nw))) continue;
+    const size_t slab = (size_t)a.nw * a.kk * a.nn;  // from target to target
+    const double2* yb = a.Y + (size_t)(4 * p + 2 * rt) * slab + (size_t)w0 * a.kk * a.nn + (size_t)tile * 16;
+    const int* ub = a.ubeg + (size_t)(g * 2 + rt) * (a.chunks + 1);
+    const int2* sb = a.seg + (size_t)(g * 2 + rt) * a.chunks * kPlanBlocks;
+    for (int c = 0; c < a.chunks; ++c) {
+      const int u0 = ub[c], len = ub[c + 1] - u0;
+      if (len <= 0) break;
+      int2 sg[kPlanSlots];
+      int kp[kPlanSlots];  // lane s: the four LDS rows of k-step s, a byte each
+#pragma unroll
+      for (int i = 0; i < kPlanSlots; ++i) {
+        sg[i] = sb[c * kPlanBlocks + wave * kPlanSlots + i];
+        kp[i] = sg[i].x + lane < sg[i].y ? a.kidx[sg[i].x + lane] : 0;
+      }
+      __syncthreads();  // the last chunk's readers are done
+      // a wave's load brings four rows of 16 columns
+      for (int j0 = 4 * wave; j0 < len; j0 += 16) {
+        const int j = a.ulist[u0 + min(j0 + lk, len - 1)];
+        const unsigned off = (unsigned)(((size_t)j * a.nn + li) * sizeof(double2));
+        dma16(yb, off, lds_addr(ys + 16 * j0));
+        dma16(yb + slab, off, lds_addr(ys1 + 16 * j0));
+      }
+      wait_vmcnt<0>();
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < kPlanSlots; ++i) {
+        const int cnt = sg[i].y - sg[i].x;
+        if (cnt <= 0) continue;
+        const double2* fr = a.frag + (size_t)sg[i].x * 64 + lane;
+        double2 m0 = fr[0], m1 = fr[64 * min(1, cnt - 1)];
+        for (int s = 0; s < cnt; ++s) {
+          const int row = __builtin_amdgcn_readlane(kp[i], s) >> (8 * lk) & 255;
+          const double2 y0 = ys[row * 16 + li], y1 = ys1[row * 16 + li], m = m0;
+          m0 = m1;
+          m1 = fr[64 * min(s + 2, cnt - 1)];
+          re[0][i] = __builtin_amdgcn_mfma_f64_16x16x4f64(m.x, y0.x, re[0][i], 0, 0, 0);
+          im[0][i] = __builtin_amdgcn_mfma_f64_16x16x4f64(m.x, y0.y, im[0][i], 0, 0, 0);
+          re[1][i] = __builtin_amdgcn_mfma_f64_16x16x4f64(m.x, y1.x, re[1][i], 0, 0, 0);
+          im[1][i] = __builtin_amdgcn_mfma_f64_16x16x4f64(m.x, y1.y, im[1][i], 0, 0, 0);
+          re[0][i] = __builtin_amdgcn_mfma_f64_16x16x4f64(m.y, y0.y, re[0][i], 0, 0, 1);
+          im[0][i] = __builtin_amdgcn_mfma_f64_16x16x4f64(m.y, y0.x, im[0][i], 0, 0, 0);
+          re[1][i] = __builtin_amdgcn_mfma_f64_16x16x4f64(m.y, y1.y, re[1][i], 0, 0, 1);
+          im[1][i] = __builtin_amdgcn_mfma_f64_16x16x4f64(m.y, y1.x, im[1][i], 0, 0, 0);
+        }
+      }
+    }
+  }
+  if (!ok) return;
+  const int nz = a.nz;
+  const size_t col = (size_t)w0 * nz * nz + (size_t)nu2 * nz + nu1;
+  long long off[kPlanSlots][4];
+#pragma unroll
+  for (int i = 0; i < kPlanSlots; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      off[i][e] = a.boff[(size_t)(g * kPlanBlocks + wave * kPlanSlots + i) * kPlanRows + lk + 4 * e];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const double2* phi = a.phi[2 * p + t] + col;
+    double2* F = a.F[2 * p + t] + col;
+    double2 o[kPlanSlots][4];
+#pragma unroll
+    for (int i = 0; i < kPlanSlots; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (off[i][e] >= 0) o[i][e] = phi[off[i][e] >> 1];
+#pragma unroll
+    for (int i = 0; i < kPlanSlots; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (off[i][e] < 0) continue;
+        if (off[i][e] & 1) {
+          const double2 lv = a.lam[2 * p + t][(size_t)nu1 + (size_t)nf * ((size_t)nu2 + (size_t)nf * w0)];
+          o[i][e].x += lv.x * a.nc_aux;
+          o[i][e].y += lv.y * a.nc_aux;
+        }
+        o[i][e].x += re[t][i][e] * a.inv_nx;
+        o[i][e].y += im[t][i][e] * a.inv_nx;
+        F[off[i][e] >> 1] = o[i][e];
+      }
+  }
+}
+
+// nonzero elements of M over Q: out[(k Nl^2 + l) kk + j]; grid (ceil(Nl^2 kk / 256), 4)
+__global__ __launch_bounds__(256) void pae_support(PaeMmArgs a, uint8_t* out) {
+  const int nl2 = a.nl * a.nl;
+  const int e = blockIdx.x * 256 + threadIdx.x;
+  if (e >= nl2 * a.kk) return;
+  const int l = e % nl2, j = e / nl2, jl = j % nl2, jr = j / nl2;
+  const double2* M = a.M[blockIdx.y];
+  bool any = false;
+  for (int m = 0; m < a.nibz; ++m) {
+    const double2 v = M[(size_t)l + (size_t)nl2 * jl + (size_t)nl2 * nl2 * (m + (size_t)a.nibz * jr)];
+    any = any || !(v.x == 0.0 && v.y == 0.0);
+  }
+  out[((size_t)blockIdx.y * nl2 + l) * a.kk + j] = any ? 1 : 0;
+}
+
+// M into the order of the plan's k-steps; one wave per step
+__global__ __launch_bounds__(256) void pae_pack(PaeMmArgs a, const int* step_blk, const int* kj, const int* brow,
+                                                double2* frag, int steps) {
+  const int st = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (st >= steps) return;
+  const int nl2 = a.nl * a.nl;
+  const int blk = step_blk[st] >> 1, rt = step_blk[st] & 1;
+  const int p = blk / kPlanBlocks >= a.ng0 ? 1 : 0;
+  const int r = brow[(size_t)blk * kPlanRows + (lane & 15)], j = kj[(size_t)st * 4 + (lane >> 4)];
+  double2 v = make_double2(0.0, 0.0);
+  if (r >= 0 && j >= 0)
+    v = a.M[2 * p + rt][(size_t)(r % nl2) + (size_t)nl2 * (j % nl2) +
+                        (size_t)nl2 * nl2 * (r / nl2 + (size_t)a.nibz * (j / nl2))];
+  frag[(size_t)st * 64 + lane] = v;
+}
+
+// device copy of the plan; dense: the plan saves too little (or its offsets would not fit)
+struct PaePlan {
+  bool dense = true;
+  int groups[2] = {0, 0}, chunks = 0, chunk_len = 0, nused = 0;
+  void* mem = nullptr;  // all tables
+  const int *ubeg = nullptr, *ulist = nullptr, *kidx = nullptr, *used = nullptr, *used_by = nullptr;
+  const int2* seg = nullptr;
+  const long long* boff = nullptr;
+  const double2* frag = nullptr;
+};
+
+void pae_plan_free(tups_ctx* c) {
+  if (!c->pae_plan) return;
+  if (c->pae_plan->mem) (void)hipFree(c->pae_plan->mem);
+  delete c->pae_plan;
+  c->pae_plan = nullptr;
+}
+
+static PaeMmArgs mm_args(tups_ctx* c) {
   const tups_sizes& s = c->sz;
   PaeMmArgs a{};
   for (int r = 0; r < 4; ++r) {
@@ -877,8 +1067,147 @@ static int pae_gemm_path(tups_ctx* c) {
   a.inv_nx = 1.0 / s.nx;
   const double f0 = c->tab.ff[0];
   a.nc_aux = std::fabs(1.0 / f0 * 1.0 / f0);
+  a.tiles = (s.nf * s.nf + 15) / 16;
+  a.nn = 16 * a.tiles;
+  return a;
+}
+
+int pae_plan_ensure(tups_ctx* c) {
+  const tups_sizes& s = c->sz;
+  if (c->pae_plan_valid || s.nl == 1 || !c->pae_ym || !c->m_built) return TUPS_OK;
+  PaeMmArgs a = mm_args(c);
+  const int nl2 = s.nl * s.nl;
+  drop_graphs(c);  // they hold the old plan's pointers
+  ++c->pae_plan_gen;
+  uint8_t* d_sup = nullptr;
+  const size_t nsup = (size_t)4 * nl2 * a.kk;
+  std::vector<uint8_t> sup(nsup);
+  TUPS_HIP(hipMalloc((void**)&d_sup, nsup));
+  hipLaunchKernelGGL(pae_support, dim3((unsigned)((nl2 * a.kk + 255) / 256), 4), dim3(256), 0, c->stream, a, d_sup);
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess) e = hipMemcpyAsync(sup.data(), d_sup, nsup, hipMemcpyDeviceToHost, c->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);  // also: nothing still reads the old plan
+  (void)hipFree(d_sup);
+  TUPS_HIP(e);
+  pae_plan_free(c);
+  PaePlanHost h;
+  build_pae_plan(sup, c->pae_rows_host, s.nl, s.nibz, a.kk, h);
+  c->pae_plan = new PaePlan();
+  PaePlan& pl = *c->pae_plan;
+  // the dense form's k-steps of 16 rows, both pairs
+  const long long dense = 2LL * ((a.rr + 15) / 16) * 2 * ((a.kk + 3) / 4);
+  // a dense tile shares its staging and its M between four times the rows, so the plan has to
+  // save at least half of the k-steps (M of the library's own tables: 8 to 16 times fewer)
+  pl.dense = 2 * h.steps > dense || (double)a.kk * a.nn * sizeof(double2) >= 4294967296.0;
+  if (!pl.dense) {
+    pl.groups[0] = h.groups[0];
+    pl.groups[1] = h.groups[1];
+    pl.chunks = h.chunks;
+    pl.chunk_len = h.chunk_len;
+    pl.nused = (int)h.used.size();
+    std::vector<long long> boff(h.brow.size(), -1);
+    for (size_t i = 0; i < h.brow.size(); ++i)
+      if (h.brow[i] >= 0) {
+        const int l = h.brow[i] % nl2, m = h.brow[i] / nl2;
+        const long long o = (long long)m * s.nw * s.nz * s.nz + (long long)(l / s.nl) * s.nf * s.nz +
+                            (long long)(l % s.nl) * s.nf;
+        boff[i] = 2 * o + (l == 0 ? 1 : 0);
+      }
+    // one allocation, every part on a 256-byte boundary
+    size_t total = 0;
+    auto part = [&](size_t bytes) {
+      const size_t at = total;
+      total += (bytes + 255) / 256 * 256;
+      return at;
+    };
+    const size_t o_frag = part((size_t)h.steps * 64 * sizeof(double2)), o_boff = part(boff.size() * sizeof(long long)),
+                 o_seg = part(h.seg.size() * sizeof(int)), o_ubeg = part(h.ubeg.size() * sizeof(int)),
+                 o_ulist = part(h.ulist.size() * sizeof(int)), o_kidx = part(h.kidx.size() * sizeof(int)),
+                 o_kj = part(h.kj.size() * sizeof(int)), o_sb = part(h.step_blk.size() * sizeof(int)),
+                 o_brow = part(h.brow.size() * sizeof(int)), o_used = part(h.used.size() * sizeof(int)),
+                 o_by = part(h.used_by.size() * sizeof(int));
+    e = hipMalloc(&pl.mem, total);
+    if (e != hipSuccess) {
+      pl.mem = nullptr;
+      pae_plan_free(c);
+      set_error(std::string("crossing plan: hipMalloc of ") + std::to_string(total) + " bytes failed: " + hipGetErrorString(e));
+      return TUPS_ENOMEM;
+    }
+    char* base = (char*)pl.mem;
+    auto send = [&](size_t at, const auto& v) {
+      if (e == hipSuccess && !v.empty())
+        e = hipMemcpyAsync(base + at, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice, c->stream);
+    };
+    e = hipSuccess;
+    send(o_boff, boff);
+    send(o_seg, h.seg);
+    send(o_ubeg, h.ubeg);
+    send(o_ulist, h.ulist);
+    send(o_kidx, h.kidx);
+    send(o_kj, h.kj);
+    send(o_sb, h.step_blk);
+    send(o_brow, h.brow);
+    send(o_used, h.used);
+    send(o_by, h.used_by);
+    a.ng0 = pl.groups[0];
+    if (e == hipSuccess && h.steps > 0) {
+      hipLaunchKernelGGL(pae_pack, dim3((unsigned)((h.steps + 3) / 4)), dim3(256), 0, c->stream, a,
+                         (const int*)(base + o_sb), (const int*)(base + o_kj), (const int*)(base + o_brow),
+                         (double2*)(base + o_frag), (int)h.steps);
+      e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    if (e != hipSuccess) pae_plan_free(c);
+    TUPS_HIP(e);
+    pl.frag = (const double2*)(base + o_frag);
+    pl.boff = (const long long*)(base + o_boff);
+    pl.seg = (const int2*)(base + o_seg);
+    pl.ubeg = (const int*)(base + o_ubeg);
+    pl.ulist = (const int*)(base + o_ulist);
+    pl.kidx = (const int*)(base + o_kidx);
+    pl.used = (const int*)(base + o_used);
+    pl.used_by = (const int*)(base + o_by);
+  }
+  c->pae_plan_valid = true;
+  return TUPS_OK;
+}
+
+static int pae_gemm_path(tups_ctx* c) {
+  const tups_sizes& s = c->sz;
+  PaeMmArgs a = mm_args(c);
+  TUPS_CHECK(c->pae_plan && c->pae_plan_valid, TUPS_ESTATE, "crossing without a plan for M");
+  const PaePlan& pl = *c->pae_plan;
+  if (!pl.dense) {
+    a.ng0 = pl.groups[0];
+    a.ng1 = pl.groups[1];
+    a.chunks = pl.chunks;
+    a.chunk_rows = (pl.chunk_len + 3) / 4 * 4;
+    a.nused = pl.nused;
+    a.ubeg = pl.ubeg;
+    a.ulist = pl.ulist;
+    a.kidx = pl.kidx;
+    a.used = pl.used;
+    a.used_by = pl.used_by;
+    a.seg = pl.seg;
+    a.boff = pl.boff;
+    a.frag = pl.frag;
+    const long long nby = (long long)((a.nn + 255) / 256) * pl.nused * s.nw;
+    const long long nbm = (long long)(a.ng0 + a.ng1) * a.tiles * s.nw;
+    TUPS_CHECK(nby < (1LL << 31) && nbm < (1LL << 31), TUPS_EINVAL, "crossing grid too large");
+    if (int rc = timer_begin(c)) return rc;
+    if (nby > 0) {
+      hipLaunchKernelGGL(pae_ybuild<true>, dim3((unsigned)nby), dim3(256), 0, c->stream, a);
+      TUPS_HIP(hipGetLastError());
+    }
+    if (int rc = timer_end(c, TUPS_K_PAE_GATHER)) return rc;
+    if (int rc = timer_begin(c)) return rc;
+    const size_t lds = (size_t)2 * a.chunk_rows * 16 * sizeof(double2);
+    hipLaunchKernelGGL(pae_sparse, dim3((unsigned)nbm), dim3(256), lds, c->stream, a);
+    TUPS_HIP(hipGetLastError());
+    return timer_end(c, TUPS_K_PAE);
+  }
   if (int rc = timer_begin(c)) return rc;
-  hipLaunchKernelGGL(pae_ybuild, dim3((unsigned)((64 * a.tiles_n + 255) / 256 * a.kk * s.nw)), dim3(256), 0,
+  hipLaunchKernelGGL(pae_ybuild<false>, dim3((unsigned)((64 * a.tiles_n + 255) / 256 * a.kk * s.nw)), dim3(256), 0,
                      c->stream, a);
   TUPS_HIP(hipGetLastError());
   if (int rc = timer_end(c, TUPS_K_PAE_GATHER)) return rc;

@@ -154,6 +154,7 @@ extern "C" int tups_iteration_full(tups_ctx* c, int32_t mode, int32_t use_graph,
   TUPS_CHECK(c->green_set, TUPS_ESTATE, "no Sigma on the device (tups_set_sigma first)");
   int rc = ensure_tables(c);
   if (rc) return rc;
+  if ((rc = pae_plan_ensure(c))) return rc;
   if (mode == TUPS_BSE_LADDER_SPLIT && (rc = bse_split_reserve(c, nullptr))) return rc;
   if ((rc = sde_reserve(c, f_range))) return rc;
   if (!(n_particle >= 0.0)) n_particle = -1.0;  // negative or NaN: mu stays
@@ -217,6 +218,7 @@ extern "C" int tups_iteration(tups_ctx* c, int32_t mode, int32_t use_graph) {
   TUPS_CHECK(c->m_built, TUPS_ESTATE, "iteration before the M tensors were built");
   int rc = ensure_tables(c);
   if (rc) return rc;
+  if ((rc = pae_plan_ensure(c))) return rc;
   if (mode == TUPS_BSE_LADDER_SPLIT && (rc = bse_split_reserve(c, nullptr))) return rc;
   bool swapped = false;
   if (!use_graph) {

@@ -35,6 +35,7 @@ struct tups_uneven {
   int parity = 0;
   int cap_batch_variant = -1, cap_pae_variant = -1;  // the variants the graphs were captured with
   const void* cap_tables = nullptr;                   // and the tables (their device pointers)
+  int cap_plan = -1;                                  // and the crossing plan
 };
 
 namespace tups {
@@ -228,6 +229,9 @@ extern "C" int tups_uneven_create(int32_t nx, int32_t nf_max, const int32_t* nf_
       rc = TUPS_EHIP;
     } else {
       u->ctx->pae_nrows = (int)rows.size();
+      u->ctx->pae_rows_host = rows;
+      u->ctx->pae_plan_valid = false;
+      rc = pae_plan_ensure(u->ctx);
     }
   }
   if (rc) {
@@ -250,6 +254,7 @@ extern "C" int tups_uneven_iteration(tups_uneven* u, int32_t use_graph) {
   tups_ctx* c = u->ctx;
   int rc = ensure_tables(c);
   if (rc) return rc;
+  if ((rc = pae_plan_ensure(c))) return rc;
   bool swapped = false;
   if (!use_graph) {
     rc = uneven_sequence(u, &swapped);
@@ -258,11 +263,12 @@ extern "C" int tups_uneven_iteration(tups_uneven* u, int32_t use_graph) {
   }
   // tile variants and tables are part of the captured launches
   if (u->cap_batch_variant != u->batch->variant || u->cap_pae_variant != c->pae_variant ||
-      u->cap_tables != c->d_ph_coef) {
+      u->cap_tables != c->d_ph_coef || u->cap_plan != c->pae_plan_gen) {
     uneven_drop_graphs(u);
     u->cap_batch_variant = u->batch->variant;
     u->cap_pae_variant = c->pae_variant;
     u->cap_tables = c->d_ph_coef;
+    u->cap_plan = c->pae_plan_gen;
   }
   if (!u->graph[u->parity]) {
     const int slot = u->parity;
