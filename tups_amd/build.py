@@ -26,8 +26,8 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
 SOURCES = ["context.cpp", "tables.cpp", "iteration.cpp", "prms.cpp", "bse.hip", "phir.hip", "eqmatrix.hip",
-           "crossing.hip", "crossing_plan.cpp", "vertex_ops.hip", "bse_split.hip", "bse_closed.hip", "chi.hip", "sde.hip", "gtau.hip",
-           "conv.hip", "sus.hip", "uneven.hip"]
+           "crossing.hip", "crossing_plan.cpp", "vertex_ops.hip", "bse_split.hip", "bse_closed.hip", "bubble.hip", "chi.hip",
+           "sde.hip", "gtau.hip", "conv.hip", "sus.hip", "uneven.hip"]
 
 # Packed FP32 instructions are disabled for every device compile.
 DEVICE_FLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]

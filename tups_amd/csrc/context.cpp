@@ -9,6 +9,7 @@
 #include <cmath>
 #include <cstring>
 
+#include "bubble.h"
 #include "internal.h"
 
 namespace tups {
@@ -124,7 +125,7 @@ int upload_tables(tups_ctx* c) {
   TUPS_HIP(hipMalloc((void**)&c->d_ph_coef, std::max<size_t>(1, pb.coef.size()) * sizeof(double)));
   TUPS_HIP(hipMemcpyAsync(c->d_ph_coef, pb.coef.data(), pb.coef.size() * sizeof(double),
                           hipMemcpyHostToDevice, c->stream));
-  TUPS_HIP(hipStreamSynchronize(c->stream));
+  if ((rc = upload_bubble_weights(c))) return rc;  // synchronises
   c->tables_dirty = false;
   return TUPS_OK;
 }
@@ -313,6 +314,8 @@ int tups_destroy(tups_ctx* c) {
   f(c->d_sigma);
   f(c->d_sigh);
   f(c->d_ffk);
+  if (c->green_tab_owned) f(c->green_tab);
+  f(c->d_bubble_wt);
   f(c->d_ffik);
   f(c->d_eqsr);
   f(c->d_qm);

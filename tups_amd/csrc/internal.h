@@ -117,6 +117,12 @@ __device__ __forceinline__ void st_stream(double2* p, double2 v) {
   __builtin_nontemporal_store(w, reinterpret_cast<stream2*>(p));
 }
 
+// one family of bubble weights (bubble.hip): `count` weights in groups of nw, at wt and dst
+struct BubbleSet {
+  int nw = 0, groups = 0, count = 0, dst = 0;
+  size_t wt = 0;
+};
+
 // device state of the chemical-potential search of calc_Gkw_Grt: the current mu,
 // the bracket, the last particle number and the candidates of the current pass
 struct GtauState {
@@ -158,6 +164,12 @@ struct tups_ctx {
   double2* d_ph_coef = nullptr;   // their coefficients
   int ph_first[4] = {0, 0, 0, 0}, ph_count[4] = {0, 0, 0, 0};
   int* d_flag = nullptr;
+  double* d_bubble_wt = nullptr;  // bubble weight families (bubble.h) and their destinations
+  int* d_bubble_dst = nullptr;
+  tups::BubbleSet bubble_set[4];
+  double2* green_tab = nullptr;   // table of Green's functions (bubble.h), kept from call to call
+  size_t green_tab_bytes = 0;
+  bool green_tab_owned = false;   // false: it lies in the block of d_bubble_wt
   double2* d_sigma = nullptr;   // calc_chi: Sigma(Nx Ny Nf)
   double2* d_sigh = nullptr;    // calc_chi: Sigma_H(Nx, Ny)
   double2* pae_ym = nullptr;    // Nl > 1 crossing: gathered PhiR, 8 x (Nl^2 NR, 64 ceil(Nf / 8)^2) per qw
@@ -237,12 +249,14 @@ int launch_bse_closed(tups_ctx* c);
 int launch_bse_closed_ir(tups_ctx* c);
 int launch_calc_chi(tups_ctx* c, const double* sigma, const double* sigma_h, double mu, int ngrain);
 struct GreenParams;
+struct GreenTab;
 int upload_sigma(tups_ctx* c, const double* sigma, const double* sigma_h, GreenParams* g, double mu, int ngrain);
 int launch_sde(tups_ctx* c, const double* sigma, const double* sigma_h, double mu, int ngrain, int f_range, double u,
                int use_u2, double* sigma_out);
-int launch_chi_device(tups_ctx* c, const GreenParams& g);
+int launch_chi_device(tups_ctx* c, const GreenParams& g, const GreenTab* tab);
 int sde_reserve(tups_ctx* c, int f_range);
-int launch_sde_device(tups_ctx* c, const GreenParams& g, int f_range, double u, int use_u2);
+int launch_sde_device(tups_ctx* c, const GreenParams& g, const GreenTab* tab, bool aux_done, int f_range, double u,
+                      int use_u2);
 int launch_sigma_commit(tups_ctx* c, int f_range);
 int green_params(const tups_ctx* c, GreenParams* g);
 int gtau_reserve(tups_ctx* c, int ngrain);

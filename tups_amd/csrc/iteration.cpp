@@ -8,8 +8,7 @@
 // the ping-pong partner of Gamma, so the buffers alternate and two graphs per
 // mode cover every iteration.  Nothing is allocated while capturing (the split
 // workspace is reserved beforehand) and no memset node is recorded.
-#include "green.h"
-#include "internal.h"
+#include "bubble.h"
 
 #include <cmath>
 
@@ -71,13 +70,19 @@ static int full_sequence(tups_ctx* c, int mode, int f_range, double u, int use_u
   } else if (use_u2) {
     if ((rc = launch_gtau(c, 2, 0, 0.0, u, 0.0, 1))) return rc;
   }
-  if ((rc = launch_chi_device(c, g))) return rc;
+  // one table of Green's functions for the bubbles and the self-energy (unless it takes several
+  // passes); at f_range 0 the self-energy's bubbles come from the same pairs as chi's
+  GreenTab tab;
+  if ((rc = green_tab_build(c, g, f_range, 0, &tab))) return rc;
+  const GreenTab* t = tab.split ? nullptr : &tab;
+  const bool aux = f_range == 0 && t;
+  if ((rc = aux ? launch_chi_aux_device(c, g, sde_aux_out(c, 0), t) : launch_chi_device(c, g, t))) return rc;
   if ((rc = mode == TUPS_BSE_LADDER_SPLIT ? launch_bse_split(c) : launch_bse_ladder(c))) return rc;
   swap_vertex_buffers(c);
   *swapped = true;
   if ((rc = launch_phir(c))) return rc;
   if ((rc = launch_pae(c))) return rc;
-  if ((rc = launch_sde_device(c, g, f_range, u, use_u2))) return rc;
+  if ((rc = launch_sde_device(c, g, t, aux, f_range, u, use_u2))) return rc;
   if (use_u2 && (rc = launch_order_2nd(c, u, sde_output(c, f_range)))) return rc;
   if ((rc = launch_sigma_commit(c, f_range))) return rc;
   return launch_gamma_update(c);

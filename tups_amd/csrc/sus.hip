@@ -3,11 +3,10 @@
 // Reference: calc_sus, SRC/parquet_sus.f90:18-362, with calc_GG_ph / calc_GG_pp
 // (:528-643), fillpickNu_range (:708-731) and the external form factors
 // fill_FF_sdwave (SRC/parquet_formfactors.f90:792-815: 1, cos px - cos py,
-// sin px, sin px sin py).  Two kernels:
-//  1. sus_gg: per q slot the Green's-function pairs of the enlarged box
+// sin px, sin px sin py).  Two steps:
+//  1. per q slot the Green's-function pairs of the enlarged box (bubble.hip)
 //       GG_ph(l, nu; ff) = 1/Ng^2 sum_{k, g} FF_sd(k, ff) FF(k, l) G(g; k, nu) G(g; k + q, nu + w - 1)
-//       GG_pp(l, nu; ff) = 1/Ng^2 sum_{k, g} FF_sd(k, ff) FF(k, l) G(g; k, nu) G(Ng + 1 - g; q - k, Nf - nu + w)
-//     with k split over lanes as in the SDE's auxiliary bubbles;
+//       GG_pp(l, nu; ff) = 1/Ng^2 sum_{k, g} FF_sd(k, ff) FF(k, l) G(g; k, nu) G(Ng + 1 - g; q - k, Nf - nu + w);
 //  2. sus_contract: per (q, channel) sus(ff) = sum_{L1, L2} V(L1, L2) GG(L1) GG(L2) / (Nx^2 Ny^2 beta^2),
 //     V = F inside the box and, for the pairs not both inside, the bare vertex
 //     (U, -U, 2U, 0 for d, m, s, t) / FF11^2 on the l = 1 block plus the
@@ -17,8 +16,7 @@
 // The loop's G_r_LL hold Phi when the reference calls calc_sus (before G = F - G,
 // SRC/loop.f90:193-222); after a device iteration they hold Gamma = F - Phi, and
 // Phi is read back as F - Gamma.
-#include "green.h"
-#include "internal.h"
+#include "bubble.h"
 
 #include <cmath>
 
@@ -27,101 +25,13 @@ namespace tups {
 namespace {
 
 struct SusArgs {
-  GreenParams g;
   const double2* fv[4];
   const double2* gam[4];  // Phi (after_update = 0) or Gamma = F - Phi (after_update = 1)
-  const double* ff;       // FF[l Nc + (ky-1) Nx + kx-1]
-  const int* qm;
-  const int* qw;
-  const int* ibz;
   double2* gg;            // [q][2 (ph, pp)][4 ff][nent]
   double2* out;           // [r][ff][q]
-  int nx, nf, nl, nz, nq, nibz, ext, f_range, after_update;
+  int nf, nl, nz, nq, ext, f_range, after_update;
   double bare[4], inv_ff11_sq, norm;
 };
-
-// grid: nq
-__global__ __launch_bounds__(256) void sus_gg(SusArgs a) {
-  __shared__ double2 red[8][256];
-  __shared__ double fsd[4][256];  // FF_sdwave, Nc <= 256
-  const GreenParams g = green_resolve(a.g);
-  const int q = blockIdx.x;
-  const int m = a.qm[q];
-  const int qx = a.ibz[m], qy = a.ibz[a.nibz + m], w = a.qw[q];
-  const int nx = a.nx, nc = nx * nx, nf = a.nf, ng = g.ngrain;
-  const double pi = 3.14159265358979323846;
-  for (int k = threadIdx.x; k < nc; k += 256) {
-    const int kx = k % nx + 1, ky = k / nx + 1;
-    const double px = 2.0 / nx * pi * (kx - 1), py = 2.0 / nx * pi * (ky - 1);
-    fsd[0][k] = 1.0;
-    fsd[1][k] = cos(px) - cos(py);
-    fsd[2][k] = sin(px);
-    fsd[3][k] = sin(px) * sin(py);
-  }
-  __syncthreads();
-  const int nent = a.nl * a.ext;
-  int ks = 1;
-  while (ks * 2 * nent <= 256 && ks * 2 <= nc) ks *= 2;
-  const int per = 256 / ks, part = threadIdx.x % ks, slot = threadIdx.x / ks;
-  const double inv_g2 = 1.0 / ng / ng;
-  double2* out = a.gg + (size_t)q * 8 * nent;
-  for (int e0 = 0; e0 < nent; e0 += per) {
-    const int e = e0 + slot;
-    double2 acc[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) acc[i] = make_double2(0.0, 0.0);
-    if (e < nent) {
-      const int l = e / a.ext, nu = e - l * a.ext - a.f_range * nf + 1;
-      for (int k = part; k < nc; k += ks) {
-        const int kx = k % nx + 1, ky = k / nx + 1;
-        const int kqx = (kx - 1 + qx - 1) % nx + 1, kqy = (ky - 1 + qy - 1) % nx + 1;
-        const int mkx = (-(kx - 1) + nx) % nx + 1, mky = (-(ky - 1) + nx) % nx + 1;
-        const int qmkx = (mkx - 1 + qx - 1) % nx + 1, qmky = (mky - 1 + qy - 1) % nx + 1;
-        double2 sph = make_double2(0.0, 0.0), spp = make_double2(0.0, 0.0);
-        for (int gy = 1; gy <= ng; ++gy)
-          for (int gx = 1; gx <= ng; ++gx) {
-            const double2 gk = green_coarse(g, gx, gy, kx, ky, nu);
-            const double2 p = cmul(gk, green_coarse(g, gx, gy, kqx, kqy, nu + w - 1));
-            const double2 t = cmul(gk, green_coarse(g, ng - gx + 1, ng - gy + 1, qmkx, qmky, -nu + nf + 1 + w - 1));
-            sph.x += p.x * inv_g2;
-            sph.y += p.y * inv_g2;
-            spp.x += t.x * inv_g2;
-            spp.y += t.y * inv_g2;
-          }
-        const double fl = a.ff[(size_t)l * nc + k];
-#pragma unroll
-        for (int f = 0; f < 4; ++f) {
-          const double wgt = fsd[f][k] * fl;
-          acc[f].x += wgt * sph.x;
-          acc[f].y += wgt * sph.y;
-          acc[4 + f].x += wgt * spp.x;
-          acc[4 + f].y += wgt * spp.y;
-        }
-      }
-    }
-    if (ks == 1) {
-      if (e < nent)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) out[(size_t)i * nent + e] = acc[i];
-      continue;
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) red[i][threadIdx.x] = acc[i];
-    __syncthreads();
-    if (part == 0 && e < nent) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        double2 s = red[i][threadIdx.x];
-        for (int t = 1; t < ks; ++t) {
-          s.x += red[i][threadIdx.x + t].x;
-          s.y += red[i][threadIdx.x + t].y;
-        }
-        out[(size_t)i * nent + e] = s;
-      }
-    }
-    __syncthreads();
-  }
-}
 
 // grid: (nq, 4 channels)
 __global__ __launch_bounds__(256) void sus_contract(SusArgs a) {
@@ -207,8 +117,8 @@ extern "C" int tups_calc_sus(tups_ctx* c, double u, int32_t f_range, int32_t aft
   if (rc) return rc;
   GreenParams g{};
   if ((rc = green_params(c, &g))) return rc;
+  if ((rc = green_tab_reserve(c, g.ngrain, f_range))) return rc;
   SusArgs a{};
-  a.g = g;
   a.ext = (2 * f_range + 1) * s.nf;
   const size_t nent = (size_t)s.nl * a.ext;
   const size_t need = ((size_t)s.nq * 8 * nent + 16 * (size_t)s.nq) * sizeof(double2);
@@ -225,16 +135,10 @@ extern "C" int tups_calc_sus(tups_ctx* c, double u, int32_t f_range, int32_t aft
     a.fv[r] = c->fvert[r];
     a.gam[r] = c->gamma[r];
   }
-  a.ff = c->d_ffk;
-  a.qm = c->d_qm;
-  a.qw = c->d_qw;
-  a.ibz = c->d_ibz;
-  a.nx = s.nx;
   a.nf = s.nf;
   a.nl = s.nl;
   a.nz = s.nz;
   a.nq = s.nq;
-  a.nibz = s.nibz;
   a.f_range = f_range;
   a.after_update = after_update ? 1 : 0;
   a.bare[0] = u;
@@ -245,8 +149,8 @@ extern "C" int tups_calc_sus(tups_ctx* c, double u, int32_t f_range, int32_t aft
   a.inv_ff11_sq = 1.0 / (f11 * f11);
   a.norm = 1.0 / ((double)s.nx * s.nx * s.ny * s.ny * c->beta * c->beta);
   if ((rc = timer_begin(c))) return rc;
-  hipLaunchKernelGGL(sus_gg, dim3((unsigned)s.nq), dim3(256), 0, c->stream, a);
-  TUPS_HIP(hipGetLastError());
+  const BubbleOut out[2] = {{a.gg, a.gg + 4 * nent, (long long)(8 * nent), 1, a.ext}, {}};
+  if ((rc = launch_bubbles(c, g, f_range, kBubbleSus, out, nullptr))) return rc;
   hipLaunchKernelGGL(sus_contract, dim3((unsigned)s.nq, 4), dim3(256), 0, c->stream, a);
   TUPS_HIP(hipGetLastError());
   if ((rc = timer_end(c, TUPS_K_SUS))) return rc;
