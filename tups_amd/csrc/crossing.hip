@@ -26,6 +26,8 @@
 // term depends on q only through qw), then stream Phi -> F adding the terms
 // and Lambda*Nc on the l=1 block (SRC/parquet_EQOuter.f90:48-59): F is read
 // (as Phi) and written exactly once, the minimum traffic of the crossing.
+#include <cstring>
+
 #include "internal.h"
 #include "lds_dma.h"
 
@@ -133,12 +135,24 @@ struct PaeNl1Args {
   const double2* phir[4];  // PhiR of d, m, s, t (the fused variants re-index them in place)
   const double2* phi[4];
   double2* F[4];
+  double2* G[4];           // null, or where G = F - Phi goes (SRC/loop.f90:219-222)
   const double2* lam[4];
   const double2* M[4];
   const double2* Y;
   int nf, nw, nibz, nr, nq;
   double inv_nx, nc_aux;
 };
+
+// the two targets' F, and G = F - Phi beside it where the caller takes it
+__device__ __forceinline__ void put_pair(const PaeNl1Args& a, int ta, size_t idx, double2 oa, double2 ob, double2 pa,
+                                         double2 pb) {
+  st_stream(a.F[ta] + idx, oa);
+  st_stream(a.F[ta + 1] + idx, ob);
+  if (a.G[ta]) {
+    st_stream(a.G[ta] + idx, make_double2(oa.x - pa.x, oa.y - pa.y));
+    st_stream(a.G[ta + 1] + idx, make_double2(ob.x - pb.x, ob.y - pb.y));
+  }
+}
 
 // one thread per (nu1, nu2) entry of one (q, target pair), C columns per
 // thread; with NR1 (one real-space shell) every load of all C columns is
@@ -214,8 +228,7 @@ __global__ __launch_bounds__(256) void pae_stream_nl1(PaeNl1Args a) {
     ob.x += lb[c].x * a.nc_aux + sb.x * a.inv_nx;
     ob.y += lb[c].y * a.nc_aux + sb.y * a.inv_nx;
     const size_t idx = (size_t)nu1 + (size_t)nf * nu2 + nf2 * q;
-    st_stream(a.F[ta] + idx, oa);
-    st_stream(a.F[tb] + idx, ob);
+    put_pair(a, ta, idx, oa, ob, fa[c], fb[c]);
   }
 }
 
@@ -267,8 +280,7 @@ __global__ __launch_bounds__(256) void pae_stream_nl1_mom(PaeNl1Args a) {
     ob.x += lb.x * a.nc_aux + (m0.x * yb0.x - m0.y * yb0.y + m1.x * yb1.x - m1.y * yb1.y) * a.inv_nx;
     ob.y += lb.y * a.nc_aux + (m0.x * yb0.y + m0.y * yb0.x + m1.x * yb1.y + m1.y * yb1.x) * a.inv_nx;
     const size_t idx = (size_t)nu1 + (size_t)nf * nu2 + nf2 * ((size_t)m * nw + w0);
-    st_stream(a.F[ta] + idx, oa);
-    st_stream(a.F[tb] + idx, ob);
+    put_pair(a, ta, idx, oa, ob, fa[k], fb[k]);
   }
 }
 
@@ -322,8 +334,7 @@ __global__ __launch_bounds__(256) void pae_stream_nl1_fused(PaeNl1Args a) {
     ob.x += lb.x * a.nc_aux + (m0.x * yb0.x - m0.y * yb0.y + m1.x * yb1.x - m1.y * yb1.y) * a.inv_nx;
     ob.y += lb.y * a.nc_aux + (m0.x * yb0.y + m0.y * yb0.x + m1.x * yb1.y + m1.y * yb1.x) * a.inv_nx;
     const size_t idx = (size_t)nu1 + (size_t)nf * nu2 + nf2 * ((size_t)m * nw + w0);
-    st_stream(a.F[ta] + idx, oa);
-    st_stream(a.F[tb] + idx, ob);
+    put_pair(a, ta, idx, oa, ob, fa[k], fb[k]);
   }
 }
 
@@ -395,8 +406,7 @@ __global__ __launch_bounds__(256, 8) void pae_stream_nl1_all(PaeNl1Args a) {
       oa.y += la.y * a.nc_aux + (m0.x * ya0.y + m0.y * ya0.x + m1.x * ya1.y + m1.y * ya1.x) * a.inv_nx;
       ob.x += lb.x * a.nc_aux + (m0.x * yb0.x - m0.y * yb0.y + m1.x * yb1.x - m1.y * yb1.y) * a.inv_nx;
       ob.y += lb.y * a.nc_aux + (m0.x * yb0.y + m0.y * yb0.x + m1.x * yb1.y + m1.y * yb1.x) * a.inv_nx;
-      st_stream(a.F[ta] + base + mstride * m, oa);
-      st_stream(a.F[tb] + base + mstride * m, ob);
+      put_pair(a, ta, base + mstride * m, oa, ob, fa[k], fb[k]);
     }
     if (PF) {
 #pragma unroll
@@ -476,8 +486,7 @@ __global__ __launch_bounds__(256, 8 / EPT) void pae_stream_nl1_multi(PaeNl1Args 
       oa.y += la[e].y * a.nc_aux + (m0.x * ya0[e].y + m0.y * ya0[e].x + m1.x * ya1[e].y + m1.y * ya1[e].x) * a.inv_nx;
       ob.x += lb[e].x * a.nc_aux + (m0.x * yb0[e].x - m0.y * yb0[e].y + m1.x * yb1[e].x - m1.y * yb1[e].y) * a.inv_nx;
       ob.y += lb[e].y * a.nc_aux + (m0.x * yb0[e].y + m0.y * yb0[e].x + m1.x * yb1[e].y + m1.y * yb1[e].x) * a.inv_nx;
-      st_stream(a.F[ta] + base[e] + mstride * m, oa);
-      st_stream(a.F[tb] + base[e] + mstride * m, ob);
+      put_pair(a, ta, base[e] + mstride * m, oa, ob, fa[e], fb[e]);
     }
 #pragma unroll
     for (int e = 0; e < EPT; ++e) {
@@ -535,13 +544,14 @@ static int pae_nl1_launch(tups_ctx* c, int v, const PaeNl1Args& b) {
   return TUPS_OK;
 }
 
-static PaeNl1Args nl1_args(tups_ctx* c) {
+static PaeNl1Args nl1_args(tups_ctx* c, bool update) {
   const tups_sizes& s = c->sz;
   PaeNl1Args b{};
   for (int r = 0; r < 4; ++r) {
     b.phir[r] = c->phir[r];
     b.phi[r] = c->gamma[r];
     b.F[r] = c->fvert[r];
+    b.G[r] = update ? c->spare[r] : nullptr;
     b.lam[r] = c->lam[r];
     b.M[r] = c->mten[r];
   }
@@ -572,7 +582,7 @@ static int pae_pregather(tups_ctx* c) {
 int autotune_pae(tups_ctx* c, int reps, int* chosen, float* best_ms) {
   TUPS_CHECK(c->sz.nl == 1 && c->pae_y, TUPS_EINVAL, "crossing variants exist for Nl = 1 only");
   if (int rc = pae_pregather(c)) return rc;
-  const PaeNl1Args b = nl1_args(c);
+  const PaeNl1Args b = nl1_args(c, false);
   float best = 0.f;
   int arg = -1;
   for (int v = 0; v < kNumPaeVariants; ++v) {
@@ -622,6 +632,7 @@ int autotune_pae(tups_ctx* c, int reps, int* chosen, float* best_ms) {
 struct PaeMmArgs {
   const double2* phi[4];
   double2* F[4];
+  double2* G[4];  // null, or where G = F - Phi goes
   const double2* lam[4];
   const double2* M[4];
   const double2* phir[4];
@@ -858,7 +869,8 @@ __global__ __launch_bounds__(256, 4) void pae_mm(PaeMmArgs a) {
         const int l1 = l % nl, l2 = l / nl;
         const size_t q = (size_t)m * a.nw + w0;
         const size_t idx = q * nz2 + (size_t)(l2 * nf + nu2) * nz + (size_t)(l1 * nf + nu1);
-        double2 o = a.phi[tgt][idx];
+        const double2 f = a.phi[tgt][idx];
+        double2 o = f;
         if (l == 0) {
           const double2 lv = a.lam[tgt][(size_t)nu1 + (size_t)nf * ((size_t)nu2 + (size_t)nf * w0)];
           o.x += lv.x * a.nc_aux;
@@ -867,6 +879,7 @@ __global__ __launch_bounds__(256, 4) void pae_mm(PaeMmArgs a) {
         o.x += acc_re[i][j][e] * a.inv_nx;
         o.y += acc_im[i][j][e] * a.inv_nx;
         a.F[tgt][idx] = o;
+        if (a.G[tgt]) a.G[tgt][idx] = make_double2(o.x - f.x, o.y - f.y);
       }
     }
 }
@@ -966,25 +979,28 @@ __global__ __launch_bounds__(256, 3) void pae_sparse(PaeMmArgs a) {
   for (int t = 0; t < 2; ++t) {
     const double2* phi = a.phi[2 * p + t] + col;
     double2* F = a.F[2 * p + t] + col;
-    double2 o[kPlanSlots][4];
+    double2* G = a.G[2 * p + t] ? a.G[2 * p + t] + col : nullptr;
+    double2 f[kPlanSlots][4];
 #pragma unroll
     for (int i = 0; i < kPlanSlots; ++i)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        if (off[i][e] >= 0) o[i][e] = phi[off[i][e] >> 1];
+        if (off[i][e] >= 0) f[i][e] = phi[off[i][e] >> 1];
 #pragma unroll
     for (int i = 0; i < kPlanSlots; ++i)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         if (off[i][e] < 0) continue;
+        double2 o = f[i][e];
         if (off[i][e] & 1) {
           const double2 lv = a.lam[2 * p + t][(size_t)nu1 + (size_t)nf * ((size_t)nu2 + (size_t)nf * w0)];
-          o[i][e].x += lv.x * a.nc_aux;
-          o[i][e].y += lv.y * a.nc_aux;
+          o.x += lv.x * a.nc_aux;
+          o.y += lv.y * a.nc_aux;
         }
-        o[i][e].x += re[t][i][e] * a.inv_nx;
-        o[i][e].y += im[t][i][e] * a.inv_nx;
-        F[off[i][e] >> 1] = o[i][e];
+        o.x += re[t][i][e] * a.inv_nx;
+        o.y += im[t][i][e] * a.inv_nx;
+        F[off[i][e] >> 1] = o;
+        if (G) G[off[i][e] >> 1] = make_double2(o.x - f[i][e].x, o.y - f[i][e].y);
       }
   }
 }
@@ -1038,12 +1054,13 @@ void pae_plan_free(tups_ctx* c) {
   c->pae_plan = nullptr;
 }
 
-static PaeMmArgs mm_args(tups_ctx* c) {
+static PaeMmArgs mm_args(tups_ctx* c, bool update) {
   const tups_sizes& s = c->sz;
   PaeMmArgs a{};
   for (int r = 0; r < 4; ++r) {
     a.phi[r] = c->gamma[r];
     a.F[r] = c->fvert[r];
+    a.G[r] = update ? c->spare[r] : nullptr;
     a.lam[r] = c->lam[r];
     a.M[r] = c->mten[r];
     a.phir[r] = c->phir[r];
@@ -1075,7 +1092,7 @@ static PaeMmArgs mm_args(tups_ctx* c) {
 int pae_plan_ensure(tups_ctx* c) {
   const tups_sizes& s = c->sz;
   if (c->pae_plan_valid || s.nl == 1 || !c->pae_ym || !c->m_built) return TUPS_OK;
-  PaeMmArgs a = mm_args(c);
+  PaeMmArgs a = mm_args(c, false);
   const int nl2 = s.nl * s.nl;
   drop_graphs(c);  // they hold the old plan's pointers
   ++c->pae_plan_gen;
@@ -1172,9 +1189,9 @@ int pae_plan_ensure(tups_ctx* c) {
   return TUPS_OK;
 }
 
-static int pae_gemm_path(tups_ctx* c) {
+static int pae_gemm_path(tups_ctx* c, bool update) {
   const tups_sizes& s = c->sz;
-  PaeMmArgs a = mm_args(c);
+  PaeMmArgs a = mm_args(c, update);
   TUPS_CHECK(c->pae_plan && c->pae_plan_valid, TUPS_ESTATE, "crossing without a plan for M");
   const PaePlan& pl = *c->pae_plan;
   if (!pl.dense) {
@@ -1220,21 +1237,35 @@ static int pae_gemm_path(tups_ctx* c) {
   return TUPS_OK;
 }
 
-int launch_pae(tups_ctx* c) {
+// The variant without autotuning, times in us at (Nx, Nf) of it | pre-pass + 4 columns:
+// up to Nf = 16 the all-momenta form, whose few workgroups each do all of the work of
+// their entries (4, 16: 4.8 | 6.5); 56 < Nf <= 64 fills the rows of its 64-wide tiles and
+// four entries per thread put one workgroup on each CU ((8, 64): 52 | 74, (16, 64): 141 |
+// 188); else 16 momenta per thread with PhiR re-indexed on the way ((6, 30): 7.1 | 11.7,
+// (8, 32): 8.0 | 15.9, (20, 40): 57 | 85, (8, 128): 397 | 553, (16, 96): 518 | 770).
+static int pae_default(const tups_ctx* c) {
+  const tups_sizes& s = c->sz;
+  const char* name = s.nr != 1 ? "nl1_c4_nr" : s.nf <= 16 ? "nl1_a2" : s.nf > 56 && s.nf <= 64 ? "nl1_e4p" : "nl1_f16";
+  for (int v = 0; v < kNumPaeVariants; ++v)
+    if (std::strcmp(kPaeVariants[v].name, name) == 0) return v;
+  return 1;
+}
+
+int launch_pae(tups_ctx* c, bool update) {
   const tups_sizes& s = c->sz;
   if (s.nl > 1) {
     TUPS_CHECK(c->pae_ym, TUPS_ESTATE, "crossing operand buffer missing (not a full-IBZ context)");
-    return pae_gemm_path(c);
+    return pae_gemm_path(c, update);
   }
   TUPS_CHECK(c->pae_y, TUPS_ESTATE, "crossing operand buffer missing (not a full-IBZ context)");
   int v = c->pae_variant;
-  if (!pae_variant_ok(c, v)) v = s.nr == 1 ? 1 : 3;
+  if (!pae_variant_ok(c, v)) v = pae_default(c);
   if (!kPaeVariants[v].fused) {
     if (int rc = timer_begin(c)) return rc;
     if (int rc = pae_pregather(c)) return rc;
     if (int rc = timer_end(c, TUPS_K_PAE_GATHER)) return rc;
   }
-  const PaeNl1Args b = nl1_args(c);
+  const PaeNl1Args b = nl1_args(c, update);
   if (int rc = timer_begin(c)) return rc;
   if (int rc = pae_nl1_launch(c, v, b)) return rc;
   if (int rc = timer_end(c, TUPS_K_PAE)) return rc;

@@ -279,7 +279,8 @@ const char* pae_variant_name(int v);
 bool pae_variant_ok(const tups_ctx* c, int v);
 int launch_phir(tups_ctx* c);
 int launch_build_m(tups_ctx* c);
-int launch_pae(tups_ctx* c);
+// update: also G = F - Phi into the spare vertex buffers (the caller swaps them in)
+int launch_pae(tups_ctx* c, bool update = false);
 // builds the crossing plan of M when it is stale; before a launch or a capture of launch_pae.  Synchronous
 int pae_plan_ensure(tups_ctx* c);
 void pae_plan_free(tups_ctx* c);
