@@ -154,6 +154,13 @@ __device__ __forceinline__ void static_for(F&& f) {
   }
 }
 
+// consecutive workgroups go round-robin over the 8 XCDs: a contiguous range each
+__device__ __forceinline__ int closed_xcd_remap(int bid, int nblk) {
+  const int xcd = bid & 7, idx = bid >> 3;
+  const int per = nblk >> 3, rem = nblk & 7;
+  return xcd < rem ? xcd * (per + 1) + idx : rem * (per + 1) + (xcd - rem) * per + idx;
+}
+
 struct ClosedArgs {
   const double2* gam[4];
   double2* out[4];
@@ -161,6 +168,8 @@ struct ClosedArgs {
   void* W;      // [mat][2D columns][D rows], column-major: double2 (direct) or float2 (inverse)
   void* S;      // closed_solve_b64: [mat][CL_BB columns][D rows], the block column being factored
   void* T;      // closed_solve_b64: [mat][2][CL_BB][CL_BB], L11^-1 (then T = U11^-1 L11^-1) and U11^-1
+  double2* gx;  // refinement mode: [mat][D][D] Gamma chi in FP64
+  float2* g32;  // and fp32(Gamma), the first right-hand side of the inverse
   int* info;    // first failing pivot (1-based column) over all matrices, 0 if none
   int D, nf, nl, q0, nqb;
   double kappa[4];
@@ -173,7 +182,9 @@ __global__ void closed_clear(int* info) { *info = 0; }
 // matrix) forms the Nl columns (l2, nu) of the left block from the Nl columns
 // (l1, nu) of Gamma, each read once: (Gamma chi)(row, (l2, nu)) =
 // sum_l1 Gamma(row, (l1, nu)) chi_nu(l1, l2), and writes the columns (l1, nu)
-// of the right block from the same reads.  grid: (Nf, 4 nqb); one thread per row.
+// of the right block from the same reads; in refinement mode also Gamma chi itself,
+// which the residuals multiply with, and the rounded Gamma.  grid: (Nf, 4 nqb); one
+// thread per row.
 constexpr int CL_NL_MAX = 9;
 template <class T, bool IR>
 __global__ __launch_bounds__(256) void closed_build_nu(ClosedArgs a) {
@@ -197,8 +208,10 @@ __global__ __launch_bounds__(256) void closed_build_nu(ClosedArgs a) {
         const int j = l1 * nf + nu;
         g[l1] = G[(size_t)j * D + row];
         // the right-hand side: Gamma's column j (the identity's for the FP32 inverse)
-        if constexpr (IR) W[(size_t)(D + j) * D + row] = put(row == j ? 1.0 : 0.0, 0.0);
-        else W[(size_t)(D + j) * D + row] = g[l1];
+        if constexpr (IR) {
+          W[(size_t)(D + j) * D + row] = put(row == j ? 1.0 : 0.0, 0.0);
+          a.g32[((size_t)mat * D + j) * D + row] = put(g[l1].x, g[l1].y);
+        } else W[(size_t)(D + j) * D + row] = g[l1];
       }
     for (int l2 = 0; l2 < nl; ++l2) {
       double sr = 0.0, si = 0.0;
@@ -211,6 +224,7 @@ __global__ __launch_bounds__(256) void closed_build_nu(ClosedArgs a) {
         }
       const int j = l2 * nf + nu;
       W[(size_t)j * D + row] = put((row == j ? 1.0 : 0.0) - kap * sr, -kap * si);
+      if constexpr (IR) a.gx[((size_t)mat * D + j) * D + row] = make_double2(sr, si);
     }
   }
 }
@@ -1245,73 +1259,148 @@ __global__ __launch_bounds__(256, 2) void closed_solve_b64(ClosedArgs a) {
 struct IrArgs {
   const double2* gam[4];
   double2* x[4];             // X_r, the solution, in the output arrays
-  const double2* chi[2];
   const float2* inv;         // [mat][2D][D]: the inverse is columns D..2D-1
-  const double2* b;          // [mat][D][D] FP64 right-hand side of an apply (Gamma when null)
-  double2* rres;             // [mat][D][D] residual R
-  double2* y;                // [mat][D][D] chi X
+  float2* rhs;               // [mat][D][D] right-hand side of the next product: fp32(Gamma), then fp32(R)
+  const double2* gx;         // [mat][D][D] Gamma chi
   double* part;              // [mat][tiles][2]: sum |R|^2, sum |Gamma|^2 per tile
   double* res;               // [mat] |R|_F / |Gamma|_F
   unsigned long long* rmax;  // bits of the largest res (non-negative doubles order as integers)
-  int D, nf, nl, q0, nqb, tiles_n;
+  int D, q0, nqb, tiles_n;
   double kappa[4];
 };
 
 __global__ void ir_clear(unsigned long long* rmax) { *rmax = 0ull; }
 
-// Y = chi X: Y((l1, nu), c) = sum_l2 chi_nu(l1, l2) X((l2, nu), c), X the
-// solution in the output arrays.  One workgroup per (IR_CHI_COLS columns,
-// matrix); thread t takes the pairs u = t + 256 k of (nu, c), nu fastest,
-// and forms all Nl rows (l1, nu) of each from the Nl entries (l2, nu) of
-// column c, each read once.  grid: (ceil(D / IR_CHI_COLS), 4 nqb)
-constexpr int IR_CHI_COLS = 16;
-__global__ __launch_bounds__(256) void ir_chi(IrArgs a) {
-  const int mat = blockIdx.y, c0 = blockIdx.x * IR_CHI_COLS;
-  const int r = mat / a.nqb, q = a.q0 + (mat - r * a.nqb);
-  const int D = a.D, nf = a.nf, nl = a.nl;
-  const double2* X = a.x[r] + (size_t)D * D * q;
-  double2* Y = a.y + (size_t)mat * D * D;
-  const double2* cq = a.chi[r >> 1] + (size_t)nf * nl * nl * q;
-  const int ncols = min(IR_CHI_COLS, D - c0);
-  for (int u = threadIdx.x; u < nf * ncols; u += 256) {
-    const int nu = u % nf, c = c0 + u / nf;
-    const double2* cb = cq + (size_t)nu * nl * nl;
-    const double2* Xc = X + (size_t)c * D + nu;
-    double2* Yc = Y + (size_t)c * D + nu;
-    double2 x[CL_NL_MAX];
+// Chunks of the inner index in the products below: 16 KiB a stage (A and B), three
+// stages, so two chunks are in flight while one multiplies and three workgroups share a
+// CU.
+template <class R>
+constexpr int ir_kc() {
+  return sizeof(R) == 8 ? 8 : 16;
+}
+constexpr int IR_STAGES = 3;
+
+// A 64 x 64 tile at (tr, tc) of A B, both D x D column-major (D even), by a ring of LDS
+// stages filled with direct global-to-LDS loads; four waves of 2 x 2 blocks of 16 x 16 x 4
+// MFMAs.  One barrier per chunk: after it every wave is done with the chunk before, whose
+// stage takes the chunk two ahead.  A stage holds A as [k][row] and B as [column][k], its
+// 16-byte pieces (a double2, two float2) XOR-swizzled by the column, so 8 consecutive
+// lanes of a fragment read cover 32 banks or more.  Rows, columns and inner indices
+// beyond D load clamped addresses: the products of such inner indices are masked in the
+// last chunk, rows and columns dropped by the caller.  The register-fed form without
+// prefetch took 11.39 ms for the FP64 residual (and 4.08 ms more to form chi X) and 5.7 ms
+// for an FP32 product at D = 320, 480 q; this one 8.17 and 4.5 ms (61.6 and 112 TFLOP/s).
+template <class R>
+__device__ __forceinline__ void ir_tile(const typename Prec<R>::C* A, const typename Prec<R>::C* B, int D, int tr,
+                                        int tc, char* lds, typename Prec<R>::V (&ar)[2][2],
+                                        typename Prec<R>::V (&ai)[2][2]) {
+  using P = Prec<R>;
+  using C = typename P::C;
+  constexpr int KC = ir_kc<R>();
+  constexpr int E = 16 / sizeof(C);           // elements of a 16-byte piece
+  constexpr int RP = CL_T / E, KP = KC / E;   // pieces per row of A (one k) and per column of B
+  constexpr int STAGE = 2 * KC * CL_T * (int)sizeof(C), HALF = STAGE / 2;
+  static_assert(HALF == 8192 && KP == 8, "16 KiB stages of 8 pieces a column");
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
+  const int li = lane & 15, lk = lane >> 4;
+  const int nch = (D + KC - 1) / KC;
+  const unsigned lbase = lds_addr(lds);
+  // this lane's pieces: of A, slots (wave + 4 v) 64 + lane -> k = slot / RP, piece slot % RP;
+  // of B, slot -> column slot / 8, piece (slot % 8) ^ (column % 8)
+  int ak[2], arow[2], bk[2], bcol[2];
 #pragma unroll
-    for (int l2 = 0; l2 < CL_NL_MAX; ++l2)
-      if (l2 < nl) x[l2] = Xc[(size_t)l2 * nf];
-    for (int l1 = 0; l1 < nl; ++l1) {
-      double sr = 0.0, si = 0.0;
+  for (int v = 0; v < 2; ++v) {
+    const int slot = (wave + 4 * v) * 64 + lane;
+    ak[v] = slot / RP;
+    arow[v] = min(tr + (slot % RP) * E, D - E);
+    bcol[v] = min(tc + slot / KP, D - 1);
+    bk[v] = ((slot % KP) ^ ((slot / KP) % KP)) * E;
+  }
+  auto issue = [&](int ch) {
+    const unsigned st = lbase + (ch % IR_STAGES) * STAGE;
+    const int k0 = ch * KC;
 #pragma unroll
-      for (int l2 = 0; l2 < CL_NL_MAX; ++l2)
-        if (l2 < nl) {
-          const double2 cc = cb[l1 + nl * l2];
-          sr += cc.x * x[l2].x - cc.y * x[l2].y;
-          si += cc.x * x[l2].y + cc.y * x[l2].x;
-        }
-      Yc[(size_t)l1 * nf] = make_double2(sr, si);
+    for (int v = 0; v < 2; ++v) {
+      const int k = min(k0 + ak[v], D - 1);
+      dma16(A, (unsigned)(((size_t)k * D + arow[v]) * sizeof(C)), st + (wave + 4 * v) * 1024);
     }
+#pragma unroll
+    for (int v = 0; v < 2; ++v) {
+      const int k = min(k0 + bk[v], D - E);
+      dma16(B, (unsigned)(((size_t)bcol[v] * D + k) * sizeof(C)), st + HALF + (wave + 4 * v) * 1024);
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) ar[i][j][e] = ai[i][j][e] = 0;
+  auto steps = [&](const char* st, int left, auto masked) {
+    const C* sa = reinterpret_cast<const C*>(st);
+    const char* sb = st + HALF;
+#pragma unroll
+    for (int kk = 0; kk < KC; kk += 4) {
+      if (masked.value && kk >= left) break;
+      const int k = kk + lk;
+      C fa[2], fb[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) fa[i] = sa[k * CL_T + wr + i * 16 + li];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int col = wc + j * 16 + li;
+        fb[j] = *reinterpret_cast<const C*>(sb + (col * KP + ((k / E) ^ (col % KP))) * 16 + (k % E) * sizeof(C));
+      }
+      if (masked.value && k >= left)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) fa[i] = fb[i] = mkc((R)0, (R)0);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          ar[i][j] = P::fma_add(fa[i].x, fb[j].x, ar[i][j]);
+          ai[i][j] = P::fma_add(fa[i].x, fb[j].y, ai[i][j]);
+          ar[i][j] = P::fma_sub(fa[i].y, fb[j].y, ar[i][j]);
+          ai[i][j] = P::fma_add(fa[i].y, fb[j].x, ai[i][j]);
+        }
+    }
+  };
+  issue(0);
+  if (nch > 1) issue(1);
+  for (int ch = 0; ch < nch; ++ch) {
+    // this wave's four loads of chunk ch have landed (those of ch + 1 may be in flight)
+    if (ch + 1 < nch)
+      wait_vmcnt<4>();
+    else
+      wait_vmcnt<0>();
+    stage_barrier();
+    if (ch + 2 < nch) issue(ch + 2);
+    const char* st = lds + (ch % IR_STAGES) * STAGE;
+    if ((ch + 1) * KC <= D)
+      steps(st, KC, std::false_type{});
+    else
+      steps(st, D - ch * KC, std::true_type{});
   }
 }
 
-// 64 x 64 tile of a batched complex product per workgroup (four waves of 2 x 2
-// blocks of 16 x 16 x 4 MFMAs), K in chunks of 16 through LDS.
-//   MODE 0: X  = fp64(A32^-1 fp32(B))    MODE 1: X += fp64(A32^-1 fp32(B))
-//   MODE 2: R  = Gamma - X + kappa Gamma Y (FP64), with per-tile |R|^2, |Gamma|^2
+// Batched complex products of the refinement, one 64 x 64 tile per workgroup, the tiles of
+// a matrix on one XCD so that they share its L2.
+//   MODE 0: X  = fp64(A32^-1 fp32(Gamma))    MODE 1: X += fp64(A32^-1 fp32(R))
+//   MODE 2: R  = Gamma - X + kappa (Gamma chi) X in FP64, kept as fp32(R), the only form a
+//           product reads, with per-tile |R|^2, |Gamma|^2 of the FP64 values
 // grid: tiles_n^2 * 4 nqb
 template <int MODE>
-__global__ __launch_bounds__(256) void ir_gemm(IrArgs a) {
+__global__ __launch_bounds__(256, 3) void ir_gemm(IrArgs a) {
   using R = typename std::conditional<MODE == 2, double, float>::type;
   using P = Prec<R>;
   using C = typename P::C;
   using V = typename P::V;
-  __shared__ C As[CL_NB][CL_T + 1];
-  __shared__ C Bs[CL_NB][CL_T + 1];
-  __shared__ double red[2][256];
+  __shared__ __attribute__((aligned(16))) char stage[IR_STAGES * 16384];
   const int tiles = a.tiles_n * a.tiles_n;
-  const int mat = blockIdx.x / tiles, t = blockIdx.x - mat * tiles;
+  const int logical = closed_xcd_remap(blockIdx.x, gridDim.x);
+  const int mat = logical / tiles, t = logical - mat * tiles;
   const int tr = (t / a.tiles_n) * CL_T, tc = (t % a.tiles_n) * CL_T;
   const int r = mat / a.nqb, q = a.q0 + (mat - r * a.nqb);
   const int D = a.D;
@@ -1321,53 +1410,14 @@ __global__ __launch_bounds__(256) void ir_gemm(IrArgs a) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
   const int li = lane & 15, lk = lane >> 4;
-  const C zero = mkc((R)0, (R)0);
   V ar[2][2], ai[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) ar[i][j][e] = ai[i][j][e] = 0;
-  const double2* Bsrc = MODE == 2 ? a.y + DD * mat : (a.b ? a.b + DD * mat : G);
-  for (int k0 = 0; k0 < D; k0 += CL_NB) {
-    for (int u = tid; u < CL_NB * CL_T; u += 256) {
-      const int row = u & (CL_T - 1), ka = u >> 6;
-      const int kb = u % CL_NB, col = u / CL_NB;
-      const bool aok = tr + row < D && k0 + ka < D, bok = tc + col < D && k0 + kb < D;
-      if (MODE == 2) {
-        As[ka][row] = aok ? reinterpret_cast<const C*>(G)[(size_t)(k0 + ka) * D + tr + row] : zero;
-        Bs[kb][col] = bok ? reinterpret_cast<const C*>(Bsrc)[(size_t)(tc + col) * D + k0 + kb] : zero;
-      } else {
-        As[ka][row] = aok ? reinterpret_cast<const C*>(a.inv + 2 * DD * mat + DD)[(size_t)(k0 + ka) * D + tr + row]
-                          : zero;
-        const double2 v = bok ? Bsrc[(size_t)(tc + col) * D + k0 + kb] : make_double2(0.0, 0.0);
-        Bs[kb][col] = mkc((R)v.x, (R)v.y);
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < CL_NB; kk += 4) {
-      C fa[2], fb[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) fa[i] = As[kk + lk][wr + i * 16 + li];
-#pragma unroll
-      for (int j = 0; j < 2; ++j) fb[j] = Bs[kk + lk][wc + j * 16 + li];
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          ar[i][j] = P::fma_add(fa[i].x, fb[j].x, ar[i][j]);
-          ar[i][j] = P::fma_sub(fa[i].y, fb[j].y, ar[i][j]);
-          ai[i][j] = P::fma_add(fa[i].x, fb[j].y, ai[i][j]);
-          ai[i][j] = P::fma_add(fa[i].y, fb[j].x, ai[i][j]);
-        }
-    }
-    __syncthreads();
-  }
+  if constexpr (MODE == 2)
+    ir_tile<R>(a.gx + DD * mat, X, D, tr, tc, stage, ar, ai);
+  else
+    ir_tile<R>(a.inv + 2 * DD * mat + DD, a.rhs + DD * mat, D, tr, tc, stage, ar, ai);
   double rr = 0.0, gg = 0.0;
   const double kap = a.kappa[r];
-  double2* Rm = a.rres + DD * mat;
+  float2* Rm = a.rhs + DD * mat;
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -1385,12 +1435,14 @@ __global__ __launch_bounds__(256) void ir_gemm(IrArgs a) {
         } else {
           const double2 g = G[idx], x = X[idx];
           const double2 v = make_double2(g.x - x.x + kap * ar[i][j][e], g.y - x.y + kap * ai[i][j][e]);
-          Rm[idx] = v;
+          Rm[idx] = make_float2((float)v.x, (float)v.y);
           rr += v.x * v.x + v.y * v.y;
           gg += g.x * g.x + g.y * g.y;
         }
       }
   if (MODE == 2) {
+    double (*red)[256] = reinterpret_cast<double (*)[256]>(stage);
+    __syncthreads();  // the stages are free
     red[0][tid] = rr;
     red[1][tid] = gg;
     __syncthreads();
@@ -1541,9 +1593,10 @@ int launch_bse_closed_ir(tups_ctx* c) {
   TUPS_CHECK(s.nl <= CL_NL_MAX, TUPS_EINVAL, "closed form: at most 9 form factors");
   const size_t D = s.nz, DD = D * D;
   const int tiles_n = (int)((D + CL_T - 1) / CL_T);
-  // per matrix: [A32 | I] (2 D^2 float2), R and chi X (D^2 double2 each), tile partials, res
+  // per matrix: [A32 | I] (2 D^2 float2), the rounded right-hand side (D^2 float2), Gamma chi (D^2
+  // double2), tile partials, res
   const bool blk = closed_blocked(c);
-  const size_t per_mat = 2 * DD * sizeof(float2) + 2 * DD * sizeof(double2) +
+  const size_t per_mat = 3 * DD * sizeof(float2) + DD * sizeof(double2) +
                          (size_t)tiles_n * tiles_n * 2 * sizeof(double) + sizeof(double) + 64 +
                          (blk ? closed_b64_elems(D) * sizeof(float2) : 0);
   int qbatch = 0;
@@ -1556,20 +1609,16 @@ int launch_bse_closed_ir(tups_ctx* c) {
     b.x[r] = c->spare[r];
     b.kappa[r] = a.kappa[r];
   }
-  b.chi[0] = c->chi[0];
-  b.chi[1] = c->chi[1];
   b.D = a.D;
-  b.nf = a.nf;
-  b.nl = a.nl;
   b.tiles_n = tiles_n;
   const size_t mats_max = 4 * (size_t)qbatch;
   char* base = static_cast<char*>(a.W);
   b.inv = reinterpret_cast<const float2*>(base);
   base += mats_max * 2 * DD * sizeof(float2);
-  b.rres = reinterpret_cast<double2*>(base);
+  b.gx = a.gx = reinterpret_cast<double2*>(base);
   base += mats_max * DD * sizeof(double2);
-  b.y = reinterpret_cast<double2*>(base);
-  base += mats_max * DD * sizeof(double2);
+  b.rhs = a.g32 = reinterpret_cast<float2*>(base);
+  base += mats_max * DD * sizeof(float2);
   b.part = reinterpret_cast<double*>(base);
   base += mats_max * tiles_n * tiles_n * 2 * sizeof(double);
   b.res = reinterpret_cast<double*>(base);
@@ -1598,15 +1647,12 @@ int launch_bse_closed_ir(tups_ctx* c) {
     else
       hipLaunchKernelGGL((closed_solve<float, false>), dim3(mats), dim3(256), 0, c->stream, a);
     TUPS_HIP(hipGetLastError());
-    b.b = nullptr;  // X = A32^-1 Gamma
+    // X = A32^-1 Gamma
     hipLaunchKernelGGL(ir_gemm<0>, dim3(gblk), dim3(256), 0, c->stream, b);
     TUPS_HIP(hipGetLastError());
     int steps = 0;
     double res = INFINITY;
     for (;;) {
-      hipLaunchKernelGGL(ir_chi, dim3((unsigned)((D + IR_CHI_COLS - 1) / IR_CHI_COLS), mats), dim3(256), 0,
-                         c->stream, b);
-      TUPS_HIP(hipGetLastError());
       hipLaunchKernelGGL(ir_clear, dim3(1), dim3(1), 0, c->stream, b.rmax);
       TUPS_HIP(hipGetLastError());
       hipLaunchKernelGGL(ir_gemm<2>, dim3(gblk), dim3(256), 0, c->stream, b);
@@ -1618,7 +1664,7 @@ int launch_bse_closed_ir(tups_ctx* c) {
       TUPS_HIP(hipStreamSynchronize(c->stream));
       std::memcpy(&res, &bits, sizeof(res));
       if (res <= c->ir_tol || steps >= c->ir_max_steps) break;
-      b.b = b.rres;  // X += A32^-1 R
+      // X += A32^-1 R
       hipLaunchKernelGGL(ir_gemm<1>, dim3(gblk), dim3(256), 0, c->stream, b);
       TUPS_HIP(hipGetLastError());
       ++steps;
