@@ -165,9 +165,12 @@ struct ClosedArgs {
   const double2* gam[4];
   double2* out[4];
   const double2* chi[2];
-  void* W;      // [mat][2D columns][D rows], column-major: double2 (direct) or float2 (inverse)
-  void* S;      // closed_solve_b64: [mat][CL_BB columns][D rows], the block column being factored
-  void* T;      // closed_solve_b64: [mat][2][CL_BB][CL_BB], L11^-1 (then T = U11^-1 L11^-1) and U11^-1
+  void* W;      // column-major, double2 (direct) or float2 (refinement): [mat][2D columns][D rows] for
+                // closed_solve, [mat][D columns][D rows] for the block form
+  void* S;      // block form: [mat][CL_BB columns][D rows], the block column being factored
+  void* T;      // block form: [mat][block][2][CL_BB][CL_BB], L_kk^-1 and U_kk^-1
+  int* perm;    // block form: [mat][D + 1]: row i of L U is row perm[i] of A; then whether any row moved
+  int blk;      // the block form
   double2* gx;  // refinement mode: [mat][D][D] Gamma chi in FP64
   float2* g32;  // and fp32(Gamma), the first right-hand side of the inverse
   int* info;    // first failing pivot (1-based column) over all matrices, 0 if none
@@ -178,7 +181,8 @@ struct ClosedArgs {
 __global__ void closed_clear(int* info) { *info = 0; }
 
 // [I - kappa Gamma chi | Gamma] (direct mode) or [fp32(I - kappa Gamma chi) | I]
-// (refinement mode, A formed in FP64 and rounded).  One workgroup per (nu,
+// (refinement mode, A formed in FP64 and rounded); the block form takes the left block
+// only, its right-hand sides come from Gamma itself.  One workgroup per (nu,
 // matrix) forms the Nl columns (l2, nu) of the left block from the Nl columns
 // (l1, nu) of Gamma, each read once: (Gamma chi)(row, (l2, nu)) =
 // sum_l1 Gamma(row, (l1, nu)) chi_nu(l1, l2), and writes the columns (l1, nu)
@@ -192,7 +196,7 @@ __global__ __launch_bounds__(256) void closed_build_nu(ClosedArgs a) {
   const int r = mat / a.nqb, q = a.q0 + (mat - r * a.nqb);
   const int D = a.D, nf = a.nf, nl = a.nl;
   const double2* G = a.gam[r] + (size_t)D * D * q;
-  T* W = static_cast<T*>(a.W) + (size_t)mat * 2 * D * D;
+  T* W = static_cast<T*>(a.W) + (size_t)mat * (a.blk ? 1 : 2) * D * D;
   auto put = [](double re, double im) -> T {
     if constexpr (IR) return make_float2((float)re, (float)im);
     else return make_double2(re, im);
@@ -209,9 +213,11 @@ __global__ __launch_bounds__(256) void closed_build_nu(ClosedArgs a) {
         g[l1] = G[(size_t)j * D + row];
         // the right-hand side: Gamma's column j (the identity's for the FP32 inverse)
         if constexpr (IR) {
-          W[(size_t)(D + j) * D + row] = put(row == j ? 1.0 : 0.0, 0.0);
+          if (!a.blk) W[(size_t)(D + j) * D + row] = put(row == j ? 1.0 : 0.0, 0.0);
           a.g32[((size_t)mat * D + j) * D + row] = put(g[l1].x, g[l1].y);
-        } else W[(size_t)(D + j) * D + row] = g[l1];
+        } else if (!a.blk) {
+          W[(size_t)(D + j) * D + row] = g[l1];
+        }
       }
     for (int l2 = 0; l2 < nl; ++l2) {
       double sr = 0.0, si = 0.0;
@@ -832,18 +838,20 @@ __device__ __forceinline__ void list_moved_rows(const int* piv, int r0, int nr, 
   if (lane == 0) *cnt = ni + __popcll(mo);
 }
 
-// Block Gauss-Jordan with CL_BB-wide blocks, one workgroup per (q, r) matrix.
-// For the block column k0 .. k0 + nb:
-//  A. its rows k0 .. D - 1 are copied to S and factored there (LU with partial
-//     pivoting, CL_NB-wide sub-panels: column-by-column within a sub-panel,
-//     then the sub-panel's rank-CL_NB update of the rest of the block); each
-//     row swap is applied to W from column k0 on, so W keeps the permuted
-//     original block column;
-//  B. T = A11^-1 = U11^-1 L11^-1 from the factors (nb x nb);
-//  C. the block rows of the later columns become X = T Z1, in place;
-//  D. every other row r: Z(r, .) -= W(r, k0 .. k0 + nb) X (rank-nb MFMA updates).
-// Each block thus passes the later columns through memory once, where the
-// CL_NB-wide form (closed_solve) passes them once per CL_NB columns.
+// LU factorisation with partial pivoting in CL_BB-wide blocks, one workgroup per
+// (q, r) matrix.  For the block column k0 .. k0 + nb:
+//  A. its rows k0 .. D - 1 are copied to S and factored there (CL_NB-wide
+//     sub-panels: column-by-column within a sub-panel, then the sub-panel's
+//     rank-CL_NB update of the rest of the block); the row swaps are applied to
+//     the other columns of W and to perm, and the factors go back to W;
+//  B. L11^-1 and U11^-1 (nb x nb) from the factors, kept in T;
+//  C. the block rows of the later columns become U12 = L11^-1 Z1, in place;
+//  D. the rows below: Z -= L21 U12 (rank-nb MFMA updates).
+// The right-hand sides are no part of it: closed_lu_solve takes them through the
+// factors column panel by column panel, which is where 8 of the 10.7 D^3 flops are and
+// where the matrix alone would leave most of the chip to one workgroup's column steps.
+// (Gauss-Jordan on [A | Gamma] by one workgroup per matrix, 12 D^3: 28.1 ms at D = 320,
+// 480 q, against FACTOR_MS + SOLVE_MS.)
 // RP > 0 (D <= 256 RP): a sub-panel's column steps run on registers (thread t
 // holds rows s0 + t + 256 i, i < RP, of the CL_NB columns).  One barrier per
 // step: before it each wave leaves its best pivot candidate (by a wave
@@ -854,8 +862,8 @@ __device__ __forceinline__ void list_moved_rows(const int* piv, int r0, int nr, 
 // other columns of the block at the end of the sub-panel and W at the end of
 // A.  RP = 0: every column step works on S in memory and swaps the rows of W
 // at once.
-template <class R, bool PHI, int RP>
-__global__ __launch_bounds__(256, 2) void closed_solve_b64(ClosedArgs a) {
+template <class R, int RP>
+__global__ __launch_bounds__(256, 2) void closed_factor_b64(ClosedArgs a) {
   using C = typename Prec<R>::C;
   constexpr int RMAX = RP > 0 ? 256 * RP : 1;  // rows of the register path
   constexpr int RQ = RP > 0 ? 1 : 0;
@@ -878,16 +886,19 @@ __global__ __launch_bounds__(256, 2) void closed_solve_b64(ClosedArgs a) {
   __shared__ int mv_dst[2 * CL_BB * RQ + 1], mv_src[2 * CL_BB * RQ + 1];
   __shared__ int mv_n;
   const int mat = blockIdx.x;
-  const int D = a.D, D2 = 2 * D;
-  C* W = static_cast<C*>(a.W) + (size_t)mat * 2 * D * D;
+  const int D = a.D, nblk = (D + CL_BB - 1) / CL_BB;
+  C* W = static_cast<C*>(a.W) + (size_t)mat * D * D;
   C* S = static_cast<C*>(a.S) + (size_t)mat * CL_BB * D;
-  C* Linv = static_cast<C*>(a.T) + (size_t)mat * 2 * CL_BB * CL_BB;  // column-major, leading dimension CL_BB
-  C* Uinv = Linv + CL_BB * CL_BB;
+  int* perm = a.perm + (size_t)mat * (D + 1);
   const int tid = threadIdx.x;
   const C one = mkc((R)1, (R)0), zero = mkc((R)0, (R)0);
-  int info = 0;
+  int info = 0, moved = 0;
+  for (int x = tid; x < D; x += 256) perm[x] = x;
   for (int k0 = 0; k0 < D; k0 += CL_BB) {
     const int nb = min(CL_BB, D - k0);
+    // column-major, leading dimension CL_BB
+    C* Linv = static_cast<C*>(a.T) + ((size_t)mat * nblk + k0 / CL_BB) * 2 * CL_BB * CL_BB;
+    C* Uinv = Linv + CL_BB * CL_BB;
     // S(row, col) for col in [k0, k0 + nb): Sk[col * D + row]
     C* Sk = S - (size_t)k0 * D;
     // A. copy, then factor
@@ -1047,7 +1058,13 @@ __global__ __launch_bounds__(256, 2) void closed_solve_b64(ClosedArgs a) {
           continue;
         }
         if (p != c) {
-          for (int col = k0 + tid; col < D2; col += 256) {
+          if (tid == 0) {
+            const int x = perm[c];
+            perm[c] = perm[p];
+            perm[p] = x;
+          }
+          moved = 1;
+          for (int col = tid; col < D; col += 256) {
             const C x = W[(size_t)col * D + c];
             W[(size_t)col * D + c] = W[(size_t)col * D + p];
             W[(size_t)col * D + p] = x;
@@ -1090,18 +1107,28 @@ __global__ __launch_bounds__(256, 2) void closed_solve_b64(ClosedArgs a) {
         closed_update_b64<R>(Sk, D, s0 + sb, D, s0 + sb, k0 + nb, s0, sb, As, Bs, As1, Bs1);
       }
     }
-    if constexpr (RP > 0) {  // the block's swaps on W from column k0 on
+    if constexpr (RP > 0) {  // the block's swaps on W (its own columns are replaced below) and perm
       if (tid < 64) list_moved_rows(piv, k0, nb, map_b, k0, mv_dst, mv_src, &mv_n);
       __syncthreads();
-      move_rows_waves<R, 8>(W, D, k0, D2, mv_dst, mv_src, mv_n);
+      if (mv_n) {
+        moved = 1;
+        const int px = tid < mv_n ? perm[mv_src[tid]] : 0;
+        __syncthreads();
+        if (tid < mv_n) perm[mv_dst[tid]] = px;
+        move_rows_waves<R, 8>(W, D, 0, D, mv_dst, mv_src, mv_n);
+        __syncthreads();
+      }
     }
-    // B. T = U11^-1 L11^-1 (identity-padded to CL_BB) by 16 x 16 blocks: the
+    for (int u = tid; u < nb * (D - k0); u += 256) {
+      const int col = k0 + u / (D - k0), row = k0 + u % (D - k0);
+      W[(size_t)col * D + row] = Sk[(size_t)col * D + row];
+    }
+    // B. L11^-1 and U11^-1 (identity-padded to CL_BB) by 16 x 16 blocks: the
     // inverses of the four diagonal blocks of L11 and U11 from copies in LDS
     // (thread = block column), then the off-diagonal blocks by their distance d
     // from the diagonal, all blocks at one distance at once,
     //   Linv_ab = -Linv_aa sum_{c=b}^{a-1} L_ac Linv_cb      (a > b)
-    //   Uinv_ab = -Uinv_aa sum_{c=a+1}^{b} U_ac Uinv_cb      (a < b),
-    // then T = Uinv Linv on MFMA.
+    //   Uinv_ab = -Uinv_aa sum_{c=a+1}^{b} U_ac Uinv_cb      (a < b).
     {
       constexpr int NBB = CL_BB / CL_NB;
       // L11 (unit lower) and U11 (upper) entry (i, s), identity beyond nb
@@ -1234,24 +1261,15 @@ __global__ __launch_bounds__(256, 2) void closed_solve_b64(ClosedArgs a) {
         }
         __syncthreads();
       }
-      // T = Uinv Linv, in place in Linv
-      closed_apply_T_b64<R>(Linv, Uinv, CL_BB, 0, CL_BB, 0, CL_BB, As, Bs, As1, Bs1);
     }
     const int j0 = k0 + nb;
-    // C. block rows of the later columns: X = T Z1
-    closed_apply_T_b64<R>(W, Linv, D, k0, nb, j0, D2, As, Bs, As1, Bs1);
-    // D. rows below and above the block
-    closed_update_b64<R>(W, D, k0 + nb, D, j0, D2, k0, nb, As, Bs, As1, Bs1);
-    closed_update_b64<R>(W, D, 0, k0, j0, D2, k0, nb, As, Bs, As1, Bs1);
+    // C. block rows of the later columns: U12 = L11^-1 Z1
+    closed_apply_T_b64<R>(W, Linv, D, k0, nb, j0, D, As, Bs, As1, Bs1);
+    // D. rows below the block
+    closed_update_b64<R>(W, D, j0, D, j0, D, k0, nb, As, Bs, As1, Bs1);
   }
   if (info && tid == 0) atomicCAS(a.info, 0, info);
-  if constexpr (PHI) {
-    // Phi = X - Gamma
-    const int r = mat / a.nqb, q = a.q0 + (mat - r * a.nqb);
-    const double2* G = a.gam[r] + (size_t)D * D * q;
-    double2* O = a.out[r] + (size_t)D * D * q;
-    for (size_t u = tid; u < (size_t)D * D; u += 256) O[u] = csub(W[(size_t)D * D + u], G[u]);
-  }
+  if (tid == 0) perm[D] = moved;
 }
 
 // ---- refinement products ------------------------------------------------------------
@@ -1275,28 +1293,38 @@ __global__ void ir_clear(unsigned long long* rmax) { *rmax = 0ull; }
 // stages, so two chunks are in flight while one multiplies and three workgroups share a
 // CU.
 template <class R>
-constexpr int ir_kc() {
+constexpr int tile_kc() {
   return sizeof(R) == 8 ? 8 : 16;
 }
-constexpr int IR_STAGES = 3;
+constexpr int TILE_STAGES = 3;
 
-// A 64 x 64 tile at (tr, tc) of A B, both D x D column-major (D even), by a ring of LDS
-// stages filled with direct global-to-LDS loads; four waves of 2 x 2 blocks of 16 x 16 x 4
-// MFMAs.  One barrier per chunk: after it every wave is done with the chunk before, whose
-// stage takes the chunk two ahead.  A stage holds A as [k][row] and B as [column][k], its
-// 16-byte pieces (a double2, two float2) XOR-swizzled by the column, so 8 consecutive
-// lanes of a fragment read cover 32 banks or more.  Rows, columns and inner indices
-// beyond D load clamped addresses: the products of such inner indices are masked in the
-// last chunk, rows and columns dropped by the caller.  The register-fed form without
-// prefetch took 11.39 ms for the FP64 residual (and 4.08 ms more to form chi X) and 5.7 ms
-// for an FP32 product at D = 320, 480 q; this one 8.17 and 4.5 ms (61.6 and 112 TFLOP/s).
+// One factor pair of a tile product: A(row, k) = a[k lda + row], B(k, col) = b[col ldb + k],
+// k < len.  16-byte aligned, lda, ldb and len even.
+template <class C>
+struct TileSeg {
+  const C* a;
+  const C* b;
+  int lda, len;
+};
+
+// A 64 x 64 tile of A1 B1 + A2 B2 (s1.len a multiple of the chunk, possibly 0) by a ring of
+// LDS stages filled with direct global-to-LDS loads; four waves of 2 x 2 blocks of 16 x 16
+// x 4 MFMAs.  One barrier per chunk: after it every wave is done with the chunk before,
+// whose stage takes the chunk two ahead.  A stage holds A as [k][row] and B as
+// [column][k], its 16-byte pieces (a double2, two float2) XOR-swizzled by the column, so 8
+// consecutive lanes of a fragment read cover 32 banks or more.  Rows from `rows`, columns
+// from `cols` and inner indices from s2.len on load clamped addresses: such inner indices
+// are zeroed in the last chunk, rows and columns dropped by the caller.
+// The register-fed form without prefetch took 11.39 ms for the FP64 residual (and 4.08 ms
+// more to form chi X) and 5.7 ms for an FP32 product at D = 320, 480 q; this one 8.17 and
+// 4.5 ms (61.6 and 112 TFLOP/s).
 template <class R>
-__device__ __forceinline__ void ir_tile(const typename Prec<R>::C* A, const typename Prec<R>::C* B, int D, int tr,
-                                        int tc, char* lds, typename Prec<R>::V (&ar)[2][2],
-                                        typename Prec<R>::V (&ai)[2][2]) {
+__device__ __forceinline__ void tile_product(TileSeg<typename Prec<R>::C> s1, TileSeg<typename Prec<R>::C> s2, int ldb,
+                                             int rows, int cols, char* lds, typename Prec<R>::V (&ar)[2][2],
+                                             typename Prec<R>::V (&ai)[2][2]) {
   using P = Prec<R>;
   using C = typename P::C;
-  constexpr int KC = ir_kc<R>();
+  constexpr int KC = tile_kc<R>();
   constexpr int E = 16 / sizeof(C);           // elements of a 16-byte piece
   constexpr int RP = CL_T / E, KP = KC / E;   // pieces per row of A (one k) and per column of B
   constexpr int STAGE = 2 * KC * CL_T * (int)sizeof(C), HALF = STAGE / 2;
@@ -1305,31 +1333,50 @@ __device__ __forceinline__ void ir_tile(const typename Prec<R>::C* A, const type
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
   const int li = lane & 15, lk = lane >> 4;
-  const int nch = (D + KC - 1) / KC;
+  const int n1 = s1.len / KC, nch = n1 + (s2.len + KC - 1) / KC;
   const unsigned lbase = lds_addr(lds);
   // this lane's pieces: of A, slots (wave + 4 v) 64 + lane -> k = slot / RP, piece slot % RP;
-  // of B, slot -> column slot / 8, piece (slot % 8) ^ (column % 8)
-  int ak[2], arow[2], bk[2], bcol[2];
+  // of B, slot -> column slot / 8, piece (slot % 8) ^ (column % 8).  Their byte offsets from
+  // a chunk's first element: a whole chunk costs no address arithmetic beyond its base.
+  unsigned oa1[2], oa2[2], ob[2];
 #pragma unroll
   for (int v = 0; v < 2; ++v) {
     const int slot = (wave + 4 * v) * 64 + lane;
-    ak[v] = slot / RP;
-    arow[v] = min(tr + (slot % RP) * E, D - E);
-    bcol[v] = min(tc + slot / KP, D - 1);
-    bk[v] = ((slot % KP) ^ ((slot / KP) % KP)) * E;
+    const int row = min((slot % RP) * E, rows - E);
+    oa1[v] = (unsigned)(((slot / RP) * s1.lda + row) * (int)sizeof(C));
+    oa2[v] = (unsigned)(((slot / RP) * s2.lda + row) * (int)sizeof(C));
+    ob[v] = (unsigned)(((size_t)min(slot / KP, cols - 1) * ldb + ((slot % KP) ^ ((slot / KP) % KP)) * E) * sizeof(C));
   }
   auto issue = [&](int ch) {
-    const unsigned st = lbase + (ch % IR_STAGES) * STAGE;
-    const int k0 = ch * KC;
+    const unsigned st = lbase + (ch % TILE_STAGES) * STAGE;
+    if (ch < n1) {
 #pragma unroll
-    for (int v = 0; v < 2; ++v) {
-      const int k = min(k0 + ak[v], D - 1);
-      dma16(A, (unsigned)(((size_t)k * D + arow[v]) * sizeof(C)), st + (wave + 4 * v) * 1024);
+      for (int v = 0; v < 2; ++v) dma16(s1.a + (size_t)ch * KC * s1.lda, oa1[v], st + (wave + 4 * v) * 1024);
+#pragma unroll
+      for (int v = 0; v < 2; ++v) dma16(s1.b + ch * KC, ob[v], st + HALF + (wave + 4 * v) * 1024);
+      return;
+    }
+    const int k0 = (ch - n1) * KC;
+    if (k0 + KC <= s2.len) {
+#pragma unroll
+      for (int v = 0; v < 2; ++v) dma16(s2.a + (size_t)k0 * s2.lda, oa2[v], st + (wave + 4 * v) * 1024);
+#pragma unroll
+      for (int v = 0; v < 2; ++v) dma16(s2.b + k0, ob[v], st + HALF + (wave + 4 * v) * 1024);
+      return;
     }
 #pragma unroll
     for (int v = 0; v < 2; ++v) {
-      const int k = min(k0 + bk[v], D - E);
-      dma16(B, (unsigned)(((size_t)bcol[v] * D + k) * sizeof(C)), st + HALF + (wave + 4 * v) * 1024);
+      const int slot = (wave + 4 * v) * 64 + lane;
+      const int k = min(slot / RP, s2.len - 1 - k0);
+      dma16(s2.a + (size_t)k0 * s2.lda, (unsigned)((k * s2.lda + min((slot % RP) * E, rows - E)) * (int)sizeof(C)),
+            st + (wave + 4 * v) * 1024);
+    }
+#pragma unroll
+    for (int v = 0; v < 2; ++v) {
+      const int slot = (wave + 4 * v) * 64 + lane;
+      const int k = min(((slot % KP) ^ ((slot / KP) % KP)) * E, s2.len - E - k0);
+      dma16(s2.b + k0, (unsigned)(((size_t)min(slot / KP, cols - 1) * ldb + k) * sizeof(C)),
+            st + HALF + (wave + 4 * v) * 1024);
     }
   };
 #pragma unroll
@@ -1338,35 +1385,7 @@ __device__ __forceinline__ void ir_tile(const typename Prec<R>::C* A, const type
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int e = 0; e < 4; ++e) ar[i][j][e] = ai[i][j][e] = 0;
-  auto steps = [&](const char* st, int left, auto masked) {
-    const C* sa = reinterpret_cast<const C*>(st);
-    const char* sb = st + HALF;
-#pragma unroll
-    for (int kk = 0; kk < KC; kk += 4) {
-      if (masked.value && kk >= left) break;
-      const int k = kk + lk;
-      C fa[2], fb[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) fa[i] = sa[k * CL_T + wr + i * 16 + li];
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int col = wc + j * 16 + li;
-        fb[j] = *reinterpret_cast<const C*>(sb + (col * KP + ((k / E) ^ (col % KP))) * 16 + (k % E) * sizeof(C));
-      }
-      if (masked.value && k >= left)
-#pragma unroll
-        for (int i = 0; i < 2; ++i) fa[i] = fb[i] = mkc((R)0, (R)0);
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          ar[i][j] = P::fma_add(fa[i].x, fb[j].x, ar[i][j]);
-          ai[i][j] = P::fma_add(fa[i].x, fb[j].y, ai[i][j]);
-          ar[i][j] = P::fma_sub(fa[i].y, fb[j].y, ar[i][j]);
-          ai[i][j] = P::fma_add(fa[i].y, fb[j].x, ai[i][j]);
-        }
-    }
-  };
+  stage_barrier();  // the stages' last readers are done
   issue(0);
   if (nch > 1) issue(1);
   for (int ch = 0; ch < nch; ++ch) {
@@ -1377,17 +1396,187 @@ __device__ __forceinline__ void ir_tile(const typename Prec<R>::C* A, const type
       wait_vmcnt<0>();
     stage_barrier();
     if (ch + 2 < nch) issue(ch + 2);
-    const char* st = lds + (ch % IR_STAGES) * STAGE;
-    if ((ch + 1) * KC <= D)
-      steps(st, KC, std::false_type{});
+    char* st = lds + (ch % TILE_STAGES) * STAGE;
+    C* sa = reinterpret_cast<C*>(st);
+    char* sb = st + HALF;
+    auto b_at = [&](int col, int k) {
+      return reinterpret_cast<C*>(sb + (col * KP + ((k / E) ^ (col % KP))) * 16 + (k % E) * sizeof(C));
+    };
+    const int left = s2.len - (ch - n1) * KC;
+    if (ch >= n1 && left < KC) {  // the last chunk: zeros beyond the inner range
+      for (int u = tid; u < (KC - left) * CL_T; u += 256) {
+        const int k = left + u / CL_T, x = u % CL_T;
+        sa[k * CL_T + x] = mkc((R)0, (R)0);
+        *b_at(x, k) = mkc((R)0, (R)0);
+      }
+      __syncthreads();
+    }
+#pragma unroll
+    for (int kk = 0; kk < KC; kk += 4) {
+      const int k = kk + lk;
+      C fa[2], fb[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) fa[i] = sa[k * CL_T + wr + i * 16 + li];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) fb[j] = *b_at(wc + j * 16 + li, k);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          ar[i][j] = P::fma_add(fa[i].x, fb[j].x, ar[i][j]);
+          ai[i][j] = P::fma_add(fa[i].x, fb[j].y, ai[i][j]);
+          ar[i][j] = P::fma_sub(fa[i].y, fb[j].y, ar[i][j]);
+          ai[i][j] = P::fma_add(fa[i].y, fb[j].x, ai[i][j]);
+        }
+    }
+  }
+}
+
+// ---- the block form's solves ---------------------------------------------------------
+
+// Block rows scaled by the inverses of their diagonal blocks, in place and negated: left of
+// the diagonal -L_kk^-1 L_ki, right of it -U_kk^-1 U_kj, so that a block row of a
+// triangular solve is one product, its diagonal inverse times the right-hand side
+// included.  grid: nblk (nblk - 1) blocks of every matrix
+template <class R>
+__global__ __launch_bounds__(256, 3) void closed_scale(ClosedArgs a) {
+  using P = Prec<R>;
+  using C = typename P::C;
+  using V = typename P::V;
+  __shared__ __attribute__((aligned(16))) char stage[TILE_STAGES * 16384];
+  const int D = a.D, nblk = (D + CL_BB - 1) / CL_BB, per = nblk * (nblk - 1);
+  const int logical = closed_xcd_remap(blockIdx.x, gridDim.x);
+  const int mat = logical / per, t = logical - mat * per;
+  const int kb = t / (nblk - 1), o = t - kb * (nblk - 1), ib = o < kb ? o : o + 1;
+  const int k0 = kb * CL_BB, c0 = ib * CL_BB, nb = min(CL_BB, D - k0), nc = min(CL_BB, D - c0);
+  C* W = static_cast<C*>(a.W) + (size_t)mat * D * D + (size_t)c0 * D + k0;
+  const C* T = static_cast<const C*>(a.T) + (((size_t)mat * nblk + kb) * 2 + (ib < kb ? 0 : 1)) * CL_BB * CL_BB;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32, li = lane & 15, lk = lane >> 4;
+  V ar[2][2], ai[2][2];
+  tile_product<R>({T, W, CL_BB, 0}, {T, W, CL_BB, nb}, D, CL_BB, nc, stage, ar, ai);
+  // every wave's loads have landed before the last barrier: the block may be replaced
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int row = wr + i * 16 + P::orow(lk, e), col = wc + j * 16 + li;
+        if (row < nb && col < nc) W[(size_t)col * D + row] = mkc(-ar[i][j][e], -ai[i][j][e]);
+      }
+}
+
+struct LuArgs {
+  const double2* gam[4];
+  double2* x[4];        // the output arrays: X, or Phi
+  const void* W;        // scaled block rows
+  const void* T;        // diagonal inverses
+  const int* perm;
+  const float2* rhs;    // refinement: [mat][D][D]
+  float2* y;            // refinement: [mat][D][D] solution of the product in FP32
+  int D, q0, nqb;
+};
+
+// X = U^-1 L^-1 P B for the 64 columns of one panel of one matrix: forward, then backward,
+// a block row at a time, each one tile product whose inner index runs over the block rows
+// that are done and its own right-hand side.  The panel lives in the output (direct) or in
+// y (refinement); a block row is stored, and waited for, before the next one reads it.
+// MFMA-bound: 9.6 D^3 flops with the diagonal inverses, the factors shared through L2 by
+// the panels of a matrix, which run next to each other on one XCD.
+//   MODE 0: FP64, B = Gamma, Phi = X - Gamma    MODE 1: X = fp64(A32^-1 rhs)
+//   MODE 2: X += fp64(A32^-1 rhs)               MODE 3: Phi = X + fp64(A32^-1 rhs) - Gamma
+// grid: ceil(D / 64) panels of every matrix
+template <int MODE>
+__global__ __launch_bounds__(256, 3) void closed_lu_solve(LuArgs a) {
+  using R = typename std::conditional<MODE == 0, double, float>::type;
+  using P = Prec<R>;
+  using C = typename P::C;
+  using V = typename P::V;
+  __shared__ __attribute__((aligned(16))) char stage[TILE_STAGES * 16384];
+  const int D = a.D, nblk = (D + CL_BB - 1) / CL_BB;
+  const int logical = closed_xcd_remap(blockIdx.x, gridDim.x);
+  const int mat = logical / nblk, c0 = (logical - mat * nblk) * CL_T;
+  const int r = mat / a.nqb, q = a.q0 + (mat - r * a.nqb);
+  const size_t DD = (size_t)D * D, base = DD * q + (size_t)c0 * D;
+  const int nc = min(CL_T, D - c0);
+  const double2* G = a.gam[r] + base;
+  double2* X = a.x[r] + base;
+  C* buf;
+  const C* src;
+  if constexpr (MODE == 0) {
+    buf = X;
+    src = G;
+  } else {
+    buf = a.y + DD * mat + (size_t)c0 * D;
+    src = a.rhs + DD * mat + (size_t)c0 * D;
+  }
+  const C* W = static_cast<const C*>(a.W) + DD * mat;
+  const C* T = static_cast<const C*>(a.T) + (size_t)mat * nblk * 2 * CL_BB * CL_BB;
+  const int* perm = a.perm + (size_t)mat * (D + 1);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32, li = lane & 15, lk = lane >> 4;
+  auto settle = [&]() {  // the stores of this workgroup are done, for its direct loads
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+    __syncthreads();
+  };
+  if (perm[D]) {  // the factorisation moved rows: the panel in their order first
+    for (int u = tid; u < nc * D; u += 256) {
+      const int col = u / D, row = u - col * D;
+      buf[(size_t)col * D + row] = src[(size_t)col * D + perm[row]];
+    }
+    settle();
+    src = buf;
+  }
+  V ar[2][2], ai[2][2];
+  auto store = [&](int k0, int nb, bool last) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int row = wr + i * 16 + P::orow(lk, e), col = wc + j * 16 + li;
+          if (row >= nb || col >= nc) continue;
+          const size_t at = (size_t)col * D + k0 + row;
+          buf[at] = mkc(ar[i][j][e], ai[i][j][e]);
+          if constexpr (MODE == 1) {
+            if (last) X[at] = make_double2((double)ar[i][j][e], (double)ai[i][j][e]);
+          } else if constexpr (MODE >= 2) {
+            if (last) {
+              const double2 x = X[at];
+              const double2 v = make_double2(x.x + (double)ar[i][j][e], x.y + (double)ai[i][j][e]);
+              X[at] = MODE == 3 ? csub(v, G[at]) : v;
+            }
+          }
+        }
+    settle();
+  };
+  for (int kb = 0; kb < nblk; ++kb) {
+    const int k0 = kb * CL_BB, nb = min(CL_BB, D - k0);
+    tile_product<R>({W + k0, buf, D, k0}, {T + (size_t)kb * 2 * CL_BB * CL_BB, src + k0, CL_BB, nb}, D, nb, nc, stage,
+                    ar, ai);
+    store(k0, nb, false);
+  }
+  for (int kb = nblk - 1; kb >= 0; --kb) {
+    const int k0 = kb * CL_BB, nb = min(CL_BB, D - k0), k1 = k0 + nb;
+    const C* Ui = T + ((size_t)kb * 2 + 1) * CL_BB * CL_BB;
+    if (k1 < D)
+      tile_product<R>({Ui, buf + k0, CL_BB, nb}, {W + (size_t)k1 * D + k0, buf + k1, D, D - k1}, D, nb, nc, stage, ar,
+                      ai);
     else
-      steps(st, D - ch * KC, std::true_type{});
+      tile_product<R>({Ui, buf + k0, CL_BB, 0}, {Ui, buf + k0, CL_BB, nb}, D, nb, nc, stage, ar, ai);
+    store(k0, nb, true);
+  }
+  if constexpr (MODE == 0) {
+    for (int u = tid; u < nc * D; u += 256) X[u] = csub(X[u], G[u]);
   }
 }
 
 // Batched complex products of the refinement, one 64 x 64 tile per workgroup, the tiles of
 // a matrix on one XCD so that they share its L2.
 //   MODE 0: X  = fp64(A32^-1 fp32(Gamma))    MODE 1: X += fp64(A32^-1 fp32(R))
+//           (below the block form's orders, with the inverse that closed_solve leaves)
 //   MODE 2: R  = Gamma - X + kappa (Gamma chi) X in FP64, kept as fp32(R), the only form a
 //           product reads, with per-tile |R|^2, |Gamma|^2 of the FP64 values
 // grid: tiles_n^2 * 4 nqb
@@ -1397,7 +1586,7 @@ __global__ __launch_bounds__(256, 3) void ir_gemm(IrArgs a) {
   using P = Prec<R>;
   using C = typename P::C;
   using V = typename P::V;
-  __shared__ __attribute__((aligned(16))) char stage[IR_STAGES * 16384];
+  __shared__ __attribute__((aligned(16))) char stage[TILE_STAGES * 16384];
   const int tiles = a.tiles_n * a.tiles_n;
   const int logical = closed_xcd_remap(blockIdx.x, gridDim.x);
   const int mat = logical / tiles, t = logical - mat * tiles;
@@ -1411,10 +1600,15 @@ __global__ __launch_bounds__(256, 3) void ir_gemm(IrArgs a) {
   const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
   const int li = lane & 15, lk = lane >> 4;
   V ar[2][2], ai[2][2];
-  if constexpr (MODE == 2)
-    ir_tile<R>(a.gx + DD * mat, X, D, tr, tc, stage, ar, ai);
-  else
-    ir_tile<R>(a.inv + 2 * DD * mat + DD, a.rhs + DD * mat, D, tr, tc, stage, ar, ai);
+  const C *A, *B;
+  if constexpr (MODE == 2) {
+    A = a.gx + DD * mat + tr;
+    B = X + (size_t)tc * D;
+  } else {
+    A = a.inv + 2 * DD * mat + DD + tr;
+    B = a.rhs + DD * mat + (size_t)tc * D;
+  }
+  tile_product<R>({A, B, D, 0}, {A, B, D, D}, D, D - tr, D - tc, stage, ar, ai);
   double rr = 0.0, gg = 0.0;
   const double kap = a.kappa[r];
   float2* Rm = a.rhs + DD * mat;
@@ -1544,23 +1738,65 @@ static bool closed_regs(const tups_ctx* c) {
   return closed_blocked(c) && c->closed_variant != 1 && c->sz.nz <= 256 * kClosedRp;
 }
 // scratch of closed_solve_b64 per matrix, in complex elements
-static size_t closed_b64_elems(size_t D) { return (size_t)CL_BB * D + 2 * (size_t)CL_BB * CL_BB; }
+static size_t closed_blocks(size_t D) { return (D + CL_BB - 1) / CL_BB; }
+// per matrix of the block form: the factors, the block column in work and the diagonal inverses
+static size_t closed_b64_elems(size_t D) { return D * D + (size_t)CL_BB * D + 2 * closed_blocks(D) * CL_BB * CL_BB; }
+
+// the block form's parts of a workspace from `at` on; returns its end
+template <class C>
+static int* place_b64(ClosedArgs& a, C* at, size_t mats) {
+  const size_t D = a.D;
+  a.W = at;
+  at += mats * D * D;
+  a.S = at;
+  at += mats * CL_BB * D;
+  a.T = at;
+  at += mats * closed_blocks(D) * 2 * CL_BB * CL_BB;
+  a.perm = reinterpret_cast<int*>(at);
+  return a.perm + mats * (D + 1);
+}
+
+// the factorisation of every matrix and the scaling of its block rows
+template <class R>
+static int factor_b64(tups_ctx* c, const ClosedArgs& a, unsigned mats) {
+  if (closed_regs(c))
+    hipLaunchKernelGGL((closed_factor_b64<R, kClosedRp>), dim3(mats), dim3(256), 0, c->stream, a);
+  else
+    hipLaunchKernelGGL((closed_factor_b64<R, 0>), dim3(mats), dim3(256), 0, c->stream, a);
+  TUPS_HIP(hipGetLastError());
+  const unsigned nblk = (unsigned)closed_blocks(a.D);
+  if (nblk > 1) hipLaunchKernelGGL(closed_scale<R>, dim3(nblk * (nblk - 1) * mats), dim3(256), 0, c->stream, a);
+  TUPS_HIP(hipGetLastError());
+  return TUPS_OK;
+}
+
+static LuArgs lu_args(const tups_ctx* c, const ClosedArgs& a) {
+  LuArgs l{};
+  for (int r = 0; r < 4; ++r) {
+    l.gam[r] = c->gamma[r];
+    l.x[r] = c->spare[r];
+  }
+  l.W = a.W;
+  l.T = a.T;
+  l.perm = a.perm;
+  l.D = a.D;
+  l.q0 = a.q0;
+  l.nqb = a.nqb;
+  return l;
+}
 
 int launch_bse_closed(tups_ctx* c) {
   const tups_sizes& s = c->sz;
   const size_t D = s.nz;
   TUPS_CHECK(s.nl <= CL_NL_MAX, TUPS_EINVAL, "closed form: at most 9 form factors");
   const bool blk = closed_blocked(c);
-  const size_t per_mat = (2 * D * D + (blk ? closed_b64_elems(D) : 0)) * sizeof(double2);
+  const size_t per_mat = blk ? closed_b64_elems(D) * sizeof(double2) + (D + 1) * sizeof(int) : 2 * D * D * sizeof(double2);
   int qbatch = 0;
   if (int rc = closed_reserve(c, 4 * per_mat, 0, &qbatch)) return rc;
   ClosedArgs a{};
   closed_common(c, a);
-  if (blk) {
-    const size_t mats_max = 4 * (size_t)qbatch;
-    a.S = static_cast<double2*>(a.W) + mats_max * 2 * D * D;
-    a.T = static_cast<double2*>(a.S) + mats_max * CL_BB * D;
-  }
+  a.blk = blk ? 1 : 0;
+  if (blk) place_b64<double2>(a, static_cast<double2*>(a.W), 4 * (size_t)qbatch);
   hipLaunchKernelGGL(closed_clear, dim3(1), dim3(1), 0, c->stream, a.info);
   TUPS_HIP(hipGetLastError());
   for (int q0 = 0; q0 < s.nq; q0 += qbatch) {
@@ -1570,12 +1806,13 @@ int launch_bse_closed(tups_ctx* c) {
     if (int rc = timer_begin(c)) return rc;
     hipLaunchKernelGGL((closed_build_nu<double2, false>), dim3((unsigned)s.nf, mats), dim3(256), 0, c->stream, a);
     TUPS_HIP(hipGetLastError());
-    if (blk && closed_regs(c))
-      hipLaunchKernelGGL((closed_solve_b64<double, true, kClosedRp>), dim3(mats), dim3(256), 0, c->stream, a);
-    else if (blk)
-      hipLaunchKernelGGL((closed_solve_b64<double, true, 0>), dim3(mats), dim3(256), 0, c->stream, a);
-    else
+    if (blk) {
+      if (int rc = factor_b64<double>(c, a, mats)) return rc;
+      hipLaunchKernelGGL(closed_lu_solve<0>, dim3((unsigned)closed_blocks(D) * mats), dim3(256), 0, c->stream,
+                         lu_args(c, a));
+    } else {
       hipLaunchKernelGGL((closed_solve<double, true>), dim3(mats), dim3(256), 0, c->stream, a);
+    }
     TUPS_HIP(hipGetLastError());
     if (int rc = timer_end(c, TUPS_K_BSE_CLOSED)) return rc;
   }
@@ -1593,12 +1830,13 @@ int launch_bse_closed_ir(tups_ctx* c) {
   TUPS_CHECK(s.nl <= CL_NL_MAX, TUPS_EINVAL, "closed form: at most 9 form factors");
   const size_t D = s.nz, DD = D * D;
   const int tiles_n = (int)((D + CL_T - 1) / CL_T);
-  // per matrix: [A32 | I] (2 D^2 float2), the rounded right-hand side (D^2 float2), Gamma chi (D^2
-  // double2), tile partials, res
+  // per matrix: [A32 | I] (2 D^2 float2) or the block form's factors and a product's solution, the
+  // rounded right-hand side (D^2 float2), Gamma chi (D^2 double2), tile partials, res
   const bool blk = closed_blocked(c);
-  const size_t per_mat = 3 * DD * sizeof(float2) + DD * sizeof(double2) +
+  const size_t per_mat = DD * sizeof(float2) + DD * sizeof(double2) +
                          (size_t)tiles_n * tiles_n * 2 * sizeof(double) + sizeof(double) + 64 +
-                         (blk ? closed_b64_elems(D) * sizeof(float2) : 0);
+                         (blk ? (DD + closed_b64_elems(D)) * sizeof(float2) + (D + 1) * sizeof(int)
+                              : 2 * DD * sizeof(float2));
   int qbatch = 0;
   if (int rc = closed_reserve(c, 4 * per_mat, 256, &qbatch)) return rc;
   ClosedArgs a{};
@@ -1613,21 +1851,26 @@ int launch_bse_closed_ir(tups_ctx* c) {
   b.tiles_n = tiles_n;
   const size_t mats_max = 4 * (size_t)qbatch;
   char* base = static_cast<char*>(a.W);
-  b.inv = reinterpret_cast<const float2*>(base);
-  base += mats_max * 2 * DD * sizeof(float2);
   b.gx = a.gx = reinterpret_cast<double2*>(base);
   base += mats_max * DD * sizeof(double2);
   b.rhs = a.g32 = reinterpret_cast<float2*>(base);
   base += mats_max * DD * sizeof(float2);
+  a.blk = blk ? 1 : 0;
+  float2* y32 = nullptr;
+  if (blk) {
+    y32 = reinterpret_cast<float2*>(base);
+    base = reinterpret_cast<char*>(place_b64<float2>(a, y32 + mats_max * DD, mats_max));
+  } else {
+    a.W = base;
+    b.inv = reinterpret_cast<const float2*>(base);
+    base += mats_max * 2 * DD * sizeof(float2);
+  }
+  base = reinterpret_cast<char*>((reinterpret_cast<uintptr_t>(base) + 15) / 16 * 16);
   b.part = reinterpret_cast<double*>(base);
   base += mats_max * tiles_n * tiles_n * 2 * sizeof(double);
   b.res = reinterpret_cast<double*>(base);
   base += mats_max * sizeof(double);
   b.rmax = reinterpret_cast<unsigned long long*>((reinterpret_cast<uintptr_t>(base) + 63) / 64 * 64);
-  if (blk) {  // FP32 scratch of the block elimination after the counter
-    a.S = reinterpret_cast<float2*>(reinterpret_cast<char*>(b.rmax) + 64);
-    a.T = static_cast<float2*>(a.S) + mats_max * CL_BB * D;
-  }
   hipLaunchKernelGGL(closed_clear, dim3(1), dim3(1), 0, c->stream, a.info);
   TUPS_HIP(hipGetLastError());
   int steps_max = 0;
@@ -1640,17 +1883,23 @@ int launch_bse_closed_ir(tups_ctx* c) {
     if (int rc = timer_begin(c)) return rc;
     hipLaunchKernelGGL((closed_build_nu<float2, true>), dim3((unsigned)s.nf, mats), dim3(256), 0, c->stream, a);
     TUPS_HIP(hipGetLastError());
-    if (blk && closed_regs(c))
-      hipLaunchKernelGGL((closed_solve_b64<float, false, kClosedRp>), dim3(mats), dim3(256), 0, c->stream, a);
-    else if (blk)
-      hipLaunchKernelGGL((closed_solve_b64<float, false, 0>), dim3(mats), dim3(256), 0, c->stream, a);
-    else
+    LuArgs lu{};
+    const unsigned glu = (unsigned)closed_blocks(D) * mats;
+    if (blk) {
+      if (int rc = factor_b64<float>(c, a, mats)) return rc;
+      lu = lu_args(c, a);
+      lu.rhs = b.rhs;
+      lu.y = y32;
+      // X = A32^-1 Gamma
+      hipLaunchKernelGGL(closed_lu_solve<1>, dim3(glu), dim3(256), 0, c->stream, lu);
+    } else {
       hipLaunchKernelGGL((closed_solve<float, false>), dim3(mats), dim3(256), 0, c->stream, a);
-    TUPS_HIP(hipGetLastError());
-    // X = A32^-1 Gamma
-    hipLaunchKernelGGL(ir_gemm<0>, dim3(gblk), dim3(256), 0, c->stream, b);
+      TUPS_HIP(hipGetLastError());
+      hipLaunchKernelGGL(ir_gemm<0>, dim3(gblk), dim3(256), 0, c->stream, b);
+    }
     TUPS_HIP(hipGetLastError());
     int steps = 0;
+    bool phi = false;  // the output holds Phi already
     double res = INFINITY;
     for (;;) {
       hipLaunchKernelGGL(ir_clear, dim3(1), dim3(1), 0, c->stream, b.rmax);
@@ -1663,13 +1912,23 @@ int launch_bse_closed_ir(tups_ctx* c) {
       TUPS_HIP(hipMemcpyAsync(&bits, b.rmax, sizeof(bits), hipMemcpyDeviceToHost, c->stream));
       TUPS_HIP(hipStreamSynchronize(c->stream));
       std::memcpy(&res, &bits, sizeof(res));
-      if (res <= c->ir_tol || steps >= c->ir_max_steps) break;
+      // converged: the residual at hand gives one more step without another one to follow, so
+      // that a first solve good enough for the tolerance is no less exact than one that missed it
+      const bool done = res <= c->ir_tol;
+      if (steps >= c->ir_max_steps || (done && !(res > 0x1p-50))) break;
       // X += A32^-1 R
-      hipLaunchKernelGGL(ir_gemm<1>, dim3(gblk), dim3(256), 0, c->stream, b);
+      if (blk && done) {
+        hipLaunchKernelGGL(closed_lu_solve<3>, dim3(glu), dim3(256), 0, c->stream, lu);
+        phi = true;
+      } else if (blk)
+        hipLaunchKernelGGL(closed_lu_solve<2>, dim3(glu), dim3(256), 0, c->stream, lu);
+      else
+        hipLaunchKernelGGL(ir_gemm<1>, dim3(gblk), dim3(256), 0, c->stream, b);
       TUPS_HIP(hipGetLastError());
       ++steps;
+      if (done) break;
     }
-    hipLaunchKernelGGL(ir_final, dim3((unsigned)((DD + 255) / 256), mats), dim3(256), 0, c->stream, b);
+    if (!phi) hipLaunchKernelGGL(ir_final, dim3((unsigned)((DD + 255) / 256), mats), dim3(256), 0, c->stream, b);
     TUPS_HIP(hipGetLastError());
     if (int rc = timer_end(c, TUPS_K_BSE_IR)) return rc;
     steps_max = std::max(steps_max, steps);
