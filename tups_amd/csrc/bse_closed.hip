@@ -167,7 +167,6 @@ struct ClosedArgs {
   const double2* chi[2];
   void* W;      // column-major, double2 (direct) or float2 (refinement): [mat][2D columns][D rows] for
                 // closed_solve, [mat][D columns][D rows] for the block form
-  void* S;      // block form: [mat][CL_BB columns][D rows], the block column being factored
   void* T;      // block form: [mat][block][2][CL_BB][CL_BB], L_kk^-1 and U_kk^-1
   int* perm;    // block form: [mat][D + 1]: row i of L U is row perm[i] of A; then whether any row moved
   int blk;      // the block form
@@ -327,266 +326,6 @@ __device__ void closed_update(typename Prec<R>::C* W, int D, int r0, int r1, int
           }
     }
   __syncthreads();  // the updated Z is visible to the whole workgroup
-}
-
-// The FP64 products of the block elimination with the inner index staged by
-// direct global-to-LDS loads into two stages, so chunk k + 1 is in flight
-// while chunk k multiplies and no registers hold it:
-//   APPLY = false (closed_update): Z(r, c) -= sum_t W(r, k0 + t) W(k0 + t, c),
-//     r in [r0, r1), c in [c0, c1);
-//   APPLY = true (closed_apply_T): Z(k0 + i, c) <- sum_t T(i, t) Z(k0 + t, c),
-//     i < nb, T column-major with leading dimension CL_BB (each tile is read
-//     whole before it is written, so the product runs in place).
-// A stage is the A chunk sa[CL_NB][CL_T + 1] (rows padded) and the B chunk in
-// the first CL_T CL_NB slots of sb, column-major with the inner index
-// XOR-swizzled by the column (a fragment read is then free of bank
-// conflicts).  Rows and columns beyond the ranges load clamped addresses
-// (their results are not written).  nb must be a multiple of CL_NB, so every
-// chunk issues the same 8 loads per thread.
-template <bool APPLY>
-__device__ void closed_gemm_dma(double2* W, int D, const double2* T, int r0, int r1, int c0, int c1, int k0, int nb,
-                                double2 (*s0a)[CL_T + 1], double2 (*s0b)[CL_T + 1], double2 (*s1a)[CL_T + 1],
-                                double2 (*s1b)[CL_T + 1]) {
-  using P = Prec<double>;
-  using V = P::V;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
-  const int li = lane & 15, lk = lane >> 4;
-  const double2 zero = mkc(0.0, 0.0);
-  const int nch = nb / CL_NB;
-  // A(row, t) = Ab[(ka0 + t) lda + row]; the output row of A's row r is ro + r
-  const double2* Ab = APPLY ? T : W;
-  const int lda = APPLY ? CL_BB : D, ka0 = APPLY ? 0 : k0, amax = APPLY ? CL_BB : D, ro = APPLY ? k0 : 0;
-  if (APPLY) {
-    r0 = 0;
-    r1 = nb;
-  }
-  for (int tr = r0; tr < r1; tr += CL_T)
-    for (int tc = c0; tc < c1; tc += CL_T) {
-      const int arow = min(tr + lane, amax - 1);
-      auto issue = [&](int ch, double2 (*sa)[CL_T + 1], double2 (*sb)[CL_T + 1]) {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {  // A: inner index ka, rows tr .. tr + 63
-          const int ka = wave + 4 * v;
-          dma16(Ab, (unsigned)(((size_t)(ka0 + ch * CL_NB + ka) * lda + arow) * sizeof(double2)),
-                lds_addr(&sa[ka][0]));
-        }
-        const double2* sbf = &sb[0][0];
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {  // B: slots 64 d .. 64 d + 63 = columns 4 d .. 4 d + 3
-          const int d = wave + 4 * v, slot = 64 * d + lane, col = slot >> 4;
-          const int kb = (slot & 15) ^ (col & 15);
-          const int gc = min(tc + col, c1 - 1);
-          dma16(W, (unsigned)(((size_t)gc * D + k0 + ch * CL_NB + kb) * sizeof(double2)), lds_addr(sbf + 64 * d));
-        }
-      };
-      V ar[2][2], ai[2][2];
-      auto compute = [&](double2 (*sa)[CL_T + 1], double2 (*sb)[CL_T + 1]) {
-        const double2* sbf = &sb[0][0];
-#pragma unroll
-        for (int kk = 0; kk < CL_NB; kk += 4) {
-          double2 fa[2], fb[2];
-#pragma unroll
-          for (int i = 0; i < 2; ++i) fa[i] = sa[kk + lk][wr + i * 16 + li];
-#pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            const int col = wc + j * 16 + li;
-            fb[j] = sbf[col * CL_NB + ((kk + lk) ^ (col & 15))];
-          }
-#pragma unroll
-          for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-              if constexpr (APPLY) {  // + A B
-                ar[i][j] = P::fma_add(fa[i].x, fb[j].x, ar[i][j]);
-                ar[i][j] = P::fma_sub(fa[i].y, fb[j].y, ar[i][j]);
-                ai[i][j] = P::fma_add(fa[i].x, fb[j].y, ai[i][j]);
-                ai[i][j] = P::fma_add(fa[i].y, fb[j].x, ai[i][j]);
-              } else {  // - A B
-                ar[i][j] = P::fma_sub(fa[i].x, fb[j].x, ar[i][j]);
-                ar[i][j] = P::fma_add(fa[i].y, fb[j].y, ar[i][j]);
-                ai[i][j] = P::fma_sub(fa[i].x, fb[j].y, ai[i][j]);
-                ai[i][j] = P::fma_sub(fa[i].y, fb[j].x, ai[i][j]);
-              }
-            }
-        }
-      };
-      issue(0, s0a, s0b);
-      if constexpr (APPLY) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j) ar[i][j] = ai[i][j] = V{};
-      } else {
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const int row = tr + wr + i * 16 + P::orow(lk, e), col = tc + wc + j * 16 + li;
-              const double2 z = (row < r1 && col < c1) ? W[(size_t)col * D + row] : zero;
-              ar[i][j][e] = z.x;
-              ai[i][j][e] = z.y;
-            }
-        // the tile's values are waited for here, with chunk 0, and not at the
-        // first MFMA (where the wait would also cover chunk 1)
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j)
-            asm volatile("" ::"v"(ar[i][j][0]), "v"(ar[i][j][1]), "v"(ar[i][j][2]), "v"(ar[i][j][3]),
-                         "v"(ai[i][j][0]), "v"(ai[i][j][1]), "v"(ai[i][j][2]), "v"(ai[i][j][3]));
-      }
-      for (int ch = 0; ch < nch; ch += 2) {
-        if (ch + 1 < nch) {
-          issue(ch + 1, s1a, s1b);
-          wait_vmcnt<8>();
-        } else {
-          wait_vmcnt<0>();
-        }
-        stage_barrier();
-        compute(s0a, s0b);
-        stage_barrier();
-        if (ch + 1 >= nch) break;
-        if (ch + 2 < nch) {
-          issue(ch + 2, s0a, s0b);
-          wait_vmcnt<8>();
-        } else {
-          wait_vmcnt<0>();
-        }
-        stage_barrier();
-        compute(s1a, s1b);
-        stage_barrier();
-      }
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int row = tr + wr + i * 16 + P::orow(lk, e), col = tc + wc + j * 16 + li;
-            if (row < r1 && col < c1) W[(size_t)col * D + ro + row] = mkc(ar[i][j][e], ai[i][j][e]);
-          }
-    }
-  __syncthreads();  // the result is visible to the whole workgroup
-}
-
-// the update of the block elimination: in FP64 with the DMA stages when nb
-// allows, else (and in FP32) closed_update on the first stage
-template <class R>
-__device__ __forceinline__ void closed_update_b64(typename Prec<R>::C* W, int D, int r0, int r1, int c0, int c1,
-                                                  int k0, int nb, typename Prec<R>::C (*s0a)[CL_T + 1],
-                                                  typename Prec<R>::C (*s0b)[CL_T + 1],
-                                                  typename Prec<R>::C (*s1a)[CL_T + 1],
-                                                  typename Prec<R>::C (*s1b)[CL_T + 1]) {
-  if constexpr (std::is_same<R, double>::value) {
-    if (nb % CL_NB == 0) {
-      closed_gemm_dma<false>(W, D, nullptr, r0, r1, c0, c1, k0, nb, s0a, s0b, s1a, s1b);
-      return;
-    }
-  }
-  closed_update<R>(W, D, r0, r1, c0, c1, k0, nb, s0a, s0b);
-}
-
-// Z(k0 + i, c) <- sum_t T(i, t) Z(k0 + t, c) for i, t < nb (nb <= CL_BB) and every
-// column c in [c0, c1): T column-major with leading dimension CL_BB.  Each 64 x
-// 64 tile of Z is read whole (through LDS, CL_NB rows at a time) before its
-// result is written back, so the product runs in place.
-template <class R>
-__device__ void closed_apply_T(typename Prec<R>::C* W, const typename Prec<R>::C* T, int D, int k0, int nb, int c0,
-                               int c1, typename Prec<R>::C (*As)[CL_T + 1], typename Prec<R>::C (*Bs)[CL_T + 1]) {
-  using P = Prec<R>;
-  using C = typename P::C;
-  using V = typename P::V;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
-  const int li = lane & 15, lk = lane >> 4;
-  const C zero = mkc((R)0, (R)0);
-  for (int tc = c0; tc < c1; tc += CL_T) {
-    V ar[2][2], ai[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) ar[i][j] = ai[i][j] = V{};
-    // staging as in closed_update
-    constexpr bool kPrefetch = sizeof(R) == 4;
-    C pa[4], pb[4];
-    auto fetch = [&](int kc) {
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int row = tid & (CL_T - 1), ka = (tid >> 6) + 4 * v;
-        pa[v] = (row < nb && kc + ka < nb) ? T[(size_t)(kc + ka) * CL_BB + row] : zero;
-        const int kb = tid % CL_NB, col = (tid / CL_NB) + 16 * v;
-        pb[v] = (tc + col < c1 && kc + kb < nb) ? W[(size_t)(tc + col) * D + k0 + kc + kb] : zero;
-      }
-    };
-    if constexpr (kPrefetch) fetch(0);
-    for (int kc = 0; kc < nb; kc += CL_NB) {
-      if constexpr (kPrefetch) {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          As[(tid >> 6) + 4 * v][tid & (CL_T - 1)] = pa[v];
-          Bs[tid % CL_NB][(tid / CL_NB) + 16 * v] = pb[v];
-        }
-      } else {
-        for (int u = tid; u < CL_NB * CL_T; u += 256) {
-          const int row = u & (CL_T - 1), ka = u >> 6;
-          As[ka][row] = (row < nb && kc + ka < nb) ? T[(size_t)(kc + ka) * CL_BB + row] : zero;
-          const int kb = u % CL_NB, col = u / CL_NB;
-          Bs[kb][col] = (tc + col < c1 && kc + kb < nb) ? W[(size_t)(tc + col) * D + k0 + kc + kb] : zero;
-        }
-      }
-      __syncthreads();
-      if (kPrefetch && kc + CL_NB < nb) fetch(kc + CL_NB);
-#pragma unroll
-      for (int kk = 0; kk < CL_NB; kk += 4) {
-        C fa[2], fb[2];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) fa[i] = As[kk + lk][wr + i * 16 + li];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) fb[j] = Bs[kk + lk][wc + j * 16 + li];
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            // + A B: re += ar br - ai bi, im += ar bi + ai br
-            ar[i][j] = P::fma_add(fa[i].x, fb[j].x, ar[i][j]);
-            ar[i][j] = P::fma_sub(fa[i].y, fb[j].y, ar[i][j]);
-            ai[i][j] = P::fma_add(fa[i].x, fb[j].y, ai[i][j]);
-            ai[i][j] = P::fma_add(fa[i].y, fb[j].x, ai[i][j]);
-          }
-      }
-      __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int row = wr + i * 16 + P::orow(lk, e), col = tc + wc + j * 16 + li;
-          if (row < nb && col < c1) W[(size_t)col * D + k0 + row] = mkc(ar[i][j][e], ai[i][j][e]);
-        }
-  }
-  __syncthreads();
-}
-
-// the T products of the block elimination: in FP64 with the DMA stages when
-// nb allows, else (and in FP32) closed_apply_T on the first stage
-template <class R>
-__device__ __forceinline__ void closed_apply_T_b64(typename Prec<R>::C* W, const typename Prec<R>::C* T, int D, int k0,
-                                                   int nb, int c0, int c1, typename Prec<R>::C (*s0a)[CL_T + 1],
-                                                   typename Prec<R>::C (*s0b)[CL_T + 1],
-                                                   typename Prec<R>::C (*s1a)[CL_T + 1],
-                                                   typename Prec<R>::C (*s1b)[CL_T + 1]) {
-  if constexpr (std::is_same<R, double>::value) {
-    if (nb % CL_NB == 0) {
-      closed_gemm_dma<true>(W, D, T, 0, nb, c0, c1, k0, nb, s0a, s0b, s1a, s1b);
-      return;
-    }
-  }
-  closed_apply_T<R>(W, T, D, k0, nb, c0, c1, s0a, s0b);
 }
 
 // Z(k0 + i, c) <- sum_t M[i][t] Z(k0 + t, c) for i, t < nb and every column c in
@@ -838,44 +577,39 @@ __device__ __forceinline__ void list_moved_rows(const int* piv, int r0, int nr, 
   if (lane == 0) *cnt = ni + __popcll(mo);
 }
 
-// LU factorisation with partial pivoting in CL_BB-wide blocks, one workgroup per
-// (q, r) matrix.  For the block column k0 .. k0 + nb:
-//  A. its rows k0 .. D - 1 are copied to S and factored there (CL_NB-wide
-//     sub-panels: column-by-column within a sub-panel, then the sub-panel's
-//     rank-CL_NB update of the rest of the block); the row swaps are applied to
-//     the other columns of W and to perm, and the factors go back to W;
-//  B. L11^-1 and U11^-1 (nb x nb) from the factors, kept in T;
-//  C. the block rows of the later columns become U12 = L11^-1 Z1, in place;
-//  D. the rows below: Z -= L21 U12 (rank-nb MFMA updates).
-// The right-hand sides are no part of it: closed_lu_solve takes them through the
-// factors column panel by column panel, which is where 8 of the 10.7 D^3 flops are and
-// where the matrix alone would leave most of the chip to one workgroup's column steps.
-// (Gauss-Jordan on [A | Gamma] by one workgroup per matrix, 12 D^3: 28.1 ms at D = 320,
-// 480 q, against FACTOR_MS + SOLVE_MS.)
-// RP > 0 (D <= 256 RP): a sub-panel's column steps run on registers (thread t
-// holds rows s0 + t + 256 i, i < RP, of the CL_NB columns).  One barrier per
-// step: before it each wave leaves its best pivot candidate (by a wave
-// reduction) and that candidate's whole row in LDS, and thread c - s0 its row
-// c; after it every thread picks the same winner, the two rows are exchanged
-// from LDS and the rank-1 update runs on registers.  The swaps are recorded
-// as a row map; the rows they move (none when no row is swapped) reach the
-// other columns of the block at the end of the sub-panel and W at the end of
-// A.  RP = 0: every column step works on S in memory and swaps the rows of W
-// at once.
+// LU factorisation with partial pivoting in CL_BB-wide blocks, right-looking, in place in
+// W.  Per block column k0 .. k0 + nb, each a launch over every matrix:
+//  A. closed_panel: its rows k0 .. D - 1 factored by one workgroup per matrix (CL_NB-wide
+//     sub-panels: column by column within a sub-panel, then the sub-panel's rank-CL_NB
+//     update of the rest of the block); the row swaps are applied to the other columns
+//     of W and to perm;
+//  B. closed_diag: L11^-1 and U11^-1 (nb x nb) from the factors, kept in T;
+//  C. closed_row: the block rows of the later columns become U12 = L11^-1 Z1;
+//  D. closed_trail: the rows below, Z -= L21 U12, a 64 x 64 tile per workgroup.
+// The right-hand sides are no part of it: closed_lu_solve takes them through the factors
+// column panel by column panel, which is where 8 of the 10.7 D^3 flops are.  A is a chain
+// of column steps (a pivot search, an exchange and a rank-1 update between two barriers);
+// on its own it has the registers and the VALU for itself, where beside the products of
+// another workgroup every VALU instruction waits for an F64 MFMA.  D = 320, 480 q (1920
+// matrices): 8.9 ms in FP64 with the scaling of the block rows, 2.9 of them A (one kernel
+// per matrix doing all of it 14.2 ms; Gauss-Jordan on [A | Gamma] 28.1 ms against 8.9 + 10.0
+// with the right-hand sides).
+// closed_panel, RP > 0 (D - k0 <= 256 RP): a sub-panel's column steps run on registers
+// (thread t holds rows s0 + t + 256 i, i < RP, of the CL_NB columns).  One barrier per
+// step: before it each wave leaves its best pivot candidate (by a wave reduction) and
+// that candidate's whole row in LDS, and thread c - s0 its row c; after it every thread
+// picks the same winner, the two rows are exchanged from LDS and the rank-1 update runs
+// on registers.  The swaps are recorded as a row map; the rows they move (none when no
+// row is swapped) reach the other columns of the block at the end of the sub-panel and
+// the rest of W at the end of the block.  RP = 0: every column step works on W in memory
+// and swaps its rows at once.  grid: matrices
 template <class R, int RP>
-__global__ __launch_bounds__(256, 2) void closed_factor_b64(ClosedArgs a) {
+__global__ __launch_bounds__(256, RP == 1 ? 3 : 2) void closed_panel(ClosedArgs a, int k0) {
   using C = typename Prec<R>::C;
   constexpr int RMAX = RP > 0 ? 256 * RP : 1;  // rows of the register path
   constexpr int RQ = RP > 0 ? 1 : 0;
-  // two stages of the update; the first is also the staging of the other
-  // products (As, Bs), the second holds L11 and its inverse of a sub-panel
-  __shared__ C stages[4][CL_NB][CL_T + 1];  // As, Bs, As1, Bs1, one object so phase B can use them whole
-  C (*As)[CL_T + 1] = stages[0];
-  C (*Bs)[CL_T + 1] = stages[1];
-  C (*As1)[CL_T + 1] = stages[2];
-  C (*Bs1)[CL_T + 1] = stages[3];
-  C (*Ls)[CL_NB] = reinterpret_cast<C (*)[CL_NB]>(&As1[0][0]);
-  C (*Li)[CL_NB] = reinterpret_cast<C (*)[CL_NB]>(&Bs1[0][0]);
+  __shared__ C Ls[CL_NB][CL_NB];          // L11 of a sub-panel
+  __shared__ C Us[CL_NB][CL_BB - CL_NB];  // U12 beside it
   __shared__ R red_v[256 * (1 - RQ) + 1];
   __shared__ int red_i[256 * (1 - RQ) + 1];
   __shared__ unsigned long long pk[2][4 * RQ + 1];  // per-wave pivot keys, two buffers
@@ -885,391 +619,416 @@ __global__ __launch_bounds__(256, 2) void closed_factor_b64(ClosedArgs a) {
   __shared__ int map_s[RMAX], map_b[RMAX];     // row sources after the sub-panel's / block's swaps
   __shared__ int mv_dst[2 * CL_BB * RQ + 1], mv_src[2 * CL_BB * RQ + 1];
   __shared__ int mv_n;
-  const int mat = blockIdx.x;
-  const int D = a.D, nblk = (D + CL_BB - 1) / CL_BB;
+  const int mat = blockIdx.x, D = a.D, nb = min(CL_BB, D - k0);
   C* W = static_cast<C*>(a.W) + (size_t)mat * D * D;
-  C* S = static_cast<C*>(a.S) + (size_t)mat * CL_BB * D;
   int* perm = a.perm + (size_t)mat * (D + 1);
   const int tid = threadIdx.x;
-  const C one = mkc((R)1, (R)0), zero = mkc((R)0, (R)0);
+  const C zero = mkc((R)0, (R)0);
   int info = 0, moved = 0;
-  for (int x = tid; x < D; x += 256) perm[x] = x;
-  for (int k0 = 0; k0 < D; k0 += CL_BB) {
-    const int nb = min(CL_BB, D - k0);
-    // column-major, leading dimension CL_BB
-    C* Linv = static_cast<C*>(a.T) + ((size_t)mat * nblk + k0 / CL_BB) * 2 * CL_BB * CL_BB;
-    C* Uinv = Linv + CL_BB * CL_BB;
-    // S(row, col) for col in [k0, k0 + nb): Sk[col * D + row]
-    C* Sk = S - (size_t)k0 * D;
-    // A. copy, then factor
-    for (int u = tid; u < nb * (D - k0); u += 256) {
-      const int col = k0 + u / (D - k0), row = k0 + u % (D - k0);
-      Sk[(size_t)col * D + row] = W[(size_t)col * D + row];
-    }
-    if constexpr (RP > 0)
-      for (int x = k0 + tid; x < D; x += 256) map_b[x - k0] = x;
-    __syncthreads();
-    for (int s0 = k0; s0 < k0 + nb; s0 += CL_NB) {
-      const int sb = min(CL_NB, k0 + nb - s0);
-      if constexpr (RP > 0) {
-        const int lane = tid & 63, wave = tid >> 6;
-        for (int x = s0 + tid; x < D; x += 256) map_s[x - s0] = x;
-        C v[RP][CL_NB];
+  if (k0 == 0)
+    for (int x = tid; x <= D; x += 256) perm[x] = x < D ? x : 0;
+  if constexpr (RP > 0)
+    for (int x = k0 + tid; x < D; x += 256) map_b[x - k0] = x;
+  __syncthreads();
+  for (int s0 = k0; s0 < k0 + nb; s0 += CL_NB) {
+    const int sb = min(CL_NB, k0 + nb - s0);
+    if constexpr (RP > 0) {
+      const int lane = tid & 63, wave = tid >> 6;
+      for (int x = s0 + tid; x < D; x += 256) map_s[x - s0] = x;
+      C v[RP][CL_NB];
+#pragma unroll
+      for (int i = 0; i < RP; ++i) {
+        const int row = s0 + tid + 256 * i;
+#pragma unroll
+        for (int j = 0; j < CL_NB; ++j) v[i][j] = (row < D && j < sb) ? W[(size_t)(s0 + j) * D + row] : zero;
+      }
+      // the CL_NB steps unrolled: the register columns take static indices
+      static_for<0, CL_NB>([&](auto jc) {
+        constexpr int j = decltype(jc)::value, buf = j & 1;
+        if (j >= sb) return;
+        const int c = s0 + j;
+        C pc[RP];  // this thread's entries of column c
+#pragma unroll
+        for (int i = 0; i < RP; ++i) pc[i] = v[i][j];
+        unsigned long long key = 0ull;
 #pragma unroll
         for (int i = 0; i < RP; ++i) {
           const int row = s0 + tid + 256 * i;
-#pragma unroll
-          for (int j = 0; j < CL_NB; ++j) v[i][j] = (row < D && j < sb) ? Sk[(size_t)(s0 + j) * D + row] : zero;
+          if (row >= c && row < D) {
+            const unsigned long long k2 = pivot_key(fabs(pc[i].x) + fabs(pc[i].y), row - s0);
+            if (k2 > key) key = k2;
+          }
         }
-        // the CL_NB steps unrolled: the register columns take static indices
-        static_for<0, CL_NB>([&](auto jc) {
-          constexpr int j = decltype(jc)::value, buf = j & 1;
-          if (j >= sb) return;
-          const int c = s0 + j;
-          C pc[RP];  // this thread's entries of column c
+        key = wave_max_u64(key);  // the wave's candidate
+        const int bi = key ? s0 + 1023 - (int)(key & 0x3ff) : c;
+        const int tb = (bi - s0) & 255, ib = (bi - s0) >> 8;
+        if (tid == tb) {
 #pragma unroll
-          for (int i = 0; i < RP; ++i) pc[i] = v[i][j];
-          unsigned long long key = 0ull;
+          for (int i = 0; i < RP; ++i)
+            if (i == ib) {
 #pragma unroll
-          for (int i = 0; i < RP; ++i) {
-            const int row = s0 + tid + 256 * i;
-            if (row >= c && row < D) {
-              const unsigned long long k2 = pivot_key(fabs(pc[i].x) + fabs(pc[i].y), row - s0);
-              if (k2 > key) key = k2;
+              for (int jj = 0; jj < CL_NB; ++jj) cand[buf][wave][jj] = v[i][jj];
             }
-          }
-          key = wave_max_u64(key);  // the wave's candidate
-          const int bi = key ? s0 + 1023 - (int)(key & 0x3ff) : c;
-          const int tb = (bi - s0) & 255, ib = (bi - s0) >> 8;
-          if (tid == tb) {
+        }
+        if (tid == j) {
 #pragma unroll
-            for (int i = 0; i < RP; ++i)
-              if (i == ib) {
+          for (int jj = 0; jj < CL_NB; ++jj) crow[buf][jj] = v[0][jj];
+        }
+        if (lane == 0) pk[buf][wave] = key;
+        __syncthreads();
+        unsigned long long kmax = pk[buf][0];
+        int pw = 0;
 #pragma unroll
-                for (int jj = 0; jj < CL_NB; ++jj) cand[buf][wave][jj] = v[i][jj];
-              }
+        for (int w = 1; w < 4; ++w) {
+          const unsigned long long k2 = pk[buf][w];
+          if (k2 > kmax) {
+            kmax = k2;
+            pw = w;
           }
+        }
+        const int p = s0 + 1023 - (int)(kmax & 0x3ff);
+        if (!(pivot_mag(kmax) > 0)) {
+          if (info == 0) info = c + 1;
+          if (tid == 0) piv[c - k0] = c;
+          return;
+        }
+        const C* prw = cand[buf][pw];
+        const int tp = (p - s0) & 255, ip = (p - s0) >> 8;
+        if (p != c) {
           if (tid == j) {
 #pragma unroll
-            for (int jj = 0; jj < CL_NB; ++jj) crow[buf][jj] = v[0][jj];
+            for (int jj = 0; jj < CL_NB; ++jj) v[0][jj] = prw[jj];
           }
-          if (lane == 0) pk[buf][wave] = key;
-          __syncthreads();
-          unsigned long long kmax = pk[buf][0];
-          int pw = 0;
+          if (tid == tp) {
 #pragma unroll
-          for (int w = 1; w < 4; ++w) {
-            const unsigned long long k2 = pk[buf][w];
-            if (k2 > kmax) {
-              kmax = k2;
-              pw = w;
-            }
+            for (int i = 0; i < RP; ++i)
+              if (i == ip) {
+                pc[i] = crow[buf][j];
+#pragma unroll
+                for (int jj = 0; jj < CL_NB; ++jj) v[i][jj] = crow[buf][jj];
+              }
           }
-          const int p = s0 + 1023 - (int)(kmax & 0x3ff);
-          if (!(pivot_mag(kmax) > 0)) {
-            if (info == 0) info = c + 1;
-            if (tid == 0) piv[c - k0] = c;
-            return;
-          }
-          const C* prw = cand[buf][pw];
-          const int tp = (p - s0) & 255, ip = (p - s0) >> 8;
+        }
+        if (tid == 0) {
+          piv[c - k0] = p;
           if (p != c) {
-            if (tid == j) {
-#pragma unroll
-              for (int jj = 0; jj < CL_NB; ++jj) v[0][jj] = prw[jj];
-            }
-            if (tid == tp) {
-#pragma unroll
-              for (int i = 0; i < RP; ++i)
-                if (i == ip) {
-                  pc[i] = crow[buf][j];
-#pragma unroll
-                  for (int jj = 0; jj < CL_NB; ++jj) v[i][jj] = crow[buf][jj];
-                }
-            }
+            const int t1 = map_s[c - s0];
+            map_s[c - s0] = map_s[p - s0];
+            map_s[p - s0] = t1;
+            const int t2 = map_b[c - k0];
+            map_b[c - k0] = map_b[p - k0];
+            map_b[p - k0] = t2;
           }
-          if (tid == 0) {
-            piv[c - k0] = p;
-            if (p != c) {
-              const int t1 = map_s[c - s0];
-              map_s[c - s0] = map_s[p - s0];
-              map_s[p - s0] = t1;
-              const int t2 = map_b[c - k0];
-              map_b[c - k0] = map_b[p - k0];
-              map_b[p - k0] = t2;
-            }
-          }
-          const C inv = cinv(prw[j]);
-#pragma unroll
-          for (int i = 0; i < RP; ++i) {
-            const int row = s0 + tid + 256 * i;
-            if (row > c && row < D) {
-              const C l = cmul(pc[i], inv);
-              v[i][j] = l;
-#pragma unroll
-              for (int jj = j + 1; jj < CL_NB; ++jj) v[i][jj] = csub(v[i][jj], cmul(l, prw[jj]));
-            }
-          }
-        });
+        }
+        const C inv = cinv(prw[j]);
 #pragma unroll
         for (int i = 0; i < RP; ++i) {
           const int row = s0 + tid + 256 * i;
-          if (row < D)
+          if (row > c && row < D) {
+            const C l = cmul(pc[i], inv);
+            v[i][j] = l;
 #pragma unroll
-            for (int j = 0; j < CL_NB; ++j)
-              if (j < sb) Sk[(size_t)(s0 + j) * D + row] = v[i][j];
-        }
-        // the sub-panel's swaps on the other columns of the block
-        if (wave == 0) list_moved_rows(piv + (s0 - k0), s0, sb, map_s, s0, mv_dst, mv_src, &mv_n);
-        __syncthreads();
-        move_rows<R, 8>(Sk, D, k0, k0 + nb, s0, s0 + sb, mv_dst, mv_src, mv_n);
-        __syncthreads();
-      } else
-      for (int c = s0; c < s0 + sb; ++c) {
-        R best = -1;
-        int bi = c;
-        for (int row = c + tid; row < D; row += 256) {
-          const C v = Sk[(size_t)c * D + row];
-          const R m = fabs(v.x) + fabs(v.y);
-          if (m > best) {
-            best = m;
-            bi = row;
+            for (int jj = j + 1; jj < CL_NB; ++jj) v[i][jj] = csub(v[i][jj], cmul(l, prw[jj]));
           }
         }
-        red_v[tid] = best;
-        red_i[tid] = bi;
-        __syncthreads();
-        for (int st = 128; st > 0; st >>= 1) {
-          if (tid < st) {
-            const R o = red_v[tid + st];
-            const int oi = red_i[tid + st];
-            if (o > red_v[tid] || (o == red_v[tid] && oi < red_i[tid])) {
-              red_v[tid] = o;
-              red_i[tid] = oi;
-            }
-          }
-          __syncthreads();
-        }
-        const int p = red_i[0];
-        const R pmax = red_v[0];
-        __syncthreads();
-        if (!(pmax > 0)) {  // zero or NaN pivot column: the system is singular
-          if (info == 0) info = c + 1;
-          continue;
-        }
-        if (p != c) {
-          if (tid == 0) {
-            const int x = perm[c];
-            perm[c] = perm[p];
-            perm[p] = x;
-          }
-          moved = 1;
-          for (int col = tid; col < D; col += 256) {
-            const C x = W[(size_t)col * D + c];
-            W[(size_t)col * D + c] = W[(size_t)col * D + p];
-            W[(size_t)col * D + p] = x;
-          }
-          for (int col = k0 + tid; col < k0 + nb; col += 256) {
-            const C x = Sk[(size_t)col * D + c];
-            Sk[(size_t)col * D + c] = Sk[(size_t)col * D + p];
-            Sk[(size_t)col * D + p] = x;
-          }
-        }
-        __syncthreads();
-        const C inv = cinv(Sk[(size_t)c * D + c]);
-        for (int row = c + 1 + tid; row < D; row += 256) {
-          const C l = cmul(Sk[(size_t)c * D + row], inv);
-          Sk[(size_t)c * D + row] = l;
-          for (int col = c + 1; col < s0 + sb; ++col)
-            Sk[(size_t)col * D + row] = csub(Sk[(size_t)col * D + row], cmul(l, Sk[(size_t)col * D + c]));
-        }
-        __syncthreads();
+      });
+#pragma unroll
+      for (int i = 0; i < RP; ++i) {
+        const int row = s0 + tid + 256 * i;
+        if (row < D)
+#pragma unroll
+          for (int j = 0; j < CL_NB; ++j)
+            if (j < sb) W[(size_t)(s0 + j) * D + row] = v[i][j];
       }
-      if (s0 + sb < k0 + nb) {
-        // the rest of the block: U12 = L11^-1 S12 on the sub-panel rows, S22 -= L21 U12 below
-        for (int u = tid; u < CL_NB * CL_NB; u += 256) {
-          const int i = u % CL_NB, j = u / CL_NB;
-          Ls[i][j] = (i < sb && j < sb) ? Sk[(size_t)(s0 + j) * D + s0 + i] : zero;
-        }
-        __syncthreads();
-        if (tid < CL_NB) {
-          const int t = tid;
-          for (int i = 0; i < CL_NB; ++i) {
-            C x = i == t ? one : zero;
-            if (i < sb && t < sb)
-              for (int s2 = t; s2 < i; ++s2) x = csub(x, cmul(Ls[i][s2], Li[s2][t]));
-            Li[i][t] = x;
-          }
-        }
-        __syncthreads();
-        panel_rows_apply<R>(Sk, D, s0, sb, s0 + sb, k0 + nb, Li);
-        __syncthreads();
-        closed_update_b64<R>(Sk, D, s0 + sb, D, s0 + sb, k0 + nb, s0, sb, As, Bs, As1, Bs1);
-      }
-    }
-    if constexpr (RP > 0) {  // the block's swaps on W (its own columns are replaced below) and perm
-      if (tid < 64) list_moved_rows(piv, k0, nb, map_b, k0, mv_dst, mv_src, &mv_n);
+      // the sub-panel's swaps on the other columns of the block
+      if (wave == 0) list_moved_rows(piv + (s0 - k0), s0, sb, map_s, s0, mv_dst, mv_src, &mv_n);
       __syncthreads();
-      if (mv_n) {
+      move_rows<R, 8>(W, D, k0, k0 + nb, s0, s0 + sb, mv_dst, mv_src, mv_n);
+      __syncthreads();
+    } else
+    for (int c = s0; c < s0 + sb; ++c) {
+      R best = -1;
+      int bi = c;
+      for (int row = c + tid; row < D; row += 256) {
+        const C v = W[(size_t)c * D + row];
+        const R m = fabs(v.x) + fabs(v.y);
+        if (m > best) {
+          best = m;
+          bi = row;
+        }
+      }
+      red_v[tid] = best;
+      red_i[tid] = bi;
+      __syncthreads();
+      for (int st = 128; st > 0; st >>= 1) {
+        if (tid < st) {
+          const R o = red_v[tid + st];
+          const int oi = red_i[tid + st];
+          if (o > red_v[tid] || (o == red_v[tid] && oi < red_i[tid])) {
+            red_v[tid] = o;
+            red_i[tid] = oi;
+          }
+        }
+        __syncthreads();
+      }
+      const int p = red_i[0];
+      const R pmax = red_v[0];
+      __syncthreads();
+      if (!(pmax > 0)) {  // zero or NaN pivot column: the system is singular
+        if (info == 0) info = c + 1;
+        continue;
+      }
+      if (p != c) {
+        if (tid == 0) {
+          const int x = perm[c];
+          perm[c] = perm[p];
+          perm[p] = x;
+        }
         moved = 1;
-        const int px = tid < mv_n ? perm[mv_src[tid]] : 0;
-        __syncthreads();
-        if (tid < mv_n) perm[mv_dst[tid]] = px;
-        move_rows_waves<R, 8>(W, D, 0, D, mv_dst, mv_src, mv_n);
-        __syncthreads();
-      }
-    }
-    for (int u = tid; u < nb * (D - k0); u += 256) {
-      const int col = k0 + u / (D - k0), row = k0 + u % (D - k0);
-      W[(size_t)col * D + row] = Sk[(size_t)col * D + row];
-    }
-    // B. L11^-1 and U11^-1 (identity-padded to CL_BB) by 16 x 16 blocks: the
-    // inverses of the four diagonal blocks of L11 and U11 from copies in LDS
-    // (thread = block column), then the off-diagonal blocks by their distance d
-    // from the diagonal, all blocks at one distance at once,
-    //   Linv_ab = -Linv_aa sum_{c=b}^{a-1} L_ac Linv_cb      (a > b)
-    //   Uinv_ab = -Uinv_aa sum_{c=a+1}^{b} U_ac Uinv_cb      (a < b).
-    {
-      constexpr int NBB = CL_BB / CL_NB;
-      // L11 (unit lower) and U11 (upper) entry (i, s), identity beyond nb
-      auto Lv = [&](int i, int s2) -> C {
-        if (i >= nb || s2 >= nb) return i == s2 ? one : zero;
-        return i > s2 ? Sk[(size_t)(k0 + s2) * D + k0 + i] : (i == s2 ? one : zero);
-      };
-      auto Uv = [&](int i, int s2) -> C {
-        if (i >= nb || s2 >= nb) return i == s2 ? one : zero;
-        return i <= s2 ? Sk[(size_t)(k0 + s2) * D + k0 + i] : zero;
-      };
-      C* Ld = &As[0][0];  // the NBB diagonal blocks of L11, [blk][col][row]
-      C* Ud = &Bs[0][0];  // and of U11
-      for (int u = tid; u < NBB * CL_NB * CL_NB; u += 256) {
-        const int blk = u / (CL_NB * CL_NB), e = u % (CL_NB * CL_NB), i = e % CL_NB, j = e / CL_NB;
-        Ld[u] = Lv(blk * CL_NB + i, blk * CL_NB + j);
-        Ud[u] = Uv(blk * CL_NB + i, blk * CL_NB + j);
+        for (int col = tid; col < D; col += 256) {
+          const C x = W[(size_t)col * D + c];
+          W[(size_t)col * D + c] = W[(size_t)col * D + p];
+          W[(size_t)col * D + p] = x;
+        }
       }
       __syncthreads();
-      if (tid < 2 * NBB * CL_NB) {
-        const bool up = tid >= NBB * CL_NB;
-        const int blk = (tid / CL_NB) % NBB, t = tid % CL_NB, off = blk * CL_NB;
-        const C* Md = (up ? Ud : Ld) + blk * CL_NB * CL_NB;
-        C* out = (up ? Uinv : Linv) + (size_t)(off + t) * CL_BB + off;  // column t of the diagonal block
-        C x[CL_NB];  // the column, in registers (static indices)
-        if (!up) {
-#pragma unroll
-          for (int i = 0; i < CL_NB; ++i) {
-            C v = i == t ? one : zero;
-#pragma unroll
-            for (int s2 = 0; s2 < i; ++s2)
-              if (s2 >= t) v = csub(v, cmul(Md[s2 * CL_NB + i], x[s2]));
-            x[i] = v;
-          }
-        } else {
-#pragma unroll
-          for (int i = CL_NB - 1; i >= 0; --i) {
-            C v = i == t ? one : zero;
-#pragma unroll
-            for (int s2 = i + 1; s2 < CL_NB; ++s2)
-              if (s2 <= t) v = csub(v, cmul(Md[s2 * CL_NB + i], x[s2]));
-            x[i] = cmul(v, cinv(Md[i * CL_NB + i]));
-          }
-        }
-#pragma unroll
-        for (int i = 0; i < CL_NB; ++i) out[i] = x[i];
-      }
-      // zero blocks: above the diagonal of Linv, below it of Uinv
-      for (int u = tid; u < CL_BB * CL_BB; u += 256) {
-        const int i = u % CL_BB, j = u / CL_BB;
-        if (i / CL_NB < j / CL_NB) Linv[u] = zero;
-        if (i / CL_NB > j / CL_NB) Uinv[u] = zero;
+      const C inv = cinv(W[(size_t)c * D + c]);
+      for (int row = c + 1 + tid; row < D; row += 256) {
+        const C l = cmul(W[(size_t)c * D + row], inv);
+        W[(size_t)c * D + row] = l;
+        for (int col = c + 1; col < s0 + sb; ++col)
+          W[(size_t)col * D + row] = csub(W[(size_t)col * D + row], cmul(l, W[(size_t)col * D + c]));
       }
       __syncthreads();
-      // the blocks of one distance through LDS (the stages are free here):
-      // per pair P (L pairs, then U pairs) the block row X_P (16 x w, rows
-      // padded to w + 1) and block column Y_P (w x 16) of the product, w = 16 d,
-      // M_P = X_P Y_P kept in registers, then M_P and the diagonal block
-      // (transposed) of the triangle's inverse for -Dinv_aa M_P
-      C* stg = &As[0][0];
-      for (int d = 1; d < NBB; ++d) {
-        const int np = NBB - d, w = CL_NB * d, per = 2 * CL_NB * w + CL_NB;
-        for (int u = tid; u < 2 * np * CL_NB * w; u += 256) {
-          const int pr = u / (CL_NB * w), e = u % (CL_NB * w);
-          const bool upp = pr >= np;
-          const int a2 = upp ? pr - np : d + pr, b2 = upp ? a2 + d : pr;
-          const int c0b = upp ? a2 + 1 : b2;  // first block of the inner range
-          C* X = stg + pr * per;
-          C* Y = X + CL_NB * (w + 1);
-          {  // X(i, kk): row a2 * 16 + i of the triangle, column c0b * 16 + kk
-            const int i = e / w, kk = e % w;
-            X[i * (w + 1) + kk] = upp ? Uv(a2 * CL_NB + i, c0b * CL_NB + kk) : Lv(a2 * CL_NB + i, c0b * CL_NB + kk);
-          }
-          {  // Y(kk, j): the inverse's row c0b * 16 + kk, column b2 * 16 + j
-            const int kk = e / CL_NB, j = e % CL_NB;
-            Y[kk * CL_NB + j] = (upp ? Uinv : Linv)[(size_t)(b2 * CL_NB + j) * CL_BB + c0b * CL_NB + kk];
-          }
-        }
-        __syncthreads();
-        constexpr int MP = (2 * (NBB - 1) * CL_NB * CL_NB + 255) / 256;  // pair elements per thread, at most
-        C mr[MP];
+    }
+    if (s0 + sb < k0 + nb) {
+      // the rest of the block (sb = CL_NB here): U12 = L11^-1 Z12 on the sub-panel rows by
+      // substitution, a column per thread, kept in LDS as well; then Z22 -= L21 U12, each
+      // wave taking strips of 16 rows with L21 and Z22 straight from memory
+      const int c1 = s0 + CL_NB, nc = k0 + nb - c1;  // at most CL_BB - CL_NB columns
+      if (tid < CL_NB * CL_NB) {
+        const int i = tid % CL_NB, j = tid / CL_NB;
+        Ls[i][j] = W[(size_t)(s0 + j) * D + s0 + i];
+      }
+      __syncthreads();
+      if (tid < nc) {
+        C* zc = W + (size_t)(c1 + tid) * D + s0;
+        C z[CL_NB];
 #pragma unroll
-        for (int q = 0; q < MP; ++q) {
-          const int u = tid + 256 * q;
-          mr[q] = zero;
-          if (u < 2 * np * CL_NB * CL_NB) {
-            const int pr = u / (CL_NB * CL_NB), e = u % (CL_NB * CL_NB), i = e % CL_NB, j = e / CL_NB;
-            const C* X = stg + pr * per;
-            const C* Y = X + CL_NB * (w + 1);
-            R xr = 0, xi = 0;
-            for (int kk = 0; kk < w; ++kk) {
-              const C x = X[i * (w + 1) + kk], y = Y[kk * CL_NB + j];
-              xr = fma(x.x, y.x, fma(-x.y, y.y, xr));
-              xi = fma(x.x, y.y, fma(x.y, y.x, xi));
+        for (int i = 0; i < CL_NB; ++i) z[i] = zc[i];
+#pragma unroll
+        for (int i = 1; i < CL_NB; ++i) {
+          __builtin_amdgcn_sched_barrier(0);  // L11 is read row by row, not all ahead into registers
+#pragma unroll
+          for (int s2 = 0; s2 < i; ++s2) z[i] = csub(z[i], cmul(Ls[i][s2], z[s2]));
+        }
+#pragma unroll
+        for (int i = 0; i < CL_NB; ++i) {
+          zc[i] = z[i];
+          Us[i][tid] = z[i];
+        }
+      }
+      __syncthreads();
+      {
+        using P = Prec<R>;
+        using V = typename P::V;
+        const int lane = tid & 63, wave = tid >> 6, li = lane & 15, lk = lane >> 4;
+        for (int r0 = c1 + 16 * wave; r0 < D; r0 += 64) {
+          C fa[CL_NB / 4];
+          const int ar = min(r0 + li, D - 1);
+#pragma unroll
+          for (int ks = 0; ks < CL_NB / 4; ++ks) fa[ks] = W[(size_t)(s0 + 4 * ks + lk) * D + ar];
+#pragma unroll
+          for (int cb = 0; cb < (CL_BB - CL_NB) / 16; ++cb) {
+            if (16 * cb >= nc) break;
+            const int col = 16 * cb + li;
+            C* zc = W + (size_t)(c1 + min(col, nc - 1)) * D;
+            V zr, zi;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const C z = zc[min(r0 + P::orow(lk, e), D - 1)];
+              zr[e] = z.x;
+              zi[e] = z.y;
             }
-            mr[q] = mkc(xr, xi);
-          }
-        }
-        __syncthreads();
-        // M_P at stg[P 512 ..], the diagonal block a of the inverse transposed after it
-        for (int u = tid; u < 2 * np * CL_NB * CL_NB; u += 256) {
-          const int pr = u / (CL_NB * CL_NB), e = u % (CL_NB * CL_NB), i = e % CL_NB, k = e / CL_NB;
-          const bool upp = pr >= np;
-          const int a2 = upp ? pr - np : d + pr;
-          const C* Dg = (upp ? Uinv : Linv) + (size_t)(a2 * CL_NB) * CL_BB + a2 * CL_NB;
-          stg[pr * 2 * CL_NB * CL_NB + CL_NB * CL_NB + k * CL_NB + i] = Dg[(size_t)k * CL_BB + i];
-        }
 #pragma unroll
-        for (int q = 0; q < MP; ++q) {
-          const int u = tid + 256 * q;
-          if (u < 2 * np * CL_NB * CL_NB) {
-            const int pr = u / (CL_NB * CL_NB), e = u % (CL_NB * CL_NB);
-            stg[pr * 2 * CL_NB * CL_NB + e] = mr[q];  // M_P(i, j) at e = j 16 + i
+            for (int ks = 0; ks < CL_NB / 4; ++ks) {
+              const C b = Us[4 * ks + lk][col];
+              zr = P::fma_sub(fa[ks].x, b.x, zr);
+              zi = P::fma_sub(fa[ks].x, b.y, zi);
+              zr = P::fma_add(fa[ks].y, b.y, zr);
+              zi = P::fma_sub(fa[ks].y, b.x, zi);
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const int row = r0 + P::orow(lk, e);
+              if (row < D && col < nc) zc[row] = mkc(zr[e], zi[e]);
+            }
           }
         }
-        __syncthreads();
-        for (int u = tid; u < 2 * np * CL_NB * CL_NB; u += 256) {
-          const int pr = u / (CL_NB * CL_NB), e = u % (CL_NB * CL_NB), i = e % CL_NB, j = e / CL_NB;
-          const bool upp = pr >= np;
-          const int a2 = upp ? pr - np : d + pr, b2 = upp ? a2 + d : pr;
-          const C* Mp = stg + pr * 2 * CL_NB * CL_NB;
-          const C* Dt = Mp + CL_NB * CL_NB;
-          R xr = 0, xi = 0;
-          for (int k = 0; k < CL_NB; ++k) {
-            const C g = Dt[k * CL_NB + i], m = Mp[j * CL_NB + k];
-            xr = fma(g.x, m.x, fma(-g.y, m.y, xr));
-            xi = fma(g.x, m.y, fma(g.y, m.x, xi));
-          }
-          (upp ? Uinv : Linv)[(size_t)(b2 * CL_NB + j) * CL_BB + a2 * CL_NB + i] = mkc(-xr, -xi);
-        }
-        __syncthreads();
       }
+      __syncthreads();
     }
-    const int j0 = k0 + nb;
-    // C. block rows of the later columns: U12 = L11^-1 Z1
-    closed_apply_T_b64<R>(W, Linv, D, k0, nb, j0, D, As, Bs, As1, Bs1);
-    // D. rows below the block
-    closed_update_b64<R>(W, D, j0, D, j0, D, k0, nb, As, Bs, As1, Bs1);
   }
-  if (info && tid == 0) atomicCAS(a.info, 0, info);
-  if (tid == 0) perm[D] = moved;
+  if constexpr (RP > 0) {  // the block's swaps on the other columns of W and on perm
+    if (tid < 64) list_moved_rows(piv, k0, nb, map_b, k0, mv_dst, mv_src, &mv_n);
+    __syncthreads();
+    if (mv_n) {
+      moved = 1;
+      const int px = tid < mv_n ? perm[mv_src[tid]] : 0;
+      __syncthreads();
+      if (tid < mv_n) perm[mv_dst[tid]] = px;
+      move_rows_waves<R, 8>(W, D, 0, k0, mv_dst, mv_src, mv_n);
+      move_rows_waves<R, 8>(W, D, k0 + nb, D, mv_dst, mv_src, mv_n);
+    }
+    __syncthreads();
+  }
+  if (tid == 0) {
+    if (info) atomicCAS(a.info, 0, info);
+    if (moved) perm[D] = 1;
+  }
+}
+
+// grid: matrices
+template <class R>
+__global__ __launch_bounds__(256, 2) void closed_diag(ClosedArgs a, int k0) {
+  using C = typename Prec<R>::C;
+  __shared__ C block[CL_BB][CL_BB + 1];
+  __shared__ C dinv[CL_BB];  // reciprocals of U11's diagonal
+  const int mat = blockIdx.x, D = a.D, nb = min(CL_BB, D - k0), nblk = (D + CL_BB - 1) / CL_BB;
+  const C* W = static_cast<const C*>(a.W) + (size_t)mat * D * D;
+  // column-major, leading dimension CL_BB
+  C* Linv = static_cast<C*>(a.T) + ((size_t)mat * nblk + k0 / CL_BB) * 2 * CL_BB * CL_BB;
+  C* Uinv = Linv + CL_BB * CL_BB;
+  const int tid = threadIdx.x;
+  const C one = mkc((R)1, (R)0), zero = mkc((R)0, (R)0);
+  // L11^-1 and U11^-1 (identity-padded to CL_BB) in place in LDS, where the block lies
+  // packed (L below, U on and above the diagonal): the inverses of the four diagonal 16 x
+  // 16 blocks of each (a column per thread, in registers), then, block column by block
+  // column from where the inverse is done, on MFMA
+  //   Linv(a, b) = -sum_{c = b+1}^{a} Linv(a, c) L(c, b) Linv(b, b)    b = 2, 1, 0
+  //   Uinv(a, b) = -sum_{c = a}^{b-1} Uinv(a, c) U(c, b) Uinv(b, b)    b = 1, 2, 3
+  {
+    using P = Prec<R>;
+    using V = typename P::V;
+    constexpr int LD = CL_BB + 1;  // a column's stride, free of bank conflicts
+    C* B = &block[0][0];           // B[col LD + row]
+    for (int u = tid; u < CL_BB * CL_BB; u += 256) {
+      const int i = u % CL_BB, j = u / CL_BB;
+      B[j * LD + i] = (i < nb && j < nb) ? W[(size_t)(k0 + j) * D + k0 + i] : (i == j ? one : zero);
+    }
+    __syncthreads();
+    if (tid < CL_BB) dinv[tid] = cinv(B[tid * LD + tid]);
+    __syncthreads();
+    {
+      const bool up = tid >= CL_BB;
+      const int t = tid % CL_NB, off = (tid / CL_NB) % (CL_BB / CL_NB) * CL_NB;
+      const C* Md = B + off * LD + off;
+      C x[CL_NB];  // column t of the diagonal block's inverse
+      if (tid < CL_BB) {
+#pragma unroll
+        for (int i = 0; i < CL_NB; ++i) {
+          __builtin_amdgcn_sched_barrier(0);
+          C v = i == t ? one : zero;
+#pragma unroll
+          for (int s2 = 0; s2 < i; ++s2)
+            if (s2 >= t) v = csub(v, cmul(Md[s2 * LD + i], x[s2]));
+          x[i] = v;
+        }
+      } else if (tid < 2 * CL_BB) {
+#pragma unroll
+        for (int i = CL_NB - 1; i >= 0; --i) {
+          __builtin_amdgcn_sched_barrier(0);
+          C v = i == t ? one : zero;
+#pragma unroll
+          for (int s2 = i + 1; s2 < CL_NB; ++s2)
+            if (s2 <= t) v = csub(v, cmul(Md[s2 * LD + i], x[s2]));
+          x[i] = cmul(v, dinv[off + i]);
+        }
+      }
+      __syncthreads();
+      if (tid < 2 * CL_BB) {
+        C* out = B + (off + t) * LD + off;
+#pragma unroll
+        for (int i = 0; i < CL_NB; ++i)
+          if (up ? i <= t : i > t) out[i] = x[i];
+      }
+      __syncthreads();
+    }
+    const int lane = tid & 63, wave = tid >> 6, li = lane & 15, lk = lane >> 4;
+    // entry (i, k) of a diagonal block's inverse, whose other triangle is not its own
+    auto diag = [&](bool up, C v, int i, int k) -> C {
+      if (up) return i <= k ? v : zero;
+      return i > k ? v : (i == k ? one : zero);
+    };
+    for (int st = 0; st < CL_BB / CL_NB - 1; ++st) {
+      // 2 (st + 1) blocks, up to two a wave: those of L's column 2 - st, then U's st + 1
+      V yr[2], yi[2];
+      int ba[2], bb[2];
+      bool upp[2], has[2];
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int job = wave + 4 * q;
+        has[q] = job < 2 * (st + 1);
+        upp[q] = job > st;
+        bb[q] = upp[q] ? st + 1 : 2 - st;
+        ba[q] = upp[q] ? job - (st + 1) : bb[q] + 1 + job;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) yr[q][e] = yi[q][e] = 0;
+        if (!has[q]) continue;
+        const int cb = upp[q] ? ba[q] : bb[q] + 1, ce = upp[q] ? bb[q] - 1 : ba[q];
+        for (int c = cb; c <= ce; ++c)
+#pragma unroll
+          for (int ks = 0; ks < CL_NB / 4; ++ks) {
+            const int kk = 4 * ks + lk;
+            C x = B[(c * CL_NB + kk) * LD + ba[q] * CL_NB + li];
+            if (c == ba[q]) x = diag(upp[q], x, li, kk);
+            const C y = B[(bb[q] * CL_NB + li) * LD + c * CL_NB + kk];
+            yr[q] = P::fma_add(x.x, y.x, yr[q]);
+            yi[q] = P::fma_add(x.x, y.y, yi[q]);
+            yr[q] = P::fma_sub(x.y, y.y, yr[q]);
+            yi[q] = P::fma_add(x.y, y.x, yi[q]);
+          }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        if (has[q])
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            B[(bb[q] * CL_NB + li) * LD + ba[q] * CL_NB + P::orow(lk, e)] = mkc(yr[q][e], yi[q][e]);
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) yr[q][e] = yi[q][e] = 0;
+        if (!has[q]) continue;
+#pragma unroll
+        for (int ks = 0; ks < CL_NB / 4; ++ks) {
+          const int kk = 4 * ks + lk;
+          const C x = B[(bb[q] * CL_NB + kk) * LD + ba[q] * CL_NB + li];
+          const C y = diag(upp[q], B[(bb[q] * CL_NB + li) * LD + bb[q] * CL_NB + kk], kk, li);
+          yr[q] = P::fma_sub(x.x, y.x, yr[q]);
+          yi[q] = P::fma_sub(x.x, y.y, yi[q]);
+          yr[q] = P::fma_add(x.y, y.y, yr[q]);
+          yi[q] = P::fma_sub(x.y, y.x, yi[q]);
+        }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        if (has[q])
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            B[(bb[q] * CL_NB + li) * LD + ba[q] * CL_NB + P::orow(lk, e)] = mkc(yr[q][e], yi[q][e]);
+      __syncthreads();
+    }
+    for (int u = tid; u < CL_BB * CL_BB; u += 256) {
+      const int i = u % CL_BB, j = u / CL_BB;
+      const C v = B[j * LD + i];
+      Linv[u] = i > j ? v : (i == j ? one : zero);
+      Uinv[u] = i <= j ? v : zero;
+    }
+  }
 }
 
 // ---- refinement products ------------------------------------------------------------
@@ -1464,6 +1223,67 @@ __global__ __launch_bounds__(256, 3) void closed_scale(ClosedArgs a) {
       for (int e = 0; e < 4; ++e) {
         const int row = wr + i * 16 + P::orow(lk, e), col = wc + j * 16 + li;
         if (row < nb && col < nc) W[(size_t)col * D + row] = mkc(-ar[i][j][e], -ai[i][j][e]);
+      }
+}
+
+// U12 = L11^-1 Z1 for a 64-column panel right of the block, in place; grid: the panels of
+// every matrix
+template <class R>
+__global__ __launch_bounds__(256, 3) void closed_row(ClosedArgs a, int k0) {
+  using P = Prec<R>;
+  using C = typename P::C;
+  using V = typename P::V;
+  __shared__ __attribute__((aligned(16))) char stage[TILE_STAGES * 16384];
+  const int D = a.D, nblk = (D + CL_BB - 1) / CL_BB, j0 = k0 + CL_BB, per = nblk - k0 / CL_BB - 1;
+  const int logical = closed_xcd_remap(blockIdx.x, gridDim.x);
+  const int mat = logical / per, c0 = j0 + (logical - mat * per) * CL_T, nc = min(CL_T, D - c0);
+  C* Z = static_cast<C*>(a.W) + (size_t)mat * D * D + (size_t)c0 * D + k0;
+  const C* T = static_cast<const C*>(a.T) + ((size_t)mat * nblk + k0 / CL_BB) * 2 * CL_BB * CL_BB;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32, li = lane & 15, lk = lane >> 4;
+  V ar[2][2], ai[2][2];
+  tile_product<R>({T, Z, CL_BB, 0}, {T, Z, CL_BB, CL_BB}, D, CL_BB, nc, stage, ar, ai);
+  // every wave's loads have landed before the last barrier: the panel may be replaced
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int row = wr + i * 16 + P::orow(lk, e), col = wc + j * 16 + li;
+        if (col < nc) Z[(size_t)col * D + row] = mkc(ar[i][j][e], ai[i][j][e]);
+      }
+}
+
+// Z -= L21 U12 for one 64 x 64 tile below and right of the block; grid: the tiles of every
+// matrix
+template <class R>
+__global__ __launch_bounds__(256, 3) void closed_trail(ClosedArgs a, int k0) {
+  using P = Prec<R>;
+  using C = typename P::C;
+  using V = typename P::V;
+  __shared__ __attribute__((aligned(16))) char stage[TILE_STAGES * 16384];
+  const int D = a.D, j0 = k0 + CL_BB, n = (D - j0 + CL_T - 1) / CL_T, per = n * n;
+  const int logical = closed_xcd_remap(blockIdx.x, gridDim.x);
+  const int mat = logical / per, t = logical - mat * per;
+  const int r0 = j0 + t % n * CL_T, c0 = j0 + t / n * CL_T, nr = min(CL_T, D - r0), nc = min(CL_T, D - c0);
+  C* W = static_cast<C*>(a.W) + (size_t)mat * D * D;
+  C* Z = W + (size_t)c0 * D + r0;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32, li = lane & 15, lk = lane >> 4;
+  V ar[2][2], ai[2][2];
+  const TileSeg<C> s{W + (size_t)k0 * D + r0, W + (size_t)c0 * D + k0, D, CL_BB};
+  tile_product<R>({s.a, s.b, D, 0}, s, D, nr, nc, stage, ar, ai);
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int row = wr + i * 16 + P::orow(lk, e), col = wc + j * 16 + li;
+        if (row >= nr || col >= nc) continue;
+        C* z = Z + (size_t)col * D + row;
+        *z = csub(*z, mkc(ar[i][j][e], ai[i][j][e]));
       }
 }
 
@@ -1739,8 +1559,8 @@ static bool closed_regs(const tups_ctx* c) {
 }
 // scratch of closed_solve_b64 per matrix, in complex elements
 static size_t closed_blocks(size_t D) { return (D + CL_BB - 1) / CL_BB; }
-// per matrix of the block form: the factors, the block column in work and the diagonal inverses
-static size_t closed_b64_elems(size_t D) { return D * D + (size_t)CL_BB * D + 2 * closed_blocks(D) * CL_BB * CL_BB; }
+// per matrix of the block form: the factors and the diagonal inverses
+static size_t closed_b64_elems(size_t D) { return D * D + 2 * closed_blocks(D) * CL_BB * CL_BB; }
 
 // the block form's parts of a workspace from `at` on; returns its end
 template <class C>
@@ -1748,8 +1568,6 @@ static int* place_b64(ClosedArgs& a, C* at, size_t mats) {
   const size_t D = a.D;
   a.W = at;
   at += mats * D * D;
-  a.S = at;
-  at += mats * CL_BB * D;
   a.T = at;
   at += mats * closed_blocks(D) * 2 * CL_BB * CL_BB;
   a.perm = reinterpret_cast<int*>(at);
@@ -1759,12 +1577,23 @@ static int* place_b64(ClosedArgs& a, C* at, size_t mats) {
 // the factorisation of every matrix and the scaling of its block rows
 template <class R>
 static int factor_b64(tups_ctx* c, const ClosedArgs& a, unsigned mats) {
-  if (closed_regs(c))
-    hipLaunchKernelGGL((closed_factor_b64<R, kClosedRp>), dim3(mats), dim3(256), 0, c->stream, a);
-  else
-    hipLaunchKernelGGL((closed_factor_b64<R, 0>), dim3(mats), dim3(256), 0, c->stream, a);
-  TUPS_HIP(hipGetLastError());
   const unsigned nblk = (unsigned)closed_blocks(a.D);
+  const bool regs = closed_regs(c);
+  for (unsigned kb = 0; kb < nblk; ++kb) {
+    const int k0 = (int)kb * CL_BB, rows = a.D - k0;
+    // the register sub-panel with the rows a thread needs; it starts at most 256 kClosedRp rows
+    auto panel = !regs ? closed_panel<R, 0> : rows <= 256 ? closed_panel<R, 1> : closed_panel<R, kClosedRp>;
+    hipLaunchKernelGGL(panel, dim3(mats), dim3(256), 0, c->stream, a, k0);
+    TUPS_HIP(hipGetLastError());
+    hipLaunchKernelGGL(closed_diag<R>, dim3(mats), dim3(256), 0, c->stream, a, k0);
+    TUPS_HIP(hipGetLastError());
+    const unsigned left = nblk - kb - 1;
+    if (!left) break;
+    hipLaunchKernelGGL(closed_row<R>, dim3(left * mats), dim3(256), 0, c->stream, a, k0);
+    TUPS_HIP(hipGetLastError());
+    hipLaunchKernelGGL(closed_trail<R>, dim3(left * left * mats), dim3(256), 0, c->stream, a, k0);
+    TUPS_HIP(hipGetLastError());
+  }
   if (nblk > 1) hipLaunchKernelGGL(closed_scale<R>, dim3(nblk * (nblk - 1) * mats), dim3(256), 0, c->stream, a);
   TUPS_HIP(hipGetLastError());
   return TUPS_OK;
