@@ -20,17 +20,24 @@
 // fermionic frequencies times all Nl form factors, so a loader thread that owns
 // one (row, nu) pair of the A operand holds all Nl values that the Nl x Nl
 // block chi_nu couples and applies it in registers before the tile goes to LDS:
-//   part 0: A = Gamma alpha chi (:, S),  B = F(S, :)
-//   part 1: A = F alpha chi (:, S),      B = Gamma(S, :)
-// ((Gamma chi) F = Gamma (chi F) and F (chi Gamma) = (F chi) Gamma.)  The
-// frequency of an A pair is uniform across a wave, so chi_nu comes through the
-// scalar cache.  On gfx950 no VALU instruction issues while an F64 MFMA runs on
-// the SIMD, so the loop keeps VALU work minimal: -Im*Im uses the MFMA negate
-// modifier.  Operand tiles are stored as split Re/Im planes so each MFMA
-// operand is one double per lane.  Global loads of chunk c+1 are issued before
-// the MFMAs of chunk c (register prefetch), and the damped mixing is fused
-// into the epilogue.
+//   part 0: A = Gamma chi (:, S),  B = F(S, :)
+//   part 1: A = F chi (:, S),      B = Gamma(S, :)
+// ((Gamma chi) F = Gamma (chi F) and F (chi Gamma) = (F chi) Gamma; alpha c f
+// multiplies the sum at the end.)  The frequency of an A pair is uniform across
+// a wave, so chi_nu comes through the scalar cache.  On gfx950 no VALU
+// instruction issues while an F64 MFMA runs on the SIMD, so the loop keeps VALU
+// work minimal: -Im*Im uses the MFMA negate modifier, the mixing is four fused
+// multiply-adds per complex product, and the default tile (ladder_tile4) has no
+// address arithmetic and no masks in its loop.  The damped mixing is fused into
+// the epilogue.
+//
+// ladder_tile keeps the other forms that can be chosen: the three-product ones
+// (split Re/Im planes in LDS, so that each MFMA operand is one double per lane)
+// and the four-product ones with other chunks or two LDS buffers.
 #include "internal.h"
+#include "lds_dma.h"
+
+#include <type_traits>
 
 namespace tups {
 
@@ -45,8 +52,7 @@ struct BseArgs {
   double2* out[4];         // Phi_r (must not alias gam)
   const double2* chi[2];   // (Nl, Nl, Nf, nq): ph, pp
   int D, nf, nq, tiles_n;
-  double alpha;
-  double cf[4];            // c_r * f
+  double cf[4];            // c_r * f * alpha
   double omf;              // 1 - f
 };
 
@@ -75,7 +81,7 @@ constexpr int ladder_lds_doubles() {
 template <int NL, int G, bool DB, int K3 = 0>
 __device__ __forceinline__ void ladder_tile(const double2* __restrict__ Gm, const double2* __restrict__ Fm,
                                             double2* __restrict__ O, const double2* __restrict__ chiq, int D,
-                                            int nf, double alpha, double cf, double omf, int row0, int col0,
+                                            int nf, double cf, double omf, int row0, int col0,
                                             double* lds) {
   constexpr int KC = NL * G;   // inner-dimension chunk: G frequencies x NL form factors
   constexpr int PP = G / 4;    // (row|col, nu) pairs per thread: 64 * G / 256
@@ -156,17 +162,20 @@ __device__ __forceinline__ void ladder_tile(const double2* __restrict__ Gm, cons
           (const __attribute__((address_space(4))) double*)(chiq + (size_t)nu * NL * NL);
 #pragma unroll
       for (int l2 = 0; l2 < NL; ++l2) {
-        // (X alpha chi)(i, (l2, nu)) = alpha sum_l3 X(i, (l3, nu)) chi_nu(l3, l2)
+        // (X chi)(i, (l2, nu)) = sum_l3 X(i, (l3, nu)) chi_nu(l3, l2); alpha is in cf
         double sr = 0.0, si = 0.0;
 #pragma unroll
         for (int l3 = 0; l3 < NL; ++l3) {
           const double xr = cb[2 * (l3 + NL * l2)], xi = cb[2 * (l3 + NL * l2) + 1];
-          sr += ra[p][l3].x * xr - ra[p][l3].y * xi;
-          si += ra[p][l3].x * xi + ra[p][l3].y * xr;
+          // four fused multiply-adds (a sum of two products would take three per part)
+          sr = __builtin_fma(ra[p][l3].x, xr, sr);
+          si = __builtin_fma(ra[p][l3].x, xi, si);
+          sr = __builtin_fma(-ra[p][l3].y, xi, sr);
+          si = __builtin_fma(ra[p][l3].y, xr, si);
         }
-        As[sb][0][l2 * G + g][i] = alpha * sr;
-        As[sb][1][l2 * G + g][i] = alpha * si;
-        if (K3 == 1) As[sb][NPL - 1][l2 * G + g][i] = alpha * sr + alpha * si;
+        As[sb][0][l2 * G + g][i] = sr;
+        As[sb][1][l2 * G + g][i] = si;
+        if (K3 == 1) As[sb][NPL - 1][l2 * G + g][i] = sr + si;
       }
     }
 #pragma unroll
@@ -275,6 +284,229 @@ __device__ __forceinline__ void ladder_tile(const double2* __restrict__ Gm, cons
     }
 }
 
+// The default four-product tile, B fed by direct global-to-LDS loads.
+//
+// The chunk is G frequencies of all Nl form factors (Nl = 9: its k-steps in two passes of
+// 5 and 4 form factors out of one set of loaded rows), one k-step of 4 per form factor (Nl =
+// 1: per 4 frequencies).  B goes straight to LDS: the 4 x 16 block of one k-step and 16
+// columns is 1 KiB, one instruction of a wave, in the order in which a wave's fragment reads
+// it; its addresses are a lane offset fixed for the whole tile and a scalar base.  A's rows
+// are loaded at a scalar base and a fixed lane offset too and mixed in registers.  Rows and
+// columns beyond D repeat the last one (their results are not written), frequencies beyond
+// Nf are zeros.  One buffer per operand, 40 KiB at Nl = 5 and 9: four workgroups on a CU
+// (three at Nl = 9, by registers), whose MFMAs cover each other's loads and mixing; a wave
+// that loads and mixes, or works on a cut tile, goes before one that multiplies.
+//
+// Bound by the matrix cores' issue slots: at D = 320 MFMAs take 84 % of the cycles and the
+// mixing 9 %, at 2.3 GHz (the clock falls with the load).  Against the tile with both operands
+// through registers and masked loads (three, two at Nl = 9, workgroups to a CU): D = 320,
+// Nl = 5, 512 q 18.2 -> 16.5 ms; D = 288, Nl = 9, 512 q 20.0 -> 13.9; D = 198, Nl = 9, 256 q
+// 4.45 -> 3.16; D = 150, Nl = 5, 1024 q 6.23 -> 4.77; D = 64, Nl = 1, 2880 q 1.12 -> 0.99.
+template <int NL>
+struct LadderShape {
+  static constexpr int G = NL == 1 ? 16 : 4;     // frequencies per chunk
+  static constexpr int SUB = NL == 9 ? 2 : 1;    // passes per chunk
+  static constexpr int KS = NL == 1 ? 4 : 5;     // most k-steps in a pass
+  static constexpr int LDS = 2 * KS * 4 * 64 * (int)sizeof(double2);
+  static constexpr int PER_CU = NL == 9 ? 3 : 4;  // workgroups per CU that registers and LDS allow
+};
+
+template <int NL>
+__device__ __forceinline__ void ladder_tile4(const double2* __restrict__ Gm, const double2* __restrict__ Fm,
+                                             double2* __restrict__ O, const double2* __restrict__ chiq, int D,
+                                             int nf, double cf, double omf, int row0, int col0,
+                                             double2* lds) {
+  using S = LadderShape<NL>;
+  constexpr int PP = S::G / 4;
+  double2* As = lds;                    // [k][row]
+  double2* Bs = lds + S::KS * 4 * 64;   // [k-step][16-column block][column][k]
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int li = lane & 15, lk = lane >> 4;
+  const int rows = D - row0, cols = D - col0;
+  // A wave takes 2 x 2 blocks of 16 x 16.  In a tile cut to 32 columns (rows) or fewer it takes
+  // one row (column) of blocks, so that the four waves, one to a SIMD, still share the work.
+  const bool few_r = rows <= 32, few_c = cols <= 32;
+  const int wr = few_c ? 16 * (few_r ? wave >> 1 : wave) : few_r ? 0 : (wave >> 1) * 32;
+  const int wc = few_r ? 16 * (few_c ? wave & 1 : wave) : few_c ? 0 : (wave & 1) * 32;
+  const int ro[2] = {wr, min(wr + 16, 48)}, co[2] = {wc, min(wc + 16, 48)};
+  const unsigned offa = (unsigned)min(lane, rows - 1) * 16u;
+  const unsigned colb = (unsigned)min(16 * wave + (lane >> 2), cols - 1) * (unsigned)D;
+  const unsigned offb = (colb + (lane & 3)) * 16u;
+  const unsigned bbase = lds_addr(Bs) + wave * 1024;
+
+  d4 acc_re[2][2], acc_im[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc_re[i][j] = acc_im[i][j] = d4{0.0, 0.0, 0.0, 0.0};
+  bool blk_ok[2][2];  // this wave's blocks, those with a row and a column below D
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) blk_ok[i][j] = ro[i] < rows && co[j] < cols && !(i && few_c) && !(j && few_r);
+
+  const int nch = (nf + S::G - 1) / S::G;
+  double2 ra[PP][NL];
+  auto load = [&](int it) {
+    const int part = it >= nch ? 1 : 0;
+    const int nu0 = (it - part * nch) * S::G;
+    const double2* Asrc = (part ? Fm : Gm) + row0;
+#pragma unroll
+    for (int p = 0; p < PP; ++p) {
+      const int nu = min(nu0 + 4 * p + wave, nf - 1);
+#pragma unroll
+      for (int l = 0; l < NL; ++l)
+        ra[p][l] = *reinterpret_cast<const double2*>(
+            reinterpret_cast<const char*>(Asrc + (size_t)(l * nf + nu) * D) + offa);
+    }
+  };
+  // k-step s of the pass: form factor l0 + s (Nl = 1: frequencies nu0 + 4 s ..)
+  auto fetch_b = [&](int it, int l0, int n) {
+    const int part = it >= nch ? 1 : 0;
+    const int nu0 = (it - part * nch) * S::G;
+    const double2* Bsrc = (part ? Gm : Fm) + (size_t)col0 * D;
+#pragma unroll
+    for (int s = 0; s < S::KS; ++s) {
+      if (s >= n) break;
+      const int nu = NL == 1 ? nu0 + 4 * s : nu0;
+      const double2* src = Bsrc + (NL == 1 ? 0 : (l0 + s) * nf);
+      if (nu + 4 <= nf) {
+        dma16(src + nu, offb, bbase + s * 4096);
+      } else {
+        const int at = min(nu, nf - 1);
+        dma16(src + at, (colb + min(lane & 3, nf - 1 - at)) * 16u, bbase + s * 4096);
+      }
+    }
+  };
+  auto zero_b = [&](int it, int n) {  // this wave's own blocks, after its loads have landed
+    const int part = it >= nch ? 1 : 0;
+    const int nu0 = (it - part * nch) * S::G;
+    if (nu0 + S::G <= nf) return;
+    for (int s = 0; s < n; ++s)
+      if ((NL == 1 ? nu0 + 4 * s : nu0) + (lane & 3) >= nf)
+        Bs[(s * 4 + wave) * 64 + lane] = make_double2(0.0, 0.0);
+  };
+  // (X chi)(i, (l2, nu)) = sum_l3 X(i, (l3, nu)) chi_nu(l3, l2) for l2 = l0 .. l0 + n - 1; alpha is in cf
+  auto mix = [&](int it, auto l0c, auto nc) {
+    constexpr int l0 = decltype(l0c)::value, n = decltype(nc)::value;
+    const int part = it >= nch ? 1 : 0;
+    const int nu0 = (it - part * nch) * S::G;
+#pragma unroll
+    for (int p = 0; p < PP; ++p) {
+      const int g = 4 * p + wave;
+      const bool in = nu0 + g < nf;
+      const __attribute__((address_space(4))) double* cb =
+          (const __attribute__((address_space(4))) double*)(chiq + (size_t)min(nu0 + g, nf - 1) * NL * NL);
+#pragma unroll
+      for (int s = 0; s < n; ++s) {
+        double sr = 0.0, si = 0.0;
+        if (in) {
+#pragma unroll
+          for (int l3 = 0; l3 < NL; ++l3) {
+            // four fused multiply-adds (a sum of two products would take three per part)
+            const double xr = cb[2 * (l3 + NL * (l0 + s))], xi = cb[2 * (l3 + NL * (l0 + s)) + 1];
+            sr = __builtin_fma(ra[p][l3].x, xr, sr);
+            si = __builtin_fma(ra[p][l3].x, xi, si);
+            sr = __builtin_fma(-ra[p][l3].y, xi, sr);
+            si = __builtin_fma(ra[p][l3].y, xr, si);
+          }
+        }
+        As[(NL == 1 ? g : s * 4 + wave) * 64 + lane] = make_double2(sr, si);
+      }
+    }
+  };
+  auto mfma_pass = [&](int n) {
+#pragma unroll
+    for (int s = 0; s < S::KS; ++s) {
+      if (s >= n) break;
+      double2 fa[2], fb[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        fa[i] = As[(s * 4 + lk) * 64 + ro[i] + li];
+        fb[i] = Bs[(s * 4 + co[i] / 16) * 64 + li * 4 + lk];
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          if (!blk_ok[i][j]) continue;
+          acc_re[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[i].x, fb[j].x, acc_re[i][j], 0, 0, 0);
+          acc_im[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[i].x, fb[j].y, acc_im[i][j], 0, 0, 0);
+          // blgp bit 0 negates the A operand of an F64 MFMA: acc -= Im(A) Im(B)
+          acc_re[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[i].y, fb[j].y, acc_re[i][j], 0, 0, 1);
+          acc_im[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[i].y, fb[j].x, acc_im[i][j], 0, 0, 0);
+        }
+    }
+  };
+  constexpr std::integral_constant<int, 0> first{};
+  constexpr std::integral_constant<int, S::KS> split{};
+  load(0);
+  for (int it = 0; it < 2 * nch; ++it) {
+    wait_vmcnt<0>();  // the rows of this chunk (before the loads to LDS are in flight)
+    __builtin_amdgcn_s_setprio(1);
+    fetch_b(it, 0, S::KS);
+    mix(it, first, std::integral_constant<int, NL == 1 ? 1 : S::KS>{});
+    wait_vmcnt<0>();
+    zero_b(it, S::KS);
+    __syncthreads();
+    if (S::SUB == 1 && it + 1 < 2 * nch) load(it + 1);
+    if (!few_r && !few_c) __builtin_amdgcn_s_setprio(0);
+    mfma_pass(S::KS);
+    __syncthreads();
+    if constexpr (S::SUB == 2) {
+      __builtin_amdgcn_s_setprio(1);
+      fetch_b(it, S::KS, NL - S::KS);
+      mix(it, split, std::integral_constant<int, NL - S::KS>{});
+      wait_vmcnt<0>();
+      zero_b(it, NL - S::KS);
+      __syncthreads();
+      if (it + 1 < 2 * nch) load(it + 1);
+      if (!few_r && !few_c) __builtin_amdgcn_s_setprio(0);
+      mfma_pass(NL - S::KS);
+      __syncthreads();
+    }
+  }
+
+  // Phi = c f T + (1 - f)(F - Gamma).  v_mfma_f64_16x16x4f64 leaves element e of lane l at
+  // block row (l / 16) + 4 e, column l % 16.
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      if (!blk_ok[i][j]) continue;
+      const int gj = col0 + co[j] + li;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int gi = row0 + ro[i] + lk + 4 * e;
+        if (gi < D && gj < D) {
+          const size_t idx = (size_t)gj * D + gi;
+          const double2 f = Fm[idx];
+          const double2 g = Gm[idx];
+          O[idx] = make_double2(cf * acc_re[i][j][e] + omf * (f.x - g.x), cf * acc_im[i][j][e] + omf * (f.y - g.y));
+        }
+      }
+    }
+}
+
+template <int NL>
+__global__ __launch_bounds__(256, LadderShape<NL>::PER_CU) void bse_ladder4_kernel(BseArgs a) {
+  __shared__ __attribute__((aligned(16))) double2 lds[LadderShape<NL>::LDS / sizeof(double2)];
+  const int tiles = a.tiles_n * a.tiles_n;
+  const int logical = xcd_remap(blockIdx.x, gridDim.x);
+  const int mat = logical / tiles;
+  // Each matrix starts its tiles at another place: an XCD hands its workgroups to its 32 CUs in
+  // turn, and with 16 tiles to a matrix the cut ones (few MFMAs) would meet on the same CUs
+  // (D = 208, Nl = 1: 10.1 -> 8.8 ms at 947 q).
+  const int t = (logical - mat * tiles + (a.tiles_n + 1) * mat) % tiles;
+  const int tr = t / a.tiles_n, tc = t - tr * a.tiles_n;
+  const int r = mat / a.nq;
+  const int q = mat - r * a.nq;
+  const size_t DD = (size_t)a.D * a.D;
+  ladder_tile4<NL>(a.gam[r] + DD * q, a.fv[r] + DD * q, a.out[r] + DD * q, a.chi[r >> 1] + (size_t)a.nf * NL * NL * q,
+                   a.D, a.nf, a.cf[r], a.omf, tr * BM, tc * BN, lds);
+}
+
 template <int NL, int G, bool DB, int K3 = 0>
 __global__ __launch_bounds__(256, 2) void bse_ladder_kernel(BseArgs a) {
   __shared__ double lds[ladder_lds_doubles<NL, G, DB, K3>()];
@@ -282,12 +514,12 @@ __global__ __launch_bounds__(256, 2) void bse_ladder_kernel(BseArgs a) {
   const int logical = xcd_remap(blockIdx.x, gridDim.x);
   const int mat = logical / tiles;
   const int t = logical - mat * tiles;
+  const int tr = t / a.tiles_n, tc = t - tr * a.tiles_n;
   const int r = mat / a.nq;
   const int q = mat - r * a.nq;
   const size_t DD = (size_t)a.D * a.D;
   ladder_tile<NL, G, DB, K3>(a.gam[r] + DD * q, a.fv[r] + DD * q, a.out[r] + DD * q,
-                             a.chi[r >> 1] + (size_t)a.nf * NL * NL * q, a.D, a.nf, a.alpha, a.cf[r], a.omf,
-                             (t / a.tiles_n) * BM, (t % a.tiles_n) * BN, lds);
+                             a.chi[r >> 1] + (size_t)a.nf * NL * NL * q, a.D, a.nf, a.cf[r], a.omf, tr * BM, tc * BN, lds);
 }
 
 typedef void (*BseKernel)(BseArgs);
@@ -304,13 +536,13 @@ struct BseVariant {
 
 // tile variants per form-factor count: frequency chunk G and LDS double buffering
 static const BseVariant kBseVariants[] = {
-    {1, bse_ladder_kernel<1, 16, false>, "nl1_g16"},
+    {1, bse_ladder4_kernel<1>, "nl1_g16"},
     {1, bse_ladder_kernel<1, 16, true>, "nl1_g16_db"},
     {1, bse_ladder_kernel<1, 32, false>, "nl1_g32"},
-    {5, bse_ladder_kernel<5, 4, false>, "nl5_g4"},
+    {5, bse_ladder4_kernel<5>, "nl5_g4"},
     {5, bse_ladder_kernel<5, 4, true>, "nl5_g4_db"},
     {5, bse_ladder_kernel<5, 8, false>, "nl5_g8"},
-    {9, bse_ladder_kernel<9, 4, false>, "nl9_g4"},
+    {9, bse_ladder4_kernel<9>, "nl9_g4"},
     {9, bse_ladder_kernel<9, 4, true>, "nl9_g4_db"},
     {1, bse_ladder_kernel<1, 16, false, true>, "nl1_g16_3m"},
     {5, bse_ladder_kernel<5, 4, false, true>, "nl5_g4_3m"},
@@ -342,9 +574,8 @@ static BseArgs bse_args(tups_ctx* c) {
   a.nf = s.nf;
   a.nq = s.nq;
   a.tiles_n = (s.nz + BM - 1) / BM;
-  a.alpha = s.alpha;
   const double cr[4] = {0.5, 0.5, -0.25, 0.25};
-  for (int r = 0; r < 4; ++r) a.cf[r] = cr[r] * c->f_damping;
+  for (int r = 0; r < 4; ++r) a.cf[r] = cr[r] * c->f_damping * s.alpha;
   a.omf = 1.0 - c->f_damping;
   return a;
 }
@@ -434,25 +665,39 @@ struct BatchArgs {
   int* tickets;             // per-list counters of the dynamic order (zero at launch)
   int len;                  // entries per list
   int dyn;                  // 1: entries handed out by the per-list counters
-  double alpha;
   double cf[4];
   double omf;
 };
 }  // namespace
 
+// the ladder tile of NL form factors: four products, or the three-product form K
+template <int NL, int K>
+constexpr int batch_tile_doubles() {
+  return K ? ladder_lds_doubles<NL, LadderShape<NL>::G, false, K>() : LadderShape<NL>::LDS / 8;
+}
+template <int NL, int K>
+__device__ __forceinline__ void batch_tile(const double2* g, const double2* f, double2* o, const double2* chiq, int nf,
+                                           double cf, double omf, int row0, int col0, double* lds) {
+  if constexpr (K)
+    ladder_tile<NL, LadderShape<NL>::G, false, K>(g, f, o, chiq, NL * nf, nf, cf, omf, row0, col0, lds);
+  else
+    ladder_tile4<NL>(g, f, o, chiq, NL * nf, nf, cf, omf, row0, col0, reinterpret_cast<double2*>(lds));
+}
+
 template <int K1, int K5, int K9>
 constexpr int batch_lds_doubles() {
-  constexpr int a = ladder_lds_doubles<1, 16, false, K1>();
-  constexpr int b = ladder_lds_doubles<5, 4, false, K5>();
-  constexpr int c = ladder_lds_doubles<9, 4, false, K9>();
+  constexpr int a = batch_tile_doubles<1, K1>();
+  constexpr int b = batch_tile_doubles<5, K5>();
+  constexpr int c = batch_tile_doubles<9, K9>();
   return a > b ? (a > c ? a : c) : (b > c ? b : c);
 }
 
-// workgroups per CU that the LDS footprint allows (160 KB per CU); the register
-// budget follows: 256 VGPRs per lane at two, the full 512 (AGPRs included) at one
+// workgroups per CU: with four products throughout those of the uniform path, else what
+// the LDS footprint allows (160 KB per CU); the register budget follows: 256 VGPRs per
+// lane at two, the full 512 (AGPRs included) at one
 template <int K1, int K5, int K9>
 constexpr int batch_occupancy() {
-  return 8 * batch_lds_doubles<K1, K5, K9>() <= 80 * 1024 ? 2 : 1;
+  return !K1 && !K5 && !K9 ? LadderShape<9>::PER_CU : 8 * batch_lds_doubles<K1, K5, K9>() <= 80 * 1024 ? 2 : 1;
 }
 
 __device__ __forceinline__ long long uniform64(long long v) {
@@ -472,7 +717,7 @@ __device__ __forceinline__ long long uniform64(long long v) {
 // multiple of 8.  K1, K5, K9: the complex-product form per form-factor count.
 template <int K1, int K5, int K9>
 __global__ __launch_bounds__(256, (batch_occupancy<K1, K5, K9>())) void bse_batch_kernel(BatchArgs a) {
-  extern __shared__ double lds[];
+  extern __shared__ __attribute__((aligned(16))) double lds[];
   __shared__ int ticket;
   const int x = blockIdx.x & 7, j = blockIdx.x >> 3;
   const int first = x * a.len + j;
@@ -504,11 +749,11 @@ __global__ __launch_bounds__(256, (batch_occupancy<K1, K5, K9>())) void bse_batc
     double2* o = a.out[r] + vo;
     const double2* ch = a.chi[r >> 1] + co;
     if (nl == 1)
-      ladder_tile<1, 16, false, K1>(g, f, o, ch, nf, nf, a.alpha, a.cf[r], a.omf, w.z, w.w, lds);
+      batch_tile<1, K1>(g, f, o, ch, nf, a.cf[r], a.omf, w.z, w.w, lds);
     else if (nl == 5)
-      ladder_tile<5, 4, false, K5>(g, f, o, ch, 5 * nf, nf, a.alpha, a.cf[r], a.omf, w.z, w.w, lds);
+      batch_tile<5, K5>(g, f, o, ch, nf, a.cf[r], a.omf, w.z, w.w, lds);
     else
-      ladder_tile<9, 4, false, K9>(g, f, o, ch, 9 * nf, nf, a.alpha, a.cf[r], a.omf, w.z, w.w, lds);
+      batch_tile<9, K9>(g, f, o, ch, nf, a.cf[r], a.omf, w.z, w.w, lds);
     __syncthreads();  // the next item reuses the LDS buffer
   }
 }
@@ -610,14 +855,18 @@ extern "C" int tups_batch_create(int32_t nx, int32_t nq, const int32_t* nf, cons
   std::stable_sort(order.begin(), order.end(),
                    [&](int x, int y) { return nl[x] * nf[x] > nl[y] * nf[y]; });
   std::vector<int4> lists[8];
-  long long load[8] = {};
+  long long load[8] = {}, mats[8] = {};
   long long total = 0;
   for (int q : order) {
     const int D = nl[q] * nf[q], tn = (D + BM - 1) / BM;
     for (int r = 0; r < 4; ++r) {
       const int x = (int)(std::min_element(load, load + 8) - load);
       load[x] += (long long)tn * tn * D;
-      for (int t = 0; t < tn * tn; ++t) lists[x].push_back(make_int4(q, r, (t / tn) * BM, (t % tn) * BN));
+      for (int i = 0; i < tn * tn; ++i) {  // each matrix of a list starts its tiles at another place
+        const int t = (int)((i + (long long)(tn + 1) * mats[x]) % (tn * tn));
+        lists[x].push_back(make_int4(q, r, (t / tn) * BM, (t % tn) * BN));
+      }
+      ++mats[x];
       total += tn * tn;
     }
   }
@@ -739,9 +988,8 @@ static BatchArgs batch_args(const tups_batch* b, int dyn) {
   a.tickets = b->d_tickets;
   a.len = b->len;
   a.dyn = dyn;
-  a.alpha = b->alpha;
   const double cr[4] = {0.5, 0.5, -0.25, 0.25};
-  for (int r = 0; r < 4; ++r) a.cf[r] = cr[r] * b->f_damping;
+  for (int r = 0; r < 4; ++r) a.cf[r] = cr[r] * b->f_damping * b->alpha;
   a.omf = 1.0 - b->f_damping;
   return a;
 }
