@@ -885,6 +885,16 @@ extern "C" int tups_batch_create(int32_t nx, int32_t nq, const int32_t* nf, cons
   }
   b->nitems = (int)total;
   b->len = (int)len;
+  // More entries than resident workgroups: drawn from the counters (512 q of Nf = 16 .. 64, Nl = 1, 5 and 9: 15.0 ms,
+  // in static turns 18.1, one workgroup per entry 15.2); else every workgroup has its entry.
+  int dev = 0, ncu = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
+    delete b;
+    set_error("no device for the batch");
+    return TUPS_EHIP;
+  }
+  b->variant = 8 * (long long)len > (long long)kBatchKernels[0].per_cu * ncu ? 2 : 0;
   auto fail = [&](int rc) {
     tups_batch_destroy(b);
     return rc;

@@ -321,7 +321,7 @@ struct tups_batch {
   int* d_tickets = nullptr;
   int nitems = 0;  // work items (tiles)
   int len = 0;     // entries per XCD list, padding included
-  int variant = 0;
+  int variant = 0;  // set at creation by the number of items, then by the autotuner
   bool three_mult = false;            // the autotuner may pick the three-multiplication product forms
   // split form (tups_batch_bse_split): q grouped by (Nf, Nl) class, largest D first
   std::vector<int> qlist;             // q of class 0, then class 1, ...
