@@ -238,11 +238,15 @@ __global__ __launch_bounds__(256) void crt_prep_a(CrtArgs a) {
 // on the bits of the non-negative doubles, which order as unsigned integers),
 // then lane l converts inner indices 4 l + 256 n .. + 3 and stores one dword
 // per (modulus, sign).  At the end the row maxima are the block's partial
-// rmaxp[mat][blockIdx.x][row].  grid: (Dp / 16, 4 * nqb); dynamic LDS
-// 4 Kp 16 + Dp 8 (+ nl^2 nf 16 with CL).
+// rmaxp[mat][blockIdx.x][row].  With HALF (nf <= 32) the lower half of a wave
+// mixes F and the upper Gamma.  The columns beyond D are left out: they meet
+// only results that are not written.  grid: (Dp / 16, 4 * nqb); dynamic LDS
+// 4 Kp 16 + Dp 8 (+ nl^2 nf 16 with CL).  Bound by the vector instructions of
+// the residues and, at two workgroups to a CU (LDS), their latencies: D = 198
+// (Dp = 256), Nl = 9, 110 q 785 -> 641 us; D = 320 988 us per 102 q, about as before.
 constexpr int PREP_B_CPW = PREP_B_COLS / 4;
-template <int NL, bool CL>
-__global__ __launch_bounds__(256) void crt_prep_b(CrtArgs a) {
+template <int NL, bool CL, bool HALF>
+__global__ __launch_bounds__(256, 2) void crt_prep_b(CrtArgs a) {
   extern __shared__ double2 colv[];  // [4][Kp] mixed columns, [Dp] row maxima (bits), with CL [l1][l3][nu]
   const int mat = blockIdx.y;
   int r;
@@ -265,50 +269,51 @@ __global__ __launch_bounds__(256) void crt_prep_b(CrtArgs a) {
   double2* v = colv + (size_t)wave * Kp;
   const double2* Fq = a.fv[r] + vo;
   const double2* Gq = a.gam[r] + vo;
-  // loads from a clamped address, unconditionally (the caller zeroes what lies
-  // outside), so the registers are written by the loads alone
-  auto load_x = [&](int col, int nu, double2 (&xf)[NL], double2 (&xg)[NL]) {
+  const int hl = HALF ? lane & 31 : lane;  // this lane's place in the frequencies
+  const bool second = HALF && lane >= 32;  // its matrix with HALF: F, or Gamma in the upper half
+  const double2* Xq = second ? Gq : Fq;
+  // loads from a clamped address, unconditionally, so the registers are written by the loads alone
+  auto load_x = [&](int col, int nu, double2 (&xf)[NL], double2 (&xg)[HALF ? 1 : NL]) {
     const size_t o = (size_t)(col < D ? col : 0) * D + (nu < nf ? nu : 0);
 #pragma unroll
     for (int l3 = 0; l3 < NL; ++l3) {
-      xf[l3] = Fq[o + l3 * nf];
-      xg[l3] = Gq[o + l3 * nf];
+      xf[l3] = Xq[o + l3 * nf];
+      if constexpr (!HALF) xg[l3] = Gq[o + l3 * nf];
     }
   };
   const int col0 = blockIdx.x * PREP_B_COLS + wave * PREP_B_CPW;
   // the first 64 nu of the next column are loaded before the current column's
   // conversion, so their latency hides behind it
-  double2 pf[NL], pg[NL];
-  load_x(col0, lane, pf, pg);
+  double2 pf[NL], pg[HALF ? 1 : NL];
+  load_x(col0, hl, pf, pg);
   int fkeep = 0;  // lane cc keeps column cc's exponent; stored after the loop, so no store in it
                   // holds back the prefetch (a store's data register is waited for before reuse)
-  for (int cc = 0; cc < PREP_B_CPW; ++cc) {
+  const int ncc = min(PREP_B_CPW, D - col0);
+#pragma unroll 1
+  for (int cc = 0; cc < ncc; ++cc) {  // the columns beyond D meet only results that are not written
     const int col = col0 + cc;
     // B((part, l1, nu), col) = alpha sum_l3 chi_nu(l1, l3) X((l3, nu), col), X = F (part 0), Gamma (part 1)
     double mx = 0.0;
     for (int nu0 = 0; nu0 < nf; nu0 += 64) {
-      const int nu = nu0 + lane;
-      double2 xf[NL], xg[NL];
-      if (nu0 == 0) {
+      const int nu = nu0 + hl;
+      double2 xf[NL], xg[HALF ? 1 : NL];
+      if (HALF || nu0 == 0) {
 #pragma unroll
         for (int l3 = 0; l3 < NL; ++l3) {
           xf[l3] = pf[l3];
-          xg[l3] = pg[l3];
+          if constexpr (!HALF) xg[l3] = pg[l3];
         }
       } else {
         load_x(col, nu, xf, xg);
       }
       if (nu >= nf) continue;
-      if (col >= D) {
-#pragma unroll
-        for (int l3 = 0; l3 < NL; ++l3) xf[l3] = xg[l3] = make_double2(0.0, 0.0);
-      }
 #pragma unroll
       for (int l3 = 0; l3 < NL; ++l3) {
-        const double am = fmax(fmax(fabs(xf[l3].x), fabs(xf[l3].y)), fmax(fabs(xg[l3].x), fabs(xg[l3].y)));
+        double am = fmax(fabs(xf[l3].x), fabs(xf[l3].y));
+        if constexpr (!HALF) am = fmax(am, fmax(fabs(xg[l3].x), fabs(xg[l3].y)));
         atomicMax(&rmx[l3 * nf + nu], (unsigned long long)__double_as_longlong(am));
       }
-#pragma unroll
+#pragma unroll 1
       for (int l1 = 0; l1 < NL; ++l1) {
         double fr = 0.0, fi = 0.0, gr = 0.0, gi = 0.0;
 #pragma unroll
@@ -316,14 +321,19 @@ __global__ __launch_bounds__(256) void crt_prep_b(CrtArgs a) {
           const double2 c = CL ? chil[(size_t)(l1 + nl * l3) * nf + nu] : chig[(size_t)nu * nl * nl + l1 + nl * l3];
           fr = fma(c.x, xf[l3].x, fma(-c.y, xf[l3].y, fr));
           fi = fma(c.x, xf[l3].y, fma(c.y, xf[l3].x, fi));
-          gr = fma(c.x, xg[l3].x, fma(-c.y, xg[l3].y, gr));
-          gi = fma(c.x, xg[l3].y, fma(c.y, xg[l3].x, gi));
+          if constexpr (!HALF) {
+            gr = fma(c.x, xg[l3].x, fma(-c.y, xg[l3].y, gr));
+            gi = fma(c.x, xg[l3].y, fma(c.y, xg[l3].x, gi));
+          }
         }
         const double2 mf = make_double2(a.alpha * fr, a.alpha * fi);
-        const double2 mg = make_double2(a.alpha * gr, a.alpha * gi);
-        v[l1 * nf + nu] = mf;
-        v[D + l1 * nf + nu] = mg;
-        mx = fmax(mx, fmax(fmax(fabs(mf.x), fabs(mf.y)), fmax(fabs(mg.x), fabs(mg.y))));
+        v[(second ? D : 0) + l1 * nf + nu] = mf;
+        mx = fmax(mx, fmax(fabs(mf.x), fabs(mf.y)));
+        if constexpr (!HALF) {
+          const double2 mg = make_double2(a.alpha * gr, a.alpha * gi);
+          v[D + l1 * nf + nu] = mg;
+          mx = fmax(mx, fmax(fabs(mg.x), fabs(mg.y)));
+        }
       }
     }
     for (int k = 2 * D + lane; k < Kp; k += 64) v[k] = make_double2(0.0, 0.0);
@@ -331,7 +341,7 @@ __global__ __launch_bounds__(256) void crt_prep_b(CrtArgs a) {
     int f = 0;
     if (mx > 0.0) frexp(mx, &f);
     const double sc = ldexp(1.0, a.tb - f);
-    if (cc + 1 < PREP_B_CPW) load_x(col + 1, lane, pf, pg);
+    if (cc + 1 < PREP_B_CPW) load_x(col + 1, hl, pf, pg);
     // the wave's column in LDS is complete (each wave reads only its own; the
     // LDS executes one wave's accesses in order, so only the compiler needs
     // holding back)
@@ -1022,9 +1032,16 @@ static void (*prep_b_kernel(int nl, size_t Kp, size_t Dp, int nf, size_t* lds))(
   const size_t cols = 4 * Kp * sizeof(double2) + Dp * sizeof(double), chi = (size_t)nl * nl * nf * sizeof(double2);
   const bool cl = cols + chi <= 160 * 1024;
   *lds = cols + (cl ? chi : 0);
-  if (nl == 1) return cl ? crt_prep_b<1, true> : crt_prep_b<1, false>;
-  if (nl == 5) return cl ? crt_prep_b<5, true> : crt_prep_b<5, false>;
-  return cl ? crt_prep_b<9, true> : crt_prep_b<9, false>;
+  // up to 32 frequencies the halves of a wave mix F and Gamma side by side (D = 198, Nl = 9,
+  // 110 q: 641 us against 743 with the lanes along nu alone)
+  if (nf <= 32) {
+    if (nl == 1) return cl ? crt_prep_b<1, true, true> : crt_prep_b<1, false, true>;
+    if (nl == 5) return cl ? crt_prep_b<5, true, true> : crt_prep_b<5, false, true>;
+    return cl ? crt_prep_b<9, true, true> : crt_prep_b<9, false, true>;
+  }
+  if (nl == 1) return cl ? crt_prep_b<1, true, false> : crt_prep_b<1, false, false>;
+  if (nl == 5) return cl ? crt_prep_b<5, true, false> : crt_prep_b<5, false, false>;
+  return cl ? crt_prep_b<9, true, false> : crt_prep_b<9, false, false>;
 }
 
 // workspace bytes of one matrix: residues of A and B, exponents, row maxima and
