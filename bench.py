@@ -434,7 +434,7 @@ def main():
     roof64 = {"bound": "mfma", "achieved": round(achieved, 3), "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
               "frac": round(achieved / FP64_PEAK_TFLOPS, 4),
               "traffic": profile_traffic("bse_ladder_fp64_D320_nq1024.md"),
-              "kernel": f"bse_ladder_kernel variant {variant}", "avg_launch_ms": round(lad_ms / lad_n, 4),
+              "kernel": f"BSE ladder tile {variant}", "avg_launch_ms": round(lad_ms / lad_n, 4),
               "flops_per_launch": flops_per_launch}
 
     # --- split form ----------------------------------------------------------------------
@@ -462,7 +462,7 @@ def main():
                 "kernel": f"split GEMM {svar} ({args.moduli} moduli)", "avg_launch_ms": round(gemm_ms / gemm_n, 4),
                 "ops_per_launch": ops_per_launch, "prep_ms_per_launch": round(prep_ms / prep_n, 4),
                 "launches_per_step": gemm_n // nprof}
-    # --- closed form (fixed point by pivoted Gauss-Jordan) --------------------------------
+    # --- closed form (fixed point by pivoted LU) ------------------------------------------
     batched_bse_inputs(ctx, U=U, seed=0)
     ctx.BSE(0, mode=BSE_CLOSED_LU)  # warm-up (allocates its workspace)
     ctx.sync()
@@ -473,13 +473,13 @@ def main():
     cl_ms, cl_n = ctx.kernel_time(K_BSE_CLOSED)
     ctx.set_timing(False)
     cl_step_ms = cl_ms / ncl
-    cl_flops = 12.0 * D ** 3 * 4 * nq  # Gauss-Jordan on D right-hand sides, 4 channels
+    cl_flops = (8.0 / 3.0 + 8.0) * D ** 3 * 4 * nq  # LU and D right-hand sides, 4 channels
     closed = {"value": round(nq / (cl_step_ms / 1e3), 2), "unit": "q-points/s", "ms_per_call": round(cl_step_ms, 3),
               "achieved": round(cl_flops / (cl_step_ms / 1e3) / 1e12, 3), "peak": FP64_PEAK_TFLOPS,
               "unit_roofline": "TFLOP/s", "frac": round(cl_flops / (cl_step_ms / 1e3) / 1e12 / FP64_PEAK_TFLOPS, 4),
-              "flops_per_call": cl_flops, "kernel": "closed_build_nu + closed_solve_b64 (64-column block Gauss-Jordan, register sub-panels)"}
+              "flops_per_call": cl_flops, "kernel": "closed_build_nu + closed_panel/diag/row/trail/scale (64-column block LU) + closed_lu_solve"}
     print(f"[bench] closed form: {cl_step_ms:.1f} ms per call", file=sys.stderr, flush=True)
-    # --- closed form by FP32 LU (Gauss-Jordan inverse) + FP64 iterative refinement -------
+    # --- closed form by FP32 LU + FP64 iterative refinement -------------------------------
     batched_bse_inputs(ctx, U=U, seed=0)
     ctx.BSE(0, mode=BSE_CLOSED_IR)  # warm-up (allocates its workspace)
     ctx.sync()
@@ -493,10 +493,10 @@ def main():
     refined = {"value": round(nq / (ir_step_ms / 1e3), 2), "unit": "q-points/s", "ms_per_call": round(ir_step_ms, 3),
                "refinement_steps": ir_steps, "residual": ir_res, "residual_bar": 1e-12,
                "vs_direct_fp64": round(cl_step_ms / ir_step_ms, 3),
-               "kernel": "closed_build_nu<float2> + closed_solve_b64<float> (FP32 MFMA) + ir_gemm (FP32 / FP64 MFMA) + ir_chi "
-                         "+ ir_check",
-               "flops_per_call": {"fp32": (12.0 + 8.0 * (1 + ir_steps)) * D ** 3 * 4 * nq,
-                                  "fp64": 8.0 * (ir_steps + 1) * D ** 3 * 4 * nq}}
+               "kernel": "closed_build_nu<float2> + closed_panel/diag/row/trail/scale<float> + closed_lu_solve (FP32 MFMA) "
+                         "+ ir_gemm (FP64 MFMA) + ir_check",
+               "flops_per_call": {"fp32": (8.0 / 3.0 + 8.0 * (1 + ir_steps)) * D ** 3 * 4 * nq,
+                                  "fp64": 8.0 * ir_steps * D ** 3 * 4 * nq}}
     print(f"[bench] refined closed form: {ir_step_ms:.1f} ms per call, {ir_steps} steps, residual {ir_res:.1e}",
           file=sys.stderr, flush=True)
     # --- convergence check: max |F_r| over the four resident vertices (HBM read) -----------
@@ -588,7 +588,7 @@ def main():
                  "avg_launch_ms": round(p5_ms / p5_n, 3), "flops_per_call": fl5,
                  "traffic": profile_traffic("crossing_pae_nl5_nx8_nf64.md"),
                  "bytes_per_call": crossing_bytes(c5),
-                 "kernel": "pae_ybuild + pae_mm (FP64 MFMA GEMM per bosonic frequency)",
+                 "kernel": "pae_ybuild + pae_sparse (products over the nonzero elements of M, per bosonic frequency)",
                  "workload": f"calculate_PAE Nx=8 Nf=64 Nl=5 NR={c5.nr}, Nq={c5.nq} (all IBZ q), 4 channels"}
     print(f"[bench] crossing Nl=5: {p5_ms / p5_n:.2f} ms per call", file=sys.stderr, flush=True)
     phir5 = phir_leg(c5)
@@ -684,7 +684,7 @@ def main():
     vbytes = 4.0 * sc.nz * sc.nz * sc.nq * 16
     sde = {"ms_per_call": round(sde_ms / sde_n, 3), "vertex_bytes": vbytes,
            "vertex_read_gbs": round(vbytes / (sde_ms / sde_n / 1e3) / 1e9, 1),
-           "kernel": "sde_chi_aux + sde_vchi + sde_sigma (FP64)",
+           "kernel": "green_table + bubble_kernel + sde_vchi + sde_sigma (FP64)",
            "workload": f"calc_SDE without use_U2, Nx=8 Nf=64 Nl=5, Nq={sc.nq} (all IBZ q), f_range=0"}
     print(f"[bench] sde: {sde_ms / sde_n:.2f} ms per call", file=sys.stderr, flush=True)
     # calc_sus on the same context (F and Phi resident, Sigma = 0 on the device)
@@ -698,7 +698,7 @@ def main():
     sc.set_timing(False)
     nent = sc.nz
     sus_flops = 4.0 * sc.nq * nent * nent * 4 * 8  # 4 channels x Nq x D^2 entries x 4 form factors, complex MAC
-    sus = {"ms_per_call": round(sus_ms / sus_n, 3), "kernel": "sus_gg + sus_contract (FP64)",
+    sus = {"ms_per_call": round(sus_ms / sus_n, 3), "kernel": "green_table + bubble_kernel + sus_contract (FP64)",
            "fp64_tflops": round(sus_flops / (sus_ms / sus_n / 1e3) / 1e12, 2),
            "workload": f"calc_sus, Nx=8 Nf=64 Nl=5, Nq={sc.nq}, f_range=0, 4 external form factors"}
     print(f"[bench] sus: {sus_ms / sus_n:.2f} ms per call", file=sys.stderr, flush=True)

@@ -73,13 +73,14 @@ extern "C" {
                                    residues modulo Gaussian moduli, recombined in FP64 */
 #define TUPS_BSE_CLOSED_LU 2    /* closed form: the ladder's fixed point for fixed Gamma,
                                    Phi = (I - kappa_r Gamma chi)^-1 Gamma - Gamma, kappa_r =
-                                   2 c_r alpha, by pivoted Gauss-Jordan (FP64 MFMA updates);
+                                   2 c_r alpha, by pivoted LU (FP64 MFMA products);
                                    returns TUPS_ENONFINITE on a zero pivot column */
-#define TUPS_BSE_CLOSED_IR 3    /* the same closed form by FP32 LU (pivoted Gauss-Jordan on
-                                   [fp32(A) | I], FP32 MFMA) and FP64 iterative refinement
-                                   X += A32^-1 (Gamma - A X) until |R|_F / |Gamma|_F <= the
-                                   tolerance of tups_set_refinement (default 1e-12, at most
-                                   10 steps; TUPS_ENOCONV otherwise) */
+#define TUPS_BSE_CLOSED_IR 3    /* the same closed form by FP32 LU (pivoted, of fp32(A), FP32
+                                   MFMA) and FP64 iterative refinement X += A32^-1 (Gamma - A X)
+                                   until |R|_F / |Gamma|_F <= the tolerance of
+                                   tups_set_refinement (default 1e-12, at most 10 steps;
+                                   TUPS_ENOCONV otherwise); the residual that meets it gives
+                                   one last step while steps are left */
 
 typedef struct tups_dims {
   int32_t nx;        /* Nx = Ny (even), SRC/parquet_ini.f90:304-305 */
@@ -159,10 +160,12 @@ int tups_upload_chi_dense(tups_ctx* ctx, int32_t pp, int32_t q0, int32_t nqs,
 /* BSE(ite): Gamma_r <- Phi_r for r = d,m,s,t; SRC/parquet_BSE.f90:62-132 */
 int tups_bse(tups_ctx* ctx, int32_t mode);
 /* TUPS_BSE_CLOSED_IR: refine until |Gamma - A X|_F / |Gamma|_F <= tol for every
- * (q, r), with at most max_steps refinement steps (defaults 1e-12, 10) */
+ * (q, r), with at most max_steps refinement steps (defaults 1e-12, 10).  The residual that
+ * meets the tolerance gives one last step X += A32^-1 R (max_steps permitting) */
 int tups_set_refinement(tups_ctx* ctx, double tol, int32_t max_steps);
 /* after a closed-form tups_bse: the refinement steps the last call took (the
- * most over its passes) and the largest relative residual it reached; 0 and
+ * most over its passes, the last one included) and the largest relative residual it
+ * computed, that of X before the last step; 0 and
  * NaN after the direct mode, which computes no residual */
 int tups_bse_solve_info(const tups_ctx* ctx, int32_t* steps, double* residual);
 /* calc_chi for every q slot (SRC/parquet_chi.f90:438-523 with get_green_coarse,
@@ -371,10 +374,11 @@ int tups_set_product_forms(tups_ctx* ctx, int32_t allow_three);
 const char* tups_variant_name(int32_t kernel, int32_t variant);
 /* forces a variant id (must match the context's Nl); -1 restores the default.
  * TUPS_K_BSE_CLOSED and TUPS_K_BSE_IR choose the elimination of the closed
- * forms: 0 "gj_panel16" (16-column panels), 1 "gj_block64" (64-column blocks,
- * each passing the later columns through memory once), 2 "gj_block64_rp" (the
- * same with each 16-column sub-panel factored on registers, D <= 512, above
- * that as 1; the default from D = 128 on).  The closed forms work in passes
+ * forms: 0 "gj_panel16" (Gauss-Jordan elimination in 16-column panels), 1
+ * "gj_block64" (LU factors by 64-column blocks, the right-hand sides solved
+ * with them), 2 "gj_block64_rp" (the same with each 16-column sub-panel
+ * factored on registers, D <= 512, above that as 1; the default from D = 128
+ * on).  The closed forms work in passes
  * whose workspace is at most 16 GiB and half of the free device memory. */
 int tups_set_variant(tups_ctx* ctx, int32_t kernel, int32_t variant);
 /* number of variant ids of `kernel` (ids 0 .. n-1; a ladder or crossing
@@ -398,14 +402,14 @@ int tups_event_elapsed(tups_ctx* ctx, int32_t a, int32_t b, float* ms);
 #define TUPS_K_PAE_GATHER 5   /* Nl = 1: PhiR re-indexed for contiguous crossing reads */
 #define TUPS_K_SPLIT_PREP 6   /* split ladder: operands scaled to integers and reduced to residues */
 #define TUPS_K_SPLIT_GEMM 7   /* split ladder: INT8 MFMA residue products, CRT, damping */
-#define TUPS_K_BSE_CLOSED 8   /* closed form: build of [I - kappa Gamma chi | Gamma] and its solve */
+#define TUPS_K_BSE_CLOSED 8   /* closed form: build of I - kappa Gamma chi, its factors and the solve */
 #define TUPS_K_CALC_CHI 9     /* bubbles chi_ph, chi_pp for every q slot */
 #define TUPS_K_BSE_BATCH 10   /* batching form: variant names only (tups_variant_name/count) */
-#define TUPS_K_SDE 11         /* self-energy: auxiliary bubbles, vertex contraction, star sums */
+#define TUPS_K_SDE 11         /* self-energy: Green's functions, bubbles, vertex contraction, star sums */
 #define TUPS_K_GTAU 12        /* G(tau): mu bisection, fine-grid G(k, tau), 2D transform */
 #define TUPS_K_CONV 13        /* convergence check: Sigma change, vertex maxima */
 #define TUPS_K_SUS 14         /* susceptibilities: Green's-function pairs and their contraction */
-#define TUPS_K_BSE_IR 15      /* refined closed form: FP32 inverse, products with it, FP64 residuals */
+#define TUPS_K_BSE_IR 15      /* refined closed form: FP32 factors, solves with them, FP64 residuals */
 #define TUPS_K_COUNT 16
 int tups_set_timing(tups_ctx* ctx, int32_t on);
 int tups_get_timing(const tups_ctx* ctx, int32_t kernel, double* total_ms, int64_t* launches);

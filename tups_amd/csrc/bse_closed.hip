@@ -1,4 +1,4 @@
-// Closed form of the BSE ladder, direct (FP64) and by FP32 inverse with FP64
+// Closed form of the BSE ladder, direct (FP64) and by FP32 factors with FP64
 // iterative refinement.
 //
 // For fixed Gamma the damped update of BSE(ite) (SRC/parquet_BSE.f90:62-132),
@@ -9,34 +9,32 @@
 // per (q, r) and return Phi = X - Gamma: the converged ladder in one call.  The
 // reference has no such solve; it iterates the update.
 //
-// Direct mode (TUPS_BSE_CLOSED_LU): blocked Gauss-Jordan elimination with
-// partial pivoting on the augmented matrix [A | Gamma] (D x 2D, complex128),
-// one workgroup per matrix.  Per panel of NB columns:
+// Direct mode (TUPS_BSE_CLOSED_LU), from D = 128 the block form: A = P^-1 L U by
+// 64-column blocks with partial pivoting, a launch over all matrices per phase
+// (closed_panel, closed_diag, closed_row, closed_trail), the block rows scaled
+// by the inverses of their diagonal blocks (closed_scale), then the right-hand
+// sides by panels of 64 columns (closed_lu_solve).  Work per (q, r): (8/3 + 8)
+// D^3 real flops.  Below D = 128 closed_solve: Gauss-Jordan elimination with
+// partial pivoting on the augmented matrix [A | Gamma] (D x 2D, complex128), one
+// workgroup per matrix, 12 D^3 flops.  Per panel of CL_NB columns:
 //   1. LU of the panel rows k0..D-1 with row pivoting (rows swapped over all
 //      columns from k0 on, so the right-hand side follows the equations);
 //   2. Y = L11^-1 Z on the panel rows for every trailing column Z;
 //   3. rows below the panel: Z -= L21 Y                    (MFMA);
 //   4. X = U11^-1 Y on the panel rows;
 //   5. rows above the panel: Z -= P_above X                (MFMA);
-// after the last panel the right-hand block holds the solution.  Work per
-// (q, r): 12 D^3 real flops.  From D = 128 the block form (closed_solve_b64)
-// runs the same elimination with 64-column blocks: the block column factored
-// in a side buffer (on registers, 16 columns at a time, for D <= 512), T =
-// A11^-1 from blocked triangular inverses, the block rows multiplied by T and
-// every other row updated by rank-64 MFMA products whose operands stream
-// into LDS by direct global-to-LDS loads.
+// after the last panel the right-hand block holds the solution.
 //
-// Refinement mode (TUPS_BSE_CLOSED_IR): the same elimination in FP32 on
-// [fp32(A) | I] gives the inverse of the FP32-rounded A (its LU with partial
-// pivoting applied to the identity, FP32 MFMA updates); then
-//   X  = fp64(A32^-1 fp32(Gamma))                         (FP32 MFMA GEMM)
-//   repeat: R = Gamma - A X = Gamma - X + kappa Gamma (chi X)   (FP64 MFMA GEMM)
-//           stop when max over (q, r) of |R|_F / |Gamma|_F <= tol
-//           X += fp64(A32^-1 fp32(R))                     (FP32 MFMA GEMM)
+// Refinement mode (TUPS_BSE_CLOSED_IR): the same in FP32 (MFMA) on fp32(A); the
+// block form keeps the factors, below D = 128 the elimination of [fp32(A) | I]
+// gives the inverse.  With A32^-1 standing for either,
+//   X  = fp64(A32^-1 fp32(Gamma))
+//   repeat: R = Gamma - A X = Gamma - X + kappa (Gamma chi) X   (FP64 MFMA)
+//           X += fp64(A32^-1 fp32(R))
+//           stop after the step whose R had max over (q, r) of |R|_F / |Gamma|_F <= tol
 // FP64 is used only for A's assembly, the residual and the update of X.  Each
-// step shrinks the error by about cond(A) 2^-24, so two or three steps reach
-// 1e-12.  Work per (q, r): 12 D^3 FP32 (inverse) + 8 D^3 FP32 per product with
-// the inverse + 8 D^3 FP64 per residual.
+// step shrinks the error by about cond(A) 2^-24.  Work per (q, r): 8/3 D^3 FP32
+// (factors) + 8 D^3 FP32 per solve + 8 D^3 FP64 per residual.
 #include "internal.h"
 #include "lds_dma.h"
 
@@ -49,9 +47,9 @@ namespace tups {
 typedef double d4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 
-constexpr int CL_NB = 16;  // panel width (closed_solve), sub-panel width (closed_solve_b64)
+constexpr int CL_NB = 16;  // panel width (closed_solve), sub-panel width (block form)
 constexpr int CL_T = 64;   // update tile (rows and columns)
-constexpr int CL_BB = 64;  // block width of closed_solve_b64
+constexpr int CL_BB = 64;  // block width of the block form
 
 __device__ __forceinline__ double2 mkc(double x, double y) { return make_double2(x, y); }
 __device__ __forceinline__ float2 mkc(float x, float y) { return make_float2(x, y); }
@@ -1075,8 +1073,7 @@ struct TileSeg {
 // from `cols` and inner indices from s2.len on load clamped addresses: such inner indices
 // are zeroed in the last chunk, rows and columns dropped by the caller.
 // The register-fed form without prefetch took 11.39 ms for the FP64 residual (and 4.08 ms
-// more to form chi X) and 5.7 ms for an FP32 product at D = 320, 480 q; this one 8.17 and
-// 4.5 ms (61.6 and 112 TFLOP/s).
+// more to form chi X) at D = 320, 480 q; this one 7.43 ms (68 TFLOP/s).
 template <class R>
 __device__ __forceinline__ void tile_product(TileSeg<typename Prec<R>::C> s1, TileSeg<typename Prec<R>::C> s2, int ldb,
                                              int rows, int cols, char* lds, typename Prec<R>::V (&ar)[2][2],
@@ -1303,7 +1300,8 @@ struct LuArgs {
 // that are done and its own right-hand side.  The panel lives in the output (direct) or in
 // y (refinement); a block row is stored, and waited for, before the next one reads it.
 // MFMA-bound: 9.6 D^3 flops with the diagonal inverses, the factors shared through L2 by
-// the panels of a matrix, which run next to each other on one XCD.
+// the panels of a matrix, which run next to each other on one XCD.  D = 320, 480 q: 10.0 ms
+// in FP64 (60 TFLOP/s executed), 5.6 to 6.6 in FP32 by mode.
 //   MODE 0: FP64, B = Gamma, Phi = X - Gamma    MODE 1: X = fp64(A32^-1 rhs)
 //   MODE 2: X += fp64(A32^-1 rhs)               MODE 3: Phi = X + fp64(A32^-1 rhs) - Gamma
 // grid: ceil(D / 64) panels of every matrix
@@ -1544,9 +1542,9 @@ static void closed_common(tups_ctx* c, ClosedArgs& a) {
   for (int r = 0; r < 4; ++r) a.kappa[r] = 2.0 * cr[r] * s.alpha;
 }
 
-// elimination variants: 0 = CL_NB-wide panels (closed_solve), 1 = CL_BB-wide
-// blocks (closed_solve_b64), 2 = the same with the sub-panels on registers
-// (D <= 512; above that it runs as 1); -1 = 2 from D = 128 on
+// variants: 0 = Gauss-Jordan in CL_NB-wide panels (closed_solve), 1 = LU by
+// CL_BB-wide blocks, 2 = the same with the sub-panels on registers (D <= 512;
+// above that it runs as 1); -1 = 2 from D = 128 on
 static const char* const kClosedVariants[] = {"gj_panel16", "gj_block64", "gj_block64_rp"};
 constexpr int kClosedRp = 2;  // rows per thread of the register sub-panel
 int closed_variant_count() { return 3; }
@@ -1557,7 +1555,6 @@ static bool closed_blocked(const tups_ctx* c) {
 static bool closed_regs(const tups_ctx* c) {
   return closed_blocked(c) && c->closed_variant != 1 && c->sz.nz <= 256 * kClosedRp;
 }
-// scratch of closed_solve_b64 per matrix, in complex elements
 static size_t closed_blocks(size_t D) { return (D + CL_BB - 1) / CL_BB; }
 // per matrix of the block form: the factors and the diagonal inverses
 static size_t closed_b64_elems(size_t D) { return D * D + 2 * closed_blocks(D) * CL_BB * CL_BB; }
