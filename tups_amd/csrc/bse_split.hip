@@ -239,11 +239,13 @@ __global__ __launch_bounds__(256) void crt_prep_a(CrtArgs a) {
 // then lane l converts inner indices 4 l + 256 n .. + 3 and stores one dword
 // per (modulus, sign).  At the end the row maxima are the block's partial
 // rmaxp[mat][blockIdx.x][row].  With HALF (nf <= 32) the lower half of a wave
-// mixes F and the upper Gamma.  The columns beyond D are left out: they meet
-// only results that are not written.  grid: (Dp / 16, 4 * nqb); dynamic LDS
+// mixes F and the upper Gamma, the mixing loop is rolled (221 -> 124 registers at
+// Nl = 9), and the columns beyond D, which meet only results that are not
+// written, are left out; above, where half the loads in flight would be lost with
+// the registers, both cost 0.5 to 1 % (D = 320).  grid: (Dp / 16, 4 * nqb); dynamic LDS
 // 4 Kp 16 + Dp 8 (+ nl^2 nf 16 with CL).  Bound by the vector instructions of
 // the residues and, at two workgroups to a CU (LDS), their latencies: D = 198
-// (Dp = 256), Nl = 9, 110 q 785 -> 641 us; D = 320 988 us per 102 q, about as before.
+// (Dp = 256), Nl = 9, 110 q 785 -> 641 us; D = 320 985 us per 102 q.
 constexpr int PREP_B_CPW = PREP_B_COLS / 4;
 template <int NL, bool CL, bool HALF>
 __global__ __launch_bounds__(256, 2) void crt_prep_b(CrtArgs a) {
@@ -288,9 +290,8 @@ __global__ __launch_bounds__(256, 2) void crt_prep_b(CrtArgs a) {
   load_x(col0, hl, pf, pg);
   int fkeep = 0;  // lane cc keeps column cc's exponent; stored after the loop, so no store in it
                   // holds back the prefetch (a store's data register is waited for before reuse)
-  const int ncc = min(PREP_B_CPW, D - col0);
-#pragma unroll 1
-  for (int cc = 0; cc < ncc; ++cc) {  // the columns beyond D meet only results that are not written
+  const int ncc = HALF ? min(PREP_B_CPW, D - col0) : PREP_B_CPW;
+  for (int cc = 0; cc < ncc; ++cc) {
     const int col = col0 + cc;
     // B((part, l1, nu), col) = alpha sum_l3 chi_nu(l1, l3) X((l3, nu), col), X = F (part 0), Gamma (part 1)
     double mx = 0.0;
@@ -307,13 +308,19 @@ __global__ __launch_bounds__(256, 2) void crt_prep_b(CrtArgs a) {
         load_x(col, nu, xf, xg);
       }
       if (nu >= nf) continue;
+      if constexpr (!HALF) {
+        if (col >= D) {
+#pragma unroll
+          for (int l3 = 0; l3 < NL; ++l3) xf[l3] = xg[l3] = make_double2(0.0, 0.0);
+        }
+      }
 #pragma unroll
       for (int l3 = 0; l3 < NL; ++l3) {
         double am = fmax(fabs(xf[l3].x), fabs(xf[l3].y));
         if constexpr (!HALF) am = fmax(am, fmax(fabs(xg[l3].x), fabs(xg[l3].y)));
         atomicMax(&rmx[l3 * nf + nu], (unsigned long long)__double_as_longlong(am));
       }
-#pragma unroll 1
+#pragma unroll (HALF ? 1 : NL)
       for (int l1 = 0; l1 < NL; ++l1) {
         double fr = 0.0, fi = 0.0, gr = 0.0, gi = 0.0;
 #pragma unroll
