@@ -2,6 +2,7 @@
 // from it, shared by calc_chi, the self-energy and the susceptibilities.
 #pragma once
 #include "green.h"
+#include "green_shape.h"
 #include "internal.h"
 
 namespace tups {
@@ -10,26 +11,20 @@ namespace tups {
 // lo .. lo + len - 1 (1-based, outside 1..Nf with Sigma_H): tab[(slot Nc + k) len +
 // nu - lo].  Slot s holds grain s = (gy - 1) Ng + gx - 1; when all of them would
 // exceed kGreenTabBytes, a pass holds `grains` of them from g0 on, then their
-// mirror images Ng^2 - 1 - g, then the lattice point itself (plain).
-struct GreenTab {
+// mirror images Ng^2 - 1 - g, then the lattice point itself (plain): green_shape.h.
+struct GreenTab : GreenShape {
   const double2* tab = nullptr;
-  int lo = 0, len = 0;
-  int ng2 = 1;      // grains in all
-  int grains = 1;   // grains of one pass
-  bool split = false;
-  int plain = 0;    // slot of the lattice point itself
 };
-constexpr size_t kGreenTabBytes = (size_t)256 << 20;
 
 // the weight families: groups of NW weights wt[(group Nc + k) NW + i], and per weight
 // where its sum goes, dst[3 i]: array pair, place, second place (-1: none)
 enum { kBubbleChi = 0, kBubbleAux = 1, kBubbleChiAux = 2, kBubbleSus = 3 };
 
-// reserves the table for this Ngrain and f_range (outside any capture)
+// reserves the table for this Ngrain and every shape that work at f_range builds (outside any capture)
 int green_tab_reserve(tups_ctx* c, int ngrain, int f_range);
-// forms pass `pass` of the table (one pass unless split) on the context's stream
+// forms pass `pass` of the table (one pass unless split) on the context's stream; an error
+// when the reserved table does not hold it
 int green_tab_build(tups_ctx* c, const GreenParams& g, int f_range, int pass, GreenTab* out);
-inline int green_tab_passes(const GreenTab& t) { return (t.ng2 + t.grains - 1) / t.grains; }
 
 // destination of one array pair: element q qs + o os + place us, o the frequency of the enlarged box
 struct BubbleOut {

@@ -163,7 +163,9 @@ __global__ __launch_bounds__(256) void bubble_kernel(BubbleArgs a) {
 // the widths that bubble_kernel exists for
 static const int kBubbleWidths[] = {1, 2, 5, 10, 15, 20};
 
-static void tab_shape(const tups_ctx* c, int ngrain, int f_range, GreenTab* t);
+static GreenShape tab_shape(const tups_ctx* c, int ngrain, int f_range) {
+  return green_shape(c->sz.nc, c->sz.nf, c->sz.nw, ngrain, f_range);
+}
 
 int upload_bubble_weights(tups_ctx* c) {
   const Tables& t = c->tab;
@@ -221,11 +223,9 @@ int upload_bubble_weights(tups_ctx* c) {
     }
   }
   // one block: the weights, their places, and room for the table at Ngrain 1 and f_range 0
-  GreenTab t1;
-  tab_shape(c, 1, 0, &t1);
   const size_t o_dst = wt.size() * sizeof(double);
   const size_t o_tab = (o_dst + dst.size() * sizeof(int) + 255) / 256 * 256;
-  const size_t n_tab = (size_t)nc * t1.len * sizeof(double2);
+  const size_t n_tab = tab_shape(c, 1, 0).bytes(nc);
   if (c->green_tab_owned) (void)hipFree(c->green_tab);
   if (c->d_bubble_wt) (void)hipFree(c->d_bubble_wt);
   c->green_tab = nullptr;
@@ -245,29 +245,9 @@ int upload_bubble_weights(tups_ctx* c) {
   return TUPS_OK;
 }
 
-static void tab_shape(const tups_ctx* c, int ngrain, int f_range, GreenTab* t) {
-  const tups_sizes& s = c->sz;
-  // k + q and q - k reach (f_range + 1) Nf + Nw - 1 on top, the self-energy's k - q down to 2 - Nw
-  t->lo = std::min(1 - f_range * s.nf, 2 - s.nw);
-  t->len = (f_range + 1) * s.nf + s.nw - t->lo;
-  t->ng2 = ngrain * ngrain;
-  const size_t per = (size_t)s.nc * t->len * sizeof(double2);
-  t->split = per * t->ng2 > kGreenTabBytes && t->ng2 > 1;
-  if (t->split) {
-    t->grains = (int)std::min<size_t>(t->ng2, std::max<size_t>(1, kGreenTabBytes / per / 2));
-    t->plain = 2 * t->grains;
-  } else {
-    t->grains = t->ng2;
-    const int half = (ngrain + 1) / 2 - 1;
-    t->plain = half * ngrain + half;
-  }
-}
-
 int green_tab_reserve(tups_ctx* c, int ngrain, int f_range) {
-  GreenTab t;
-  tab_shape(c, ngrain, f_range, &t);
-  const size_t slots = t.split ? 2 * (size_t)t.grains + 1 : t.grains;
-  const size_t need = slots * c->sz.nc * t.len * sizeof(double2);
+  const tups_sizes& s = c->sz;
+  const size_t need = green_reserve_bytes(s.nc, s.nf, s.nw, ngrain, f_range);
   if (c->green_tab_bytes < need) {
     drop_graphs(c);  // captured graphs hold the old table
     if (c->green_tab_owned) TUPS_HIP(hipFree(c->green_tab));
@@ -288,10 +268,11 @@ int green_tab_reserve(tups_ctx* c, int ngrain, int f_range) {
 }
 
 int green_tab_build(tups_ctx* c, const GreenParams& g, int f_range, int pass, GreenTab* out) {
-  tab_shape(c, g.ngrain, f_range, out);
+  static_cast<GreenShape&>(*out) = tab_shape(c, g.ngrain, f_range);
   out->tab = c->green_tab;
-  const int slots = out->split ? 2 * out->grains + 1 : out->grains;
-  const size_t n = (size_t)slots * c->sz.nc * out->len;
+  const int slots = (int)out->slots();
+  const size_t n = out->slots() * c->sz.nc * out->len;
+  TUPS_CHECK(out->bytes(c->sz.nc) <= c->green_tab_bytes, TUPS_ESTATE, "Green's-function table larger than reserved");
   const size_t nb = (n + 255) / 256;
   TUPS_CHECK(nb < ((size_t)1 << 31), TUPS_EINVAL, "Green's-function table grid too large");
   hipLaunchKernelGGL(green_table, dim3((unsigned)nb), dim3(256), 0, c->stream, g, c->green_tab, out->lo, out->len,
@@ -335,7 +316,7 @@ int launch_bubbles(tups_ctx* c, const GreenParams& g, int f_range, int set, cons
     } else if (int rc = green_tab_build(c, g, f_range, p, &t)) {
       return rc;
     }
-    passes = green_tab_passes(t);
+    passes = t.passes();
     a.tab = t.tab;
     a.lo = t.lo;
     a.len = t.len;
