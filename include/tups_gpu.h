@@ -79,8 +79,7 @@ extern "C" {
                                    MFMA) and FP64 iterative refinement X += A32^-1 (Gamma - A X)
                                    until |R|_F / |Gamma|_F <= the tolerance of
                                    tups_set_refinement (default 1e-12, at most 10 steps;
-                                   TUPS_ENOCONV otherwise); the residual that meets it gives
-                                   one last step while steps are left */
+                                   TUPS_ENOCONV otherwise) */
 
 typedef struct tups_dims {
   int32_t nx;        /* Nx = Ny (even), SRC/parquet_ini.f90:304-305 */
@@ -160,12 +159,13 @@ int tups_upload_chi_dense(tups_ctx* ctx, int32_t pp, int32_t q0, int32_t nqs,
 /* BSE(ite): Gamma_r <- Phi_r for r = d,m,s,t; SRC/parquet_BSE.f90:62-132 */
 int tups_bse(tups_ctx* ctx, int32_t mode);
 /* TUPS_BSE_CLOSED_IR: refine until |Gamma - A X|_F / |Gamma|_F <= tol for every
- * (q, r), with at most max_steps refinement steps (defaults 1e-12, 10).  The residual that
- * meets the tolerance gives one last step X += A32^-1 R (max_steps permitting) */
+ * (q, r), with at most max_steps refinement steps (defaults 1e-12, 10).  With tol <= 2^-36
+ * the X that meets it gets one more step if max_steps permits, which is kept if its
+ * result meets tol as well: the X returned is always one whose residual was computed and
+ * meets tol */
 int tups_set_refinement(tups_ctx* ctx, double tol, int32_t max_steps);
 /* after a closed-form tups_bse: the refinement steps the last call took (the
- * most over its passes, the last one included) and the largest relative residual it
- * computed, that of X before the last step; 0 and
+ * most over its passes) and the largest relative residual of the X it returned; 0 and
  * NaN after the direct mode, which computes no residual */
 int tups_bse_solve_info(const tups_ctx* ctx, int32_t* steps, double* residual);
 /* calc_chi for every q slot (SRC/parquet_chi.f90:438-523 with get_green_coarse,

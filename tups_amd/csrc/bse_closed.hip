@@ -30,11 +30,13 @@
 // gives the inverse.  With A32^-1 standing for either,
 //   X  = fp64(A32^-1 fp32(Gamma))
 //   repeat: R = Gamma - A X = Gamma - X + kappa (Gamma chi) X   (FP64 MFMA)
+//           stop when max over (q, r) of |R|_F / |Gamma|_F <= tol
 //           X += fp64(A32^-1 fp32(R))
-//           stop after the step whose R had max over (q, r) of |R|_F / |Gamma|_F <= tol
 // FP64 is used only for A's assembly, the residual and the update of X.  Each
-// step shrinks the error by about cond(A) 2^-24.  Work per (q, r): 8/3 D^3 FP32
-// (factors) + 8 D^3 FP32 per solve + 8 D^3 FP64 per residual.
+// step shrinks the error by about cond(A) 2^-24.  A tolerance for full double
+// precision (kIrFull) asks for one step beyond the X that meets it; the X that is
+// returned is in every case one whose own residual meets the tolerance.  Work per
+// (q, r): 8/3 D^3 FP32 (factors) + 8 D^3 FP32 per solve + 8 D^3 FP64 per residual.
 #include "internal.h"
 #include "lds_dma.h"
 
@@ -1035,6 +1037,8 @@ struct IrArgs {
   const double2* gam[4];
   double2* x[4];             // X_r, the solution, in the output arrays
   const float2* inv;         // [mat][2D][D]: the inverse is columns D..2D-1
+  float2* y;                 // the last product with A32^-1: matrix mat at y + ys mat
+  size_t ys;
   float2* rhs;               // [mat][D][D] right-hand side of the next product: fp32(Gamma), then fp32(R)
   const double2* gx;         // [mat][D][D] Gamma chi
   double* part;              // [mat][tiles][2]: sum |R|^2, sum |Gamma|^2 per tile
@@ -1286,7 +1290,7 @@ __global__ __launch_bounds__(256, 3) void closed_trail(ClosedArgs a, int k0) {
 
 struct LuArgs {
   const double2* gam[4];
-  double2* x[4];        // the output arrays: X, or Phi
+  double2* x[4];        // the output arrays: X (MODE 0: Phi)
   const void* W;        // scaled block rows
   const void* T;        // diagonal inverses
   const int* perm;
@@ -1303,7 +1307,7 @@ struct LuArgs {
 // the panels of a matrix, which run next to each other on one XCD.  D = 320, 480 q: 10.0 ms
 // in FP64 (60 TFLOP/s executed), 5.6 to 6.6 in FP32 by mode.
 //   MODE 0: FP64, B = Gamma, Phi = X - Gamma    MODE 1: X = fp64(A32^-1 rhs)
-//   MODE 2: X += fp64(A32^-1 rhs)               MODE 3: Phi = X + fp64(A32^-1 rhs) - Gamma
+//   MODE 2: X += fp64(A32^-1 rhs)
 // grid: ceil(D / 64) panels of every matrix
 template <int MODE>
 __global__ __launch_bounds__(256, 3) void closed_lu_solve(LuArgs a) {
@@ -1360,11 +1364,10 @@ __global__ __launch_bounds__(256, 3) void closed_lu_solve(LuArgs a) {
           buf[at] = mkc(ar[i][j][e], ai[i][j][e]);
           if constexpr (MODE == 1) {
             if (last) X[at] = make_double2((double)ar[i][j][e], (double)ai[i][j][e]);
-          } else if constexpr (MODE >= 2) {
+          } else if constexpr (MODE == 2) {
             if (last) {
               const double2 x = X[at];
-              const double2 v = make_double2(x.x + (double)ar[i][j][e], x.y + (double)ai[i][j][e]);
-              X[at] = MODE == 3 ? csub(v, G[at]) : v;
+              X[at] = make_double2(x.x + (double)ar[i][j][e], x.y + (double)ai[i][j][e]);
             }
           }
         }
@@ -1444,6 +1447,7 @@ __global__ __launch_bounds__(256, 3) void ir_gemm(IrArgs a) {
         } else if (MODE == 1) {
           const double2 x = X[idx];
           X[idx] = make_double2(x.x + (double)ar[i][j][e], x.y + (double)ai[i][j][e]);
+          a.y[a.ys * mat + idx] = make_float2((float)ar[i][j][e], (float)ai[i][j][e]);
         } else {
           const double2 g = G[idx], x = X[idx];
           const double2 v = make_double2(g.x - x.x + kap * ar[i][j][e], g.y - x.y + kap * ai[i][j][e]);
@@ -1488,6 +1492,19 @@ __global__ __launch_bounds__(256) void ir_check(IrArgs a, int mats) {
   const double s = v == v ? v : INFINITY;
   a.res[mat] = s;
   atomicMax(a.rmax, (unsigned long long)__double_as_longlong(s));
+}
+
+// X without its last correction; grid (ceil(D^2 / 256), 4 nqb)
+__global__ __launch_bounds__(256) void ir_take_back(IrArgs a) {
+  const int mat = blockIdx.y;
+  const int r = mat / a.nqb, q = a.q0 + (mat - r * a.nqb);
+  const size_t DD = (size_t)a.D * a.D;
+  const size_t u = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (u >= DD) return;
+  double2* X = a.x[r] + DD * q;
+  const float2 y = a.y[a.ys * mat + u];
+  const double2 x = X[u];
+  X[u] = make_double2(x.x - (double)y.x, x.y - (double)y.y);
 }
 
 // Phi = X - Gamma in place (X sits in the output array); grid (ceil(D^2 / 256), 4 nqb)
@@ -1651,6 +1668,12 @@ int launch_bse_closed(tups_ctx* c) {
   return TUPS_OK;
 }
 
+// A tolerance of the refinement up to here asks for all that FP64 gives: one step leaves
+// 1e-13 to 9e-13 (D = 16 to 576), between which and the tolerance chance would decide whether X
+// is exact to 1e-12 or to 1e-15.  Above it X is wanted as soon as it meets the tolerance.  The step
+// beyond and its residual cost 14 of 50 ms at D = 320, 480 q.
+constexpr double kIrFull = 0x1p-36;
+
 int launch_bse_closed_ir(tups_ctx* c) {
   const tups_sizes& s = c->sz;
   TUPS_CHECK(s.nl <= CL_NL_MAX, TUPS_EINVAL, "closed form: at most 9 form factors");
@@ -1691,6 +1714,9 @@ int launch_bse_closed_ir(tups_ctx* c) {
     b.inv = reinterpret_cast<const float2*>(base);
     base += mats_max * 2 * DD * sizeof(float2);
   }
+  // the corrections: the block form's product, or the columns that the elimination has used up
+  b.y = blk ? y32 : static_cast<float2*>(a.W);
+  b.ys = blk ? DD : 2 * DD;
   base = reinterpret_cast<char*>((reinterpret_cast<uintptr_t>(base) + 15) / 16 * 16);
   b.part = reinterpret_cast<double*>(base);
   base += mats_max * tiles_n * tiles_n * 2 * sizeof(double);
@@ -1725,8 +1751,10 @@ int launch_bse_closed_ir(tups_ctx* c) {
     }
     TUPS_HIP(hipGetLastError());
     int steps = 0;
-    bool phi = false;  // the output holds Phi already
+    // beyond: X has had a step beyond the X that met the tolerance; back: that step was taken back
+    bool beyond = false, back = false;
     double res = INFINITY;
+    const dim3 all((unsigned)((DD + 255) / 256), mats);
     for (;;) {
       hipLaunchKernelGGL(ir_clear, dim3(1), dim3(1), 0, c->stream, b.rmax);
       TUPS_HIP(hipGetLastError());
@@ -1738,23 +1766,30 @@ int launch_bse_closed_ir(tups_ctx* c) {
       TUPS_HIP(hipMemcpyAsync(&bits, b.rmax, sizeof(bits), hipMemcpyDeviceToHost, c->stream));
       TUPS_HIP(hipStreamSynchronize(c->stream));
       std::memcpy(&res, &bits, sizeof(res));
-      // converged: the residual at hand gives one more step without another one to follow, so
-      // that a first solve good enough for the tolerance is no less exact than one that missed it
       const bool done = res <= c->ir_tol;
-      if (steps >= c->ir_max_steps || (done && !(res > 0x1p-50))) break;
+      if (beyond && !done) {
+        // with a badly conditioned A a step need not make X better
+        hipLaunchKernelGGL(ir_take_back, all, dim3(256), 0, c->stream, b);
+        TUPS_HIP(hipGetLastError());
+        --steps;
+        beyond = false;
+        back = true;
+        continue;
+      }
+      // done: the step beyond makes a first solve that is just good enough no less exact than
+      // one that just missed the tolerance and was refined
+      const bool more = done ? c->ir_tol <= kIrFull && res > 0x1p-50 : true;
+      if (beyond || back || !more || steps >= c->ir_max_steps) break;
       // X += A32^-1 R
-      if (blk && done) {
-        hipLaunchKernelGGL(closed_lu_solve<3>, dim3(glu), dim3(256), 0, c->stream, lu);
-        phi = true;
-      } else if (blk)
+      if (blk)
         hipLaunchKernelGGL(closed_lu_solve<2>, dim3(glu), dim3(256), 0, c->stream, lu);
       else
         hipLaunchKernelGGL(ir_gemm<1>, dim3(gblk), dim3(256), 0, c->stream, b);
       TUPS_HIP(hipGetLastError());
       ++steps;
-      if (done) break;
+      beyond = done;
     }
-    if (!phi) hipLaunchKernelGGL(ir_final, dim3((unsigned)((DD + 255) / 256), mats), dim3(256), 0, c->stream, b);
+    hipLaunchKernelGGL(ir_final, all, dim3(256), 0, c->stream, b);
     TUPS_HIP(hipGetLastError());
     if (int rc = timer_end(c, TUPS_K_BSE_IR)) return rc;
     steps_max = std::max(steps_max, steps);

@@ -348,7 +348,7 @@ class TupsContext:
         _check(self.lib.tups_set_refinement(self._h, float(tol), int(max_steps)), "tups_set_refinement")
 
     def solve_info(self):
-        """(refinement steps, largest |R|_F / |Gamma|_F) of the last closed-form BSE."""
+        """(refinement steps, largest |R|_F / |Gamma|_F of what was returned) of the last closed-form BSE."""
         steps = C.c_int32(0)
         res = C.c_double(0.0)
         _check(self.lib.tups_bse_solve_info(self._h, C.byref(steps), C.byref(res)), "tups_bse_solve_info")
