@@ -85,8 +85,9 @@ int launch_chi_aux_device(tups_ctx* c, const GreenParams& g, const BubbleOut& au
 
 int launch_calc_chi(tups_ctx* c, const double* sigma, const double* sigma_h, double mu, int ngrain) {
   GreenParams g{};
-  if (int rc = upload_sigma(c, sigma, sigma_h, &g, mu, ngrain)) return rc;
+  TUPS_CHECK(ngrain >= 1 && ngrain <= 64, TUPS_EINVAL, "ngrain must be in 1..64");
   if (int rc = green_tab_reserve(c, ngrain, 0)) return rc;
+  if (int rc = upload_sigma(c, sigma, sigma_h, &g, mu, ngrain)) return rc;
   return launch_chi_device(c, g, nullptr);
 }
 

@@ -254,7 +254,7 @@ int upload_sigma(tups_ctx* c, const double* sigma, const double* sigma_h, GreenP
 int launch_sde(tups_ctx* c, const double* sigma, const double* sigma_h, double mu, int ngrain, int f_range, double u,
                int use_u2, double* sigma_out);
 int launch_chi_device(tups_ctx* c, const GreenParams& g, const GreenTab* tab);
-int sde_reserve(tups_ctx* c, int f_range);
+int sde_reserve(tups_ctx* c, int ngrain, int f_range);
 int launch_sde_device(tups_ctx* c, const GreenParams& g, const GreenTab* tab, bool aux_done, int f_range, double u,
                       int use_u2);
 int launch_sigma_commit(tups_ctx* c, int f_range);

@@ -167,7 +167,7 @@ extern "C" int tups_iteration_full(tups_ctx* c, int32_t mode, int32_t use_graph,
   if (rc) return rc;
   if ((rc = pae_plan_ensure(c))) return rc;
   if (mode == TUPS_BSE_LADDER_SPLIT && (rc = bse_split_reserve(c, nullptr))) return rc;
-  if ((rc = sde_reserve(c, f_range))) return rc;
+  if ((rc = sde_reserve(c, c->green_ngrain, f_range))) return rc;
   if (!(n_particle >= 0.0)) n_particle = -1.0;  // negative or NaN: mu stays
   const bool gtau = n_particle >= 0.0 || use_u2;
   if (gtau && (rc = gtau_reserve(c, c->green_ngrain))) return rc;

@@ -316,9 +316,11 @@ static SdeParts sde_parts(const tups_sizes& s, int f_range) {
   return p;
 }
 
-// workspace of the SDE for f_range (allocated outside any stream capture)
-int sde_reserve(tups_ctx* c, int f_range) {
+// workspace and table of the SDE for ngrain and f_range (allocated outside any stream
+// capture, and before a call changes anything: what is refused here leaves the context as it was)
+int sde_reserve(tups_ctx* c, int ngrain, int f_range) {
   const tups_sizes& s = c->sz;
+  TUPS_CHECK(ngrain >= 1 && ngrain <= 64, TUPS_EINVAL, "ngrain must be in 1..64");
   TUPS_CHECK(f_range >= 0 && f_range <= 8, TUPS_EINVAL, "f_range must be in 0..8");
   const size_t need = sde_parts(s, f_range).total() * sizeof(double2);
   if (c->sde_ws_bytes < need) {
@@ -329,7 +331,7 @@ int sde_reserve(tups_ctx* c, int f_range) {
     TUPS_HIP(hipMalloc(&c->sde_ws, need));
     c->sde_ws_bytes = need;
   }
-  return green_tab_reserve(c, c->green_ngrain, f_range);
+  return green_tab_reserve(c, ngrain, f_range);
 }
 
 // Sigma output of the last SDE launch with this f_range (inside the workspace)
@@ -458,8 +460,8 @@ int launch_sde(tups_ctx* c, const double* sigma, const double* sigma_h, double m
   const tups_sizes& s = c->sz;
   TUPS_CHECK(sigma_out, TUPS_EINVAL, "null output");
   GreenParams g{};
+  if (int rc = sde_reserve(c, ngrain, f_range)) return rc;
   if (int rc = upload_sigma(c, sigma, sigma_h, &g, mu, ngrain)) return rc;
-  if (int rc = sde_reserve(c, f_range)) return rc;
   if (int rc = launch_sde_device(c, g, nullptr, false, f_range, u, use_u2)) return rc;
   if (use_u2) {
     TUPS_CHECK(c->grt_valid && c->gt_ngrain == ngrain, TUPS_ESTATE,
