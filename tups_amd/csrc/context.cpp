@@ -674,6 +674,7 @@ int tups_copy(tups_ctx* c, int32_t wd, int32_t ws, int32_t ch) {
   double2* s = array_ptr(c, ws, ch);
   TUPS_CHECK(d && s && array_elems(c, wd) == array_elems(c, ws), TUPS_EINVAL, "incompatible arrays");
   TUPS_HIP(hipMemcpyAsync(d, s, array_elems(c, wd) * sizeof(double2), hipMemcpyDeviceToDevice, c->stream));
+  if (wd == TUPS_M) c->pae_plan_valid = false;  // the crossing's plan holds M's elements
   return TUPS_OK;
 }
 
