@@ -1237,15 +1237,20 @@ static int pae_gemm_path(tups_ctx* c, bool update) {
   return TUPS_OK;
 }
 
-// The variant without autotuning, times in us at (Nx, Nf) of it | pre-pass + 4 columns:
-// up to Nf = 16 the all-momenta form, whose few workgroups each do all of the work of
-// their entries (4, 16: 4.8 | 6.5); 56 < Nf <= 64 fills the rows of its 64-wide tiles and
-// four entries per thread put one workgroup on each CU ((8, 64): 52 | 74, (16, 64): 141 |
-// 188); else 16 momenta per thread with PhiR re-indexed on the way ((6, 30): 7.1 | 11.7,
-// (8, 32): 8.0 | 15.9, (20, 40): 57 | 85, (8, 128): 397 | 553, (16, 96): 518 | 770).
+// The variant without autotuning, times of a call in us at (Nx, Nf) with the launch:
+//  Nf <= 16: 8 momenta per thread with PhiR re-indexed on the way.  Few workgroups, so the
+//    momenta are spread; against pre-pass + 4 columns and all momenta in one workgroup
+//    (4, 16) 5.6 | 7.4 | 6.4, (8, 16) 6.0 | 7.3 | 9.8, (16, 16) 6.6 | 9.8 | 21, (32, 16) 16 | 24 | 96;
+//  56 < Nf <= 64: the rows fill 64-wide tiles and four entries per thread over all momenta
+//    put one workgroup on each CU; against pre-pass + 4 columns and 16 momenta per thread
+//    (8, 58) 43 | 65 | 46, (8, 64) 52 | 74 | 55, (16, 64) 138 | 180 | 151.  At twice the rows
+//    that is two workgroups a CU and more columns than the momenta share: (8, 120) 377 | 499 | 340,
+//    (8, 128) 430 | 536 | 395;
+//  else 16 momenta per thread, PhiR re-indexed on the way; against pre-pass + 4 columns
+//    (6, 30) 8.5 | 12, (8, 32) 9.5 | 16, (20, 40) 59 | 84, (16, 96) 527 | 755, (8, 128) 395 | 536.
 static int pae_default(const tups_ctx* c) {
   const tups_sizes& s = c->sz;
-  const char* name = s.nr != 1 ? "nl1_c4_nr" : s.nf <= 16 ? "nl1_a2" : s.nf > 56 && s.nf <= 64 ? "nl1_e4p" : "nl1_f16";
+  const char* name = s.nr != 1 ? "nl1_c4_nr" : s.nf <= 16 ? "nl1_f8" : s.nf > 56 && s.nf <= 64 ? "nl1_e4p" : "nl1_f16";
   for (int v = 0; v < kNumPaeVariants; ++v)
     if (std::strcmp(kPaeVariants[v].name, name) == 0) return v;
   return 1;
