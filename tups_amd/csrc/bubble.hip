@@ -14,8 +14,9 @@
 // is one (q, nu) with nu fastest, so the three reads of a (grain, k) are contiguous
 // runs of the table (0.4 to 8 MB, served by L1 and L2), k and with it every weight
 // is uniform over the wave (scalar operands), and the sums stay in registers: no
-// LDS between the product and the projection.  Four waves take every fourth k and
-// are added in order at the end.  Bound by the issue of the 8 + 4 NW FP64 operations
+// LDS between the product and the projection.  Four waves (with 16 lanes, for small
+// grids, 16 parts) take every fourth k and are added in order at the end.  Bound by
+// the issue of the 8 + 4 NW FP64 operations
 // per (grain, k) and, at few weights, by the L1 reads.  calc_chi and calc_chi_aux
 // together at Nx = 16, Nf = 64, Nl = 1 (1440 q): 63 us (1224 + 664 us); calc_GG at
 // Nx = 8, Nf = 64, Nl = 5, Ngrain = 4: 75 us (2681 us); the table 4 to 5 us.
@@ -63,15 +64,16 @@ struct BubbleArgs {
   double inv_g2;
 };
 
-// grid: (ceil(nq ext / 64), weight groups); 64 lanes of (q, nu) x 4 waves over k
-template <int NW>
+// grid: (ceil(nq ext / LANES), weight groups); LANES lanes of (q, nu) x 256 / LANES parts of k
+template <int NW, int LANES>
 __global__ __launch_bounds__(256) void bubble_kernel(BubbleArgs a) {
   constexpr int STEP = NW < 4 ? NW : 4;  // weights reduced at a time
-  __shared__ double2 red[3][2 * STEP][64];
-  const int lane = threadIdx.x & 63;
-  const int part = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  constexpr int PARTS = 256 / LANES;
+  __shared__ double2 red[PARTS - 1][2 * STEP][LANES];
+  const int lane = threadIdx.x & (LANES - 1);
+  const int part = LANES == 64 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x / LANES;
   const int grp = blockIdx.y;
-  const long long t = (long long)blockIdx.x * 64 + lane;
+  const long long t = (long long)blockIdx.x * LANES + lane;
   const bool ok = t < (long long)a.nq * a.ext;
   const int q = ok ? (int)(t / a.ext) : 0, o = ok ? (int)(t - (long long)q * a.ext) : 0;
   const int nx = a.nx, nc = nx * nx, m = a.qm[q];
@@ -84,7 +86,7 @@ __global__ __launch_bounds__(256) void bubble_kernel(BubbleArgs a) {
 #pragma unroll
   for (int i = 0; i < NW; ++i) ph[i] = pp[i] = make_double2(0.0, 0.0);
   const double* wt = a.wt + (size_t)grp * nc * NW;
-  for (int k = part; k < nc; k += 4) {
+  for (int k = part; k < nc; k += PARTS) {
     const int ky = k / nx, kx = k - ky * nx;
     int ax = kx + qx, ay = ky + qy, bx = qx - kx, by = qy - ky;
     ax -= ax >= nx ? nx : 0;
@@ -134,7 +136,7 @@ __global__ __launch_bounds__(256) void bubble_kernel(BubbleArgs a) {
         if (i0 + i >= NW || gi >= a.nwt) continue;
         double2 x = ph[i0 + i], y = pp[i0 + i];
 #pragma unroll
-        for (int r = 0; r < 3; ++r) {
+        for (int r = 0; r < PARTS - 1; ++r) {
           x.x += red[r][2 * i][lane].x;
           x.y += red[r][2 * i][lane].y;
           y.x += red[r][2 * i + 1][lane].x;
@@ -160,8 +162,10 @@ __global__ __launch_bounds__(256) void bubble_kernel(BubbleArgs a) {
   }
 }
 
-// the widths that bubble_kernel exists for
-static const int kBubbleWidths[] = {1, 2, 5, 10, 15, 20};
+// the widths that bubble_kernel exists for; a narrow layout has at most kNarrowWidth of
+// more than 2 kNarrowWidth weights in a group
+static const int kBubbleWidths[] = {1, 2, 5, 10, 15, 20, 23};
+constexpr int kNarrowWidth = 5;
 
 static GreenShape tab_shape(const tups_ctx* c, int ngrain, int f_range) {
   return green_shape(c->sz.nc, c->sz.nf, c->sz.nw, ngrain, f_range);
@@ -200,16 +204,19 @@ int upload_bubble_weights(tups_ctx* c) {
   const std::vector<Weight>* sets[4] = {&chi, &aux, &both, &sus};
   std::vector<double> wt;
   std::vector<int> dst;
-  for (int k = 0; k < 4; ++k) {
-    const std::vector<Weight>& v = *sets[k];
-    BubbleSet& b = c->bubble_set[k];
+  for (int kk = 0; kk < 8; ++kk) {
+    const bool wide = kk >= 4;
+    const std::vector<Weight>& v = *sets[kk & 3];
+    BubbleSet& b = c->bubble_set[wide][kk & 3];
     b.count = (int)v.size();
     b.wt = wt.size();
     b.dst = (int)dst.size();
-    // a group costs its NW weights and the products it forms again, worth about four
+    // a group costs its NW weights and the products it forms again, worth about four a grain;
+    // the wide layout is for many of them
     long long best = -1;
     for (int w : kBubbleWidths) {
-      const long long g = (b.count + w - 1) / w, cost = g * (w + 4);
+      if (!wide && w > kNarrowWidth && b.count > 2 * kNarrowWidth) continue;
+      const long long g = (b.count + w - 1) / w, cost = g * (w + (wide ? 64 : 4));
       if (best < 0 || cost < best) {
         best = cost;
         b.nw = w;
@@ -283,7 +290,14 @@ int green_tab_build(tups_ctx* c, const GreenParams& g, int f_range, int pass, Gr
 
 int launch_bubbles(tups_ctx* c, const GreenParams& g, int f_range, int set, const BubbleOut* out, const GreenTab* built) {
   const tups_sizes& s = c->sz;
-  const BubbleSet& bs = c->bubble_set[set];
+  // Narrow groups of weights where forming the products again costs little (one grain) or
+  // falls to CUs that would be idle; us a call of calc_chi, narrow | wide at (Nx, Nf, Nl, Ngrain):
+  // (4, 16, 5, 1) 27 | 31, (8, 16, 5, 1) 30 | 36, (6, 22, 9, 1) 34 | 41, (8, 64, 9, 1) 106 | 116,
+  // (4, 32, 9, 2) 32 | 43; (8, 64, 5, 2) 86 | 74, (8, 32, 9, 4) 153 | 102.
+  const long long n64 = ((long long)s.nq * (2 * f_range + 1) * s.nf + 63) / 64;
+  const long long work = (long long)s.nc * g.ngrain * g.ngrain;  // products of a lane
+  const bool wide = g.ngrain > 1 && (work > 256 || n64 * c->bubble_set[0][set].groups > 512);
+  const BubbleSet& bs = c->bubble_set[wide][set];
   BubbleArgs a{};
   a.wt = c->d_bubble_wt + bs.wt;
   a.dst = c->d_bubble_dst + bs.dst;
@@ -305,7 +319,11 @@ int launch_bubbles(tups_ctx* c, const GreenParams& g, int f_range, int set, cons
   a.f_range = f_range;
   a.nwt = bs.count;
   a.inv_g2 = 1.0 / g.ngrain / g.ngrain;
-  const long long nb = ((long long)s.nq * a.ext + 63) / 64;
+  // A grid of less than half a workgroup a CU (one, with long sums) takes 16 lanes a
+  // workgroup and splits a lane's products over 16 parts; 64 | 16 lanes at (Nx, Nf, Nl, Ngrain):
+  // (4, 16, 5, 16) 334 | 97 us, (8, 16, 5, 4) 105 | 48, (8, 24, 9, 8) 211 | 187, (8, 24, 9, 1) 59 | 73.
+  const bool few = (n64 * bs.groups <= 128 && work >= 64) || (n64 * bs.groups <= 256 && work >= 4096);
+  const long long nb = few ? ((long long)s.nq * a.ext + 15) / 16 : n64;
   TUPS_CHECK(nb < (1LL << 31), TUPS_EINVAL, "bubble grid too large");
   const dim3 grid((unsigned)nb, (unsigned)bs.groups);
   GreenTab t;
@@ -324,14 +342,17 @@ int launch_bubbles(tups_ctx* c, const GreenParams& g, int f_range, int set, cons
     a.mirror = t.split ? -1 : t.ng2 - 1;
     a.mslot = t.grains;
     a.accumulate = p > 0 ? 1 : 0;
+    void (*fn)(BubbleArgs);
     switch (bs.nw) {
-      case 1: hipLaunchKernelGGL(bubble_kernel<1>, grid, dim3(256), 0, c->stream, a); break;
-      case 2: hipLaunchKernelGGL(bubble_kernel<2>, grid, dim3(256), 0, c->stream, a); break;
-      case 5: hipLaunchKernelGGL(bubble_kernel<5>, grid, dim3(256), 0, c->stream, a); break;
-      case 10: hipLaunchKernelGGL(bubble_kernel<10>, grid, dim3(256), 0, c->stream, a); break;
-      case 15: hipLaunchKernelGGL(bubble_kernel<15>, grid, dim3(256), 0, c->stream, a); break;
-      default: hipLaunchKernelGGL(bubble_kernel<20>, grid, dim3(256), 0, c->stream, a); break;
+      case 1: fn = few ? bubble_kernel<1, 16> : bubble_kernel<1, 64>; break;
+      case 2: fn = few ? bubble_kernel<2, 16> : bubble_kernel<2, 64>; break;
+      case 5: fn = few ? bubble_kernel<5, 16> : bubble_kernel<5, 64>; break;
+      case 10: fn = few ? bubble_kernel<10, 16> : bubble_kernel<10, 64>; break;
+      case 15: fn = few ? bubble_kernel<15, 16> : bubble_kernel<15, 64>; break;
+      case 20: fn = few ? bubble_kernel<20, 16> : bubble_kernel<20, 64>; break;
+      default: fn = few ? bubble_kernel<23, 16> : bubble_kernel<23, 64>; break;
     }
+    hipLaunchKernelGGL(fn, grid, dim3(256), 0, c->stream, a);
     TUPS_HIP(hipGetLastError());
   }
   return TUPS_OK;

@@ -166,7 +166,7 @@ struct tups_ctx {
   int* d_flag = nullptr;
   double* d_bubble_wt = nullptr;  // bubble weight families (bubble.h) and their destinations
   int* d_bubble_dst = nullptr;
-  tups::BubbleSet bubble_set[4];
+  tups::BubbleSet bubble_set[2][4];  // [narrow or wide groups][family]
   double2* green_tab = nullptr;   // table of Green's functions (bubble.h), kept from call to call
   size_t green_tab_bytes = 0;
   bool green_tab_owned = false;   // false: it lies in the block of d_bubble_wt
