@@ -235,9 +235,9 @@ __global__ __launch_bounds__(256) void closed_build_nu(ClosedArgs a) {
 }
 
 // Z(r, c) -= sum_t W(r, k0 + t) W(k0 + t, c) for r in [r0, r1), c in [c0, c1),
-// t < nb (nb <= CL_BB), by 64 x 64 tiles held in registers while the inner
-// index passes through LDS CL_NB at a time; four waves of 2 x 2 blocks of
-// 16 x 16 x 4 MFMAs.  A fragments: lane l holds A[l % 16][l / 16]; B: B[l / 16][l % 16].
+// t < nb (nb <= CL_NB, the panel of closed_solve), by 64 x 64 tiles held in registers
+// with both factors in LDS; four waves of 2 x 2 blocks of 16 x 16 x 4 MFMAs.
+// A fragments: lane l holds A[l % 16][l / 16]; B: B[l / 16][l % 16].
 template <class R>
 __device__ void closed_update(typename Prec<R>::C* W, int D, int r0, int r1, int c0, int c1, int k0, int nb,
                               typename Prec<R>::C (*As)[CL_T + 1], typename Prec<R>::C (*Bs)[CL_T + 1]) {
@@ -262,59 +262,41 @@ __device__ void closed_update(typename Prec<R>::C* W, int D, int r0, int r1, int
             ar[i][j][e] = z.x;
             ai[i][j][e] = z.y;
           }
-      // staging: thread tid moves A(row tid % 64, k (tid / 64) + 4 v) and
-      // B(k tid % 16, column tid / 16 + 16 v), v < 4.  In FP32 the next chunk
-      // is loaded into registers while the MFMAs of this one run; in FP64 that
-      // costs spills in the panel kernel, and the chunk goes straight to LDS.
-      constexpr bool kPrefetch = sizeof(R) == 4;
+      // thread tid moves A(row tid % 64, t (tid / 64) + 4 v) and B(t tid % 16, column
+      // tid / 16 + 16 v), v < 4, all loads before the first store
       C pa[4], pb[4];
-      auto fetch = [&](int kc) {
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int row = tid & (CL_T - 1), ka = (tid >> 6) + 4 * v;
-          pa[v] = (tr + row < r1 && kc + ka < nb) ? W[(size_t)(k0 + kc + ka) * D + tr + row] : zero;
-          const int kb = tid % CL_NB, col = (tid / CL_NB) + 16 * v;
-          pb[v] = (tc + col < c1 && kc + kb < nb) ? W[(size_t)(tc + col) * D + k0 + kc + kb] : zero;
-        }
-      };
-      if constexpr (kPrefetch) fetch(0);
-      for (int kc = 0; kc < nb; kc += CL_NB) {
-        if constexpr (kPrefetch) {
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            As[(tid >> 6) + 4 * v][tid & (CL_T - 1)] = pa[v];
-            Bs[tid % CL_NB][(tid / CL_NB) + 16 * v] = pb[v];
-          }
-        } else {
-          for (int u = tid; u < CL_NB * CL_T; u += 256) {
-            const int row = u & (CL_T - 1), ka = u >> 6;
-            As[ka][row] = (tr + row < r1 && kc + ka < nb) ? W[(size_t)(k0 + kc + ka) * D + tr + row] : zero;
-            const int kb = u % CL_NB, col = u / CL_NB;
-            Bs[kb][col] = (tc + col < c1 && kc + kb < nb) ? W[(size_t)(tc + col) * D + k0 + kc + kb] : zero;
-          }
-        }
-        __syncthreads();
-        if (kPrefetch && kc + CL_NB < nb) fetch(kc + CL_NB);
-#pragma unroll
-        for (int kk = 0; kk < CL_NB; kk += 4) {
-          C fa[2], fb[2];
-#pragma unroll
-          for (int i = 0; i < 2; ++i) fa[i] = As[kk + lk][wr + i * 16 + li];
-#pragma unroll
-          for (int j = 0; j < 2; ++j) fb[j] = Bs[kk + lk][wc + j * 16 + li];
-#pragma unroll
-          for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-              // Z - A B: re -= ar br - ai bi, im -= ar bi + ai br
-              ar[i][j] = P::fma_sub(fa[i].x, fb[j].x, ar[i][j]);
-              ar[i][j] = P::fma_add(fa[i].y, fb[j].y, ar[i][j]);
-              ai[i][j] = P::fma_sub(fa[i].x, fb[j].y, ai[i][j]);
-              ai[i][j] = P::fma_sub(fa[i].y, fb[j].x, ai[i][j]);
-            }
-        }
-        __syncthreads();
+      for (int v = 0; v < 4; ++v) {
+        const int row = tid & (CL_T - 1), ka = (tid >> 6) + 4 * v;
+        pa[v] = (tr + row < r1 && ka < nb) ? W[(size_t)(k0 + ka) * D + tr + row] : zero;
+        const int kb = tid % CL_NB, col = tid / CL_NB + 16 * v;
+        pb[v] = (tc + col < c1 && kb < nb) ? W[(size_t)(tc + col) * D + k0 + kb] : zero;
       }
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        As[(tid >> 6) + 4 * v][tid & (CL_T - 1)] = pa[v];
+        Bs[tid % CL_NB][tid / CL_NB + 16 * v] = pb[v];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int kk = 0; kk < CL_NB; kk += 4) {
+        C fa[2], fb[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) fa[i] = As[kk + lk][wr + i * 16 + li];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) fb[j] = Bs[kk + lk][wc + j * 16 + li];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            // Z - A B: re -= ar br - ai bi, im -= ar bi + ai br
+            ar[i][j] = P::fma_sub(fa[i].x, fb[j].x, ar[i][j]);
+            ar[i][j] = P::fma_add(fa[i].y, fb[j].y, ar[i][j]);
+            ai[i][j] = P::fma_sub(fa[i].x, fb[j].y, ai[i][j]);
+            ai[i][j] = P::fma_sub(fa[i].y, fb[j].x, ai[i][j]);
+          }
+      }
+      __syncthreads();
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
