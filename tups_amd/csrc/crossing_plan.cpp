@@ -7,10 +7,10 @@
 // one or of a few (l1, l2) form a block of 16 with the union of their indices as
 // its inner dimension, in MFMA k-steps of four, instead of all rows in order with
 // every index.
+#include "crossing_plan.h"
+
 #include <algorithm>
 #include <numeric>
-
-#include "internal.h"
 
 namespace tups {
 
