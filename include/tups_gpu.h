@@ -32,6 +32,8 @@
  *    failure; tups_last_error() returns a message for the calling thread.
  *  - One host thread drives one context; calls are stream-ordered on the
  *    context's HIP stream and return without synchronising unless stated.
+ *    A call that needs more workspace than any before it allocates, and a
+ *    captured graph that held the old one is captured anew at its next use.
  */
 #ifndef TUPS_GPU_H
 #define TUPS_GPU_H
@@ -349,7 +351,11 @@ int tups_uneven_sync(tups_uneven* u);
 
 /* calc_PhiR(ite): PhiR_r from Gamma_r (holding Phi_r); SRC/parquet_PhiR.f90:35-109 */
 int tups_phir(tups_ctx* ctx);
-/* calc_M_*: the four transformation tensors; SRC/parquet_EQMatrix.f90:21-360 */
+/* calc_M_*: the four transformation tensors; SRC/parquet_EQMatrix.f90:21-360.  At
+ * Nl > 1 synchronous: the crossing's plan is made from M on the host (0.1 to 0.7
+ * ms) and its tables are allocated.  After an M from the host (tups_upload, tups_copy)
+ * the first tups_pae, tups_iteration, tups_iteration_full or tups_uneven_iteration
+ * makes the plan, is synchronous for it, and captures its graph anew. */
 int tups_build_m(tups_ctx* ctx);
 /* calculate_PAE: F_r <- Phi_r + Lambda_r*Nc + crossing; SRC/parquet_EQOuter.f90:16-118 */
 int tups_pae(tups_ctx* ctx);

@@ -63,9 +63,16 @@ static BubbleOut chi_out(tups_ctx* c) {
   return {c->chi[0], c->chi[1], (long long)s.nl * s.nl * s.nf, s.nl * s.nl, 1};
 }
 
+// The boxes that calc_chi takes.  No buffer of the bubbles grows with Nx any more; the line is
+// where the k-space bubble of a frequency filled the LDS, and larger boxes stay refused.
+static int chi_box_ok(const tups_ctx* c) {
+  TUPS_CHECK(c->sz.nx <= 70, TUPS_EINVAL, "calc_chi supports Nx <= 70");
+  return TUPS_OK;
+}
+
 // calc_chi from the Sigma already on the device (g); tab: the table when it is built already
 int launch_chi_device(tups_ctx* c, const GreenParams& g, const GreenTab* tab) {
-  TUPS_CHECK(2 * (size_t)c->sz.nc * sizeof(double2) <= 160 * 1024, TUPS_EINVAL, "calc_chi supports Nx <= 64");
+  if (int rc = chi_box_ok(c)) return rc;
   if (int rc = timer_begin(c)) return rc;
   const BubbleOut out[2] = {chi_out(c), {}};
   if (int rc = launch_bubbles(c, g, 0, kBubbleChi, out, tab)) return rc;
@@ -75,7 +82,7 @@ int launch_chi_device(tups_ctx* c, const GreenParams& g, const GreenTab* tab) {
 
 // calc_chi and, for the self-energy at f_range 0, calc_chi_aux over the same pairs
 int launch_chi_aux_device(tups_ctx* c, const GreenParams& g, const BubbleOut& aux, const GreenTab* tab) {
-  TUPS_CHECK(2 * (size_t)c->sz.nc * sizeof(double2) <= 160 * 1024, TUPS_EINVAL, "calc_chi supports Nx <= 64");
+  if (int rc = chi_box_ok(c)) return rc;
   if (int rc = timer_begin(c)) return rc;
   const BubbleOut out[2] = {chi_out(c), aux};
   if (int rc = launch_bubbles(c, g, 0, kBubbleChiAux, out, tab)) return rc;
@@ -85,6 +92,7 @@ int launch_chi_aux_device(tups_ctx* c, const GreenParams& g, const BubbleOut& au
 
 int launch_calc_chi(tups_ctx* c, const double* sigma, const double* sigma_h, double mu, int ngrain) {
   GreenParams g{};
+  if (int rc = chi_box_ok(c)) return rc;
   TUPS_CHECK(ngrain >= 1 && ngrain <= 64, TUPS_EINVAL, "ngrain must be in 1..64");
   if (int rc = green_tab_reserve(c, ngrain, 0)) return rc;
   if (int rc = upload_sigma(c, sigma, sigma_h, &g, mu, ngrain)) return rc;

@@ -112,6 +112,7 @@ extern "C" int tups_calc_sus(tups_ctx* c, double u, int32_t f_range, int32_t aft
   const tups_sizes& s = c->sz;
   TUPS_CHECK(s.full_ibz, TUPS_EINVAL, "the susceptibilities need every IBZ q of the box (nq = 0 at create)");
   TUPS_CHECK(f_range >= 0 && f_range <= 8, TUPS_EINVAL, "f_range must be in 0..8");
+  // the header's limit; no buffer grows with Nx
   TUPS_CHECK(s.nx * s.ny <= 256, TUPS_EINVAL, "the susceptibilities support Nx <= 16");
   int rc = ensure_tables(c);
   if (rc) return rc;
