@@ -496,7 +496,7 @@ def main():
                "kernel": "closed_build_nu<float2> + closed_panel/diag/row/trail/scale<float> + closed_lu_solve (FP32 MFMA) "
                          "+ ir_gemm (FP64 MFMA) + ir_check",
                "flops_per_call": {"fp32": (8.0 / 3.0 + 8.0 * (1 + ir_steps)) * D ** 3 * 4 * nq,
-                                  "fp64": 8.0 * ir_steps * D ** 3 * 4 * nq}}
+                                  "fp64": 8.0 * (1 + ir_steps) * D ** 3 * 4 * nq}}
     print(f"[bench] refined closed form: {ir_step_ms:.1f} ms per call, {ir_steps} steps, residual {ir_res:.1e}",
           file=sys.stderr, flush=True)
     # --- convergence check: max |F_r| over the four resident vertices (HBM read) -----------

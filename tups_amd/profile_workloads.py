@@ -9,6 +9,7 @@
     python -m tups_amd.profile_workloads uneven   --steps 3   # uneven-box iteration with the crossing
     python -m tups_amd.profile_workloads closed    --steps 1  # direct FP64 elimination, D=320
     python -m tups_amd.profile_workloads closed_ir --steps 1  # FP32 LU + FP64 refinement, D=320
+    python -m tups_amd.profile_workloads case --name iteration-nx16-nf64-nl1 --steps 10  # a case of perf/cases.py
 
 `calib` runs a streaming kernel whose bytes are known exactly (per element:
 read 2 x 16 B, write 16 B) so hardware counters (FETCH_SIZE, WRITE_SIZE) can be
@@ -19,6 +20,7 @@ from __future__ import annotations
 
 import argparse
 import sys
+from pathlib import Path
 
 import numpy as np
 
@@ -151,8 +153,9 @@ def batch_flops(b: TupsBatch) -> float:
 def main(argv=None):
     ap = argparse.ArgumentParser()
     ap.add_argument("workload", choices=["bse", "split", "crossing", "phir", "calib", "batch", "gtau", "config1",
-                                         "conv", "sus", "closed", "closed_ir", "uneven"])
+                                         "conv", "sus", "closed", "closed_ir", "uneven", "case"])
     ap.add_argument("--steps", type=int, default=3)
+    ap.add_argument("--name", default="", help="case: the name of a listed case")
     ap.add_argument("--nx", type=int, default=16)
     ap.add_argument("--nf", type=int, default=64)
     ap.add_argument("--nl", type=int, default=1)
@@ -162,6 +165,22 @@ def main(argv=None):
                     help="batch: tile variant by name (default: autotune); split: GEMM tile by name (default: the "
                          "library's)")
     args = ap.parse_args(argv)
+    if args.workload == "case":
+        # one pass to warm up and then `steps` passes over one state
+        import importlib.util
+
+        import torch
+
+        spec = importlib.util.spec_from_file_location("cases", Path(__file__).resolve().parents[1] / "perf" / "cases.py")
+        cases = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(cases)
+        state = cases.prepare({c["name"]: c for c in cases.listed()}[args.name], 1)
+        for _ in range(args.steps + 1):
+            cases.run(state)
+        torch.cuda.synchronize()
+        print(f"{args.name}: 1 + {args.steps} passes")
+        sys.stdout.flush()
+        return
     if args.workload == "sus":
         # calc_sus on Nx=8, Nf=64, Nl=5 (all 480 IBZ q): random F and Phi, Sigma = 0
         c = TupsContext(nx=8, nf=64, nl=5, beta=2.0, f_damping=0.5)
